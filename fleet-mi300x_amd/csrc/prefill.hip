@@ -1,0 +1,896 @@
+// A prompt's tokens through the whole model, all tokens of a chunk at once.
+//
+// Semantics: fleet_prefill on tokens[0 .. n) at positions pos0 .. equals n
+// calls of fleet_decode_step without the lm_head (src/host/reference_decode.py:
+// 210-302 per token and layer), bit for bit: the cache rows it writes and the
+// last token's residual are what the steps leave. Every projection is the
+// exact dot product rounded once (to fp32, then bf16), scores, softmax and the
+// weighted sum of cache rows are fp64, o_c and q_c are rounded once to fp32,
+// as in the decode kernels.
+//
+// Stepping reads every weight once per token (1.36 ms a step, 515 ms for 384
+// tokens); here a weight is read once per chunk (384 tokens: 50.7 ms). The dot products run on the fp64 matrix cores
+// (v_mfma_f64_16x16x4): a product of two bf16 values is exact in fp64 and so,
+// for these operands, is their sum, so the order of the additions does not
+// matter and no error bound has to be checked.
+//
+// Operand layout of every fp64 MFMA below: lane l holds A[i = l % 16][k = l /
+// 16] and B[k = l / 16][j = l % 16], and D[4 v + l / 16][l % 16] in register
+// pair v. A sum over k may run in any order, so lane group q = l / 16 takes
+// eight consecutive k of every 32 (one 16-byte load of bf16 feeds eight
+// MFMAs), for both operands alike.
+#include <cmath>
+
+#include "attn_body.h"
+
+namespace fleet_moe {
+namespace pre {
+
+using attn::kHeads;
+using attn::kLora;
+using attn::kNope;
+using attn::kQDim;
+using attn::kQkvRows;
+using attn::kRope;
+using attn::kRowElems;
+using attn::kV;
+
+constexpr int kThreads = 256;
+constexpr int kWaves = kThreads / kLanes;
+constexpr int kChunkTokens = 512;       // tokens per chunk: h, partials and q of a chunk stay resident
+constexpr int kTok = 64;                // tokens per workgroup of an expert GEMM
+constexpr int kRows = 128;              // weight rows per workgroup (32 per wave)
+constexpr int kQDimC = kLora + kRope;   // 576: q_c and q_pe of a head
+constexpr int kSlots = kTopK + 1;
+constexpr int kXcds = 8;
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f64x4 mfma64(double a, double b, f64x4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// Element e (0 .. 7) of a 16-byte bf16 chunk, widened.
+__device__ __forceinline__ double widen(const u32x4& w, int e) {
+    const uint32_t d = w[e >> 1];
+    return (double)(e & 1 ? bf_hi(d) : bf_lo(d));
+}
+
+// Row i of a 16-row A tile under the permutation that gives lane group q the
+// four consecutive rows 4 q .. 4 q + 3 of D (register pair v: row 4 q + v).
+__device__ __forceinline__ int perm16(int i) { return 4 * (i & 3) + (i >> 2); }
+
+struct Tables {
+    int32_t off[kRouted + 1];     // first sorted entry of an expert
+    int32_t blk[kRouted + 1];     // first token block (kTok tokens) of an expert
+};
+
+struct Layout {
+    size_t tab, ent, x, xn, xnf, qkv, q, oc, heads, ids, w, h, hs, part, total;
+};
+
+__host__ __device__ constexpr size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+__host__ constexpr Layout layout(int dense_inter) {
+    const size_t T = kChunkTokens;
+    const size_t hs = (size_t)(dense_inter > kSharedInter ? dense_inter : kSharedInter);
+    Layout L{};
+    L.tab = 0;
+    L.ent = up256(sizeof(Tables));
+    L.x = L.ent + up256(T * kTopK * 4);
+    L.xn = L.x + T * kHidden * 4;
+    L.xnf = L.xn + T * kHidden * 2;
+    L.qkv = L.xnf + T * kHidden * 4;
+    L.q = L.qkv + up256(T * kQkvRows * 2);
+    L.oc = L.q + T * kHeads * kQDimC * 4;
+    L.heads = L.oc + T * kHeads * kLora * 4;
+    L.ids = L.heads + T * kHeads * kV * 2;
+    L.w = L.ids + up256(T * kTopK * 4);
+    L.h = L.w + up256(T * kTopK * 4);
+    L.hs = L.h + T * kTopK * kInter * 2;
+    L.part = L.hs + up256(T * hs * 2);
+    L.total = L.part + T * kSlots * kHidden * 2;
+    return L;
+}
+constexpr int kDenseInter = 10944;
+
+// ---------------------------------------------------------------- norms
+
+struct NormLds {
+    double red[kWaves];
+};
+
+// RMSNorm of one 2048-vector held eight per thread (256 threads), the decode
+// kernels' arithmetic; returns the eight bf16 results as a 16-byte chunk.
+__device__ u32x4 norm_row(const float (&v)[8], const uint16_t* gamma, float eps, NormLds& S) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & (kLanes - 1);
+    u32x4 g = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+    if (gamma) {
+        const uint2 a = ld_global_u2(gamma, 2 * tid), b = ld_global_u2(gamma, 2 * tid + 1);
+        g = u32x4{a.x, a.y, b.x, b.y};
+    }
+    double ss = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss += (double)v[i] * v[i];
+    ss = wave_sum64(ss);
+    if (lane == 0) S.red[wave] = ss;
+    __syncthreads();
+    double ssq = 0.0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) ssq += S.red[w];
+    const float var = (float)(ssq / (double)kHidden);
+    const float inv = __fdiv_rn(1.0f, sqrt_rn(var + eps));
+    u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = bf16r(bf16r(v[2 * i] * inv) * bf_lo(g[i]));
+        const float b = bf16r(bf16r(v[2 * i + 1] * inv) * bf_hi(g[i]));
+        o[i] = bf16_bits(a) | (bf16_bits(b) << 16);
+    }
+    return o;
+}
+
+__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
+    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ void store8(float* p, const float (&v)[8]) {
+    reinterpret_cast<float4*>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
+    reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
+}
+__device__ __forceinline__ void widen8(const u32x4& c, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[2 * i] = bf_lo(c[i]);
+        v[2 * i + 1] = bf_hi(c[i]);
+    }
+}
+
+// x = embed[token] (zeros and FLEET_MOE_ABORT_TOKEN outside the vocabulary,
+// as fleet_embed), then layer 0's first norm. One workgroup per token.
+__global__ __launch_bounds__(kThreads) void embed_norm_kernel(const uint16_t* embed,
+                                                              const int32_t* tokens,
+                                                              const uint16_t* gamma, float eps,
+                                                              float* x, uint16_t* xn,
+                                                              uint32_t* status) {
+    __shared__ NormLds S;
+    const int t = blockIdx.x, tid = threadIdx.x;
+    const int tok = tokens[t];
+    u32x4 c = {0u, 0u, 0u, 0u};
+    if (tok >= 0 && tok < attn::kVocab) {
+        c = reinterpret_cast<const u32x4*>(embed + (int64_t)tok * kHidden)[tid];
+    } else if (tid == 0) {
+        __hip_atomic_fetch_or(status, FLEET_MOE_ABORT_TOKEN, __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_AGENT);
+    }
+    float v[8];
+    widen8(c, v);
+    store8(x + (int64_t)t * kHidden + 8 * tid, v);
+    reinterpret_cast<u32x4*>(xn + (int64_t)t * kHidden)[tid] = norm_row(v, gamma, eps, S);
+}
+
+// xn = norm(x), also widened to fp32 for the router when xnf is not null.
+__global__ __launch_bounds__(kThreads) void norm_kernel(const float* x, const uint16_t* gamma,
+                                                        float eps, uint16_t* xn, float* xnf) {
+    __shared__ NormLds S;
+    const int64_t at = (int64_t)blockIdx.x * kHidden;
+    const int tid = threadIdx.x;
+    float v[8];
+    load8(x + at + 8 * tid, v);
+    const u32x4 o = norm_row(v, gamma, eps, S);
+    reinterpret_cast<u32x4*>(xn + at)[tid] = o;
+    if (xnf) {
+        widen8(o, v);
+        store8(xnf + at + 8 * tid, v);
+    }
+}
+
+// The MoE layer's combine of one token, x = bf16(x + bf16(bf16(sum_k part_k) +
+// shared)) with the routed terms in slot order, then the next layer's first
+// norm (xn null after the last layer).
+__global__ __launch_bounds__(kThreads) void combine_norm_kernel(const uint16_t* part, float* x,
+                                                                const uint16_t* gamma, float eps,
+                                                                uint16_t* xn) {
+    __shared__ NormLds S;
+    const int t = blockIdx.x, tid = threadIdx.x;
+    float v[8], y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    load8(x + (int64_t)t * kHidden + 8 * tid, v);
+    u32x4 c[kSlots];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s)
+        c[s] = reinterpret_cast<const u32x4*>(part + ((int64_t)t * kSlots + s) * kHidden)[tid];
+    float p[8];
+#pragma unroll
+    for (int s = 0; s < kTopK; ++s) {
+        widen8(c[s], p);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] += p[i];
+    }
+    widen8(c[kTopK], p);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = bf16r(v[i] + bf16r(bf16r(y[i]) + p[i]));
+    store8(x + (int64_t)t * kHidden + 8 * tid, v);
+    if (xn) reinterpret_cast<u32x4*>(xn + (int64_t)t * kHidden)[tid] = norm_row(v, gamma, eps, S);
+}
+
+// ---------------------------------------------------------------- exact GEMMs
+
+// One wave: 32 weight rows (two A tiles) x 16 NT tokens, K products each, all
+// exact. wp / xp: each lane's rows, offset to its lane group's first chunk
+// (lane l: chunk l / 16 of every four). The next step's chunks are in flight
+// while the current one's 16 NT MFMAs run (64 cycles each: the loads, 2 + NT
+// per step, and the widening are hidden behind them).
+template <int K, int NT>
+__device__ __forceinline__ void gemm_wave(const u32x4* const (&wp)[2], const u32x4* const (&xp)[NT],
+                                          f64x4 (&acc)[2][NT]) {
+    static_assert(K % 32 == 0, "whole steps");
+    constexpr int S = K / 32;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[r][n] = f64x4{0.0, 0.0, 0.0, 0.0};
+    u32x4 a[2], b[NT];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) a[r] = ld_stream(wp[r]);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) b[n] = ld_global(xp[n]);
+#pragma unroll 2
+    for (int s = 0; s < S; ++s) {
+        const int nx = s + 1 < S ? 4 * (s + 1) : 0;
+        u32x4 a2[2], b2[NT];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) a2[r] = ld_stream(wp[r] + nx);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) b2[n] = ld_global(xp[n] + nx);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const double a0 = widen(a[0], e), a1 = widen(a[1], e);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const double x = widen(b[n], e);
+                acc[0][n] = mfma64(a0, x, acc[0][n]);
+                acc[1][n] = mfma64(a1, x, acc[1][n]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) a[r] = a2[r];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) b[n] = b2[n];
+    }
+}
+
+// h = bf16(bf16(silu(bf16 g)) * bf16 u)
+__device__ __forceinline__ float swiglu(double g, double u) {
+    return bf16r(bf16r(silu_rn(bf16r((float)g))) * bf16r((float)u));
+}
+
+enum Epi { kEpiBf16, kEpiResidual, kEpiSwiglu };
+
+// Rows x tokens of a plain projection: out[t][row] = bf16 (kEpiBf16, pitch
+// n_rows), x[t][row] = bf16(x + bf16(d)) (kEpiResidual, in place on fp32 x),
+// or the SwiGLU of row pairs (kEpiSwiglu, pitch n_rows / 2). Grid (row tiles,
+// token blocks of 16 NT).
+template <int K, int NT, int EPI>
+__global__ __launch_bounds__(kThreads, 2) void proj_kernel(const uint16_t* W, int n_rows,
+                                                           const uint16_t* X, int T,
+                                                           uint16_t* out, float* x) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
+    const int row0 = kRows * blockIdx.x + 32 * wave, t0 = 16 * NT * blockIdx.y;
+    if (row0 >= n_rows) return;                       // n_rows is a multiple of 32
+    const u32x4 *wp[2], *xp[NT];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+        wp[r] = reinterpret_cast<const u32x4*>(W + (int64_t)(row0 + 16 * r + perm16(i)) * K) + q;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+        xp[n] = reinterpret_cast<const u32x4*>(X + (int64_t)min(t0 + 16 * n + i, T - 1) * K) + q;
+    f64x4 acc[2][NT];
+    gemm_wave<K, NT>(wp, xp, acc);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int t = t0 + 16 * n + i;
+        if (t >= T) continue;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const f64x4 d = acc[r][n];
+            const int row = row0 + 16 * r + 4 * q;
+            if constexpr (EPI == kEpiSwiglu) {
+                const float h0 = swiglu(d[0], d[1]), h1 = swiglu(d[2], d[3]);
+                *reinterpret_cast<uint32_t*>(out + (int64_t)t * (n_rows / 2) + row / 2) =
+                    bf16_bits(h0) | (bf16_bits(h1) << 16);
+            } else if constexpr (EPI == kEpiResidual) {
+                float4* p = reinterpret_cast<float4*>(x + (int64_t)t * n_rows + row);
+                const float4 a = *p;
+                *p = make_float4(bf16r(a.x + bf16r((float)d[0])), bf16r(a.y + bf16r((float)d[1])),
+                                 bf16r(a.z + bf16r((float)d[2])), bf16r(a.w + bf16r((float)d[3])));
+            } else {
+                *reinterpret_cast<uint2*>(out + (int64_t)t * n_rows + row) =
+                    make_uint2(bf16_bits((float)d[0]) | (bf16_bits((float)d[1]) << 16),
+                               bf16_bits((float)d[2]) | (bf16_bits((float)d[3]) << 16));
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------- attention
+
+// Per token: the cache row (kv_a_layernorm of c, RoPE of k_pe) and q_pe.
+__global__ __launch_bounds__(kThreads) void rope_cache_kernel(const uint16_t* qkv,
+                                                              const uint16_t* gamma, float eps,
+                                                              const float* cos, const float* sin,
+                                                              int pos0, uint16_t* cache, float* q) {
+    __shared__ float v[kQkvRows];
+    __shared__ double red[kWaves];
+    const int t = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & (kLanes - 1);
+    const int64_t pos = pos0 + t;
+    const uint16_t* src = qkv + (int64_t)t * kQkvRows;
+    for (int k = tid; k < kQkvRows / 2; k += kThreads) {
+        const uint32_t w = reinterpret_cast<const uint32_t*>(src)[k];
+        v[2 * k] = bf_lo(w);
+        v[2 * k + 1] = bf_hi(w);
+    }
+    __syncthreads();
+    uint16_t* row = cache + pos * kRowElems;
+    const float c0 = v[kQDim + tid], c1 = v[kQDim + kThreads + tid];
+    const double ss = wave_sum64((double)c0 * c0 + (double)c1 * c1);
+    if (lane == 0) red[wave] = ss;
+    __syncthreads();
+    double ssq = 0.0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) ssq += red[w];
+    const float inv = __fdiv_rn(1.0f, sqrt_rn((float)(ssq / (double)kLora) + eps));
+    const float g0 = gamma ? bf_lo(gamma[tid]) : 1.f, g1 = gamma ? bf_lo(gamma[kThreads + tid]) : 1.f;
+    row[tid] = (uint16_t)bf16_bits(bf16r(bf16r(c0 * inv) * g0));
+    row[kThreads + tid] = (uint16_t)bf16_bits(bf16r(bf16r(c1 * inv) * g1));
+    const float cs = cos[pos * kRope + lane], sn = sin[pos * kRope + lane];
+    if (wave == 0) row[kLora + lane] = (uint16_t)bf16_bits(attn::rope_one(v + kQDim + kLora, cs, sn, lane));
+#pragma unroll
+    for (int k = 0; k < kHeads / kWaves; ++k) {
+        const int h = wave + kWaves * k;
+        q[((int64_t)t * kHeads + h) * kQDimC + kLora + lane] =
+            attn::rope_one(v + h * (kNope + kRope) + kNope, cs, sn, lane);
+    }
+}
+
+// q_c = W_UK^T q_nope, exact, rounded once to fp32. A wave: 128 columns of one
+// head x 16 tokens; lane group q sums k = 32 q .. 32 q + 31, a 16-byte load of
+// row k gives one A element of eight column tiles (column 8 i + e of tile e).
+// Grid (token blocks of 16, heads), a wave per 128 columns.
+__global__ __launch_bounds__(kThreads) void qc_kernel(const uint16_t* qkv, const uint16_t* kv_b,
+                                                      int T, float* q_out) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
+    const int h = blockIdx.y, t = 16 * blockIdx.x + i;
+    const uint16_t* xq = qkv + (int64_t)min(t, T - 1) * kQkvRows + h * (kNope + kRope) + 32 * q;
+    u32x4 b[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) b[m] = reinterpret_cast<const u32x4*>(xq)[m];
+    const u32x4* wk = reinterpret_cast<const u32x4*>(
+        kv_b + ((int64_t)h * attn::kKvbRowsPerHead + 32 * q) * kLora + 128 * wave) + i;
+    f64x4 acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        u32x4 a[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a[e] = ld_global(wk + (8 * m + e) * (kLora / kChunk));
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const double x = widen(b[m], k);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] = mfma64(widen(a[k], e), x, acc[e]);
+        }
+    }
+    if (t >= T) return;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (float)acc[e][v];
+        store8(q_out + ((int64_t)t * kHeads + h) * kQDimC + 128 * wave + 8 * (4 * v + q), o);
+    }
+}
+
+struct MlaLds {
+    alignas(16) float q[kHeads][kQDimC + 4];
+    double p[kHeads][64 + 2];
+    double mx[kWaves][kHeads];
+    double ls[kWaves][kHeads];
+};
+
+__device__ __forceinline__ double row_max64(double v) {
+    v = fmax(v, dpp64<0xB1>(v));
+    v = fmax(v, dpp64<0x4E>(v));
+    v = fmax(v, dpp64<0x141>(v));
+    return fmax(v, dpp64<0x140>(v));
+}
+__device__ __forceinline__ double row_sum64(double v) {
+    v += dpp64<0xB1>(v);
+    v += dpp64<0x4E>(v);
+    v += dpp64<0x141>(v);
+    return v + dpp64<0x140>(v);
+}
+
+// One token's 16 heads against cache rows 0 .. pos, all fp64 (the heads share
+// the cached rows, so they are the 16 rows of A). Per 64 positions: wave w
+// takes the scores of positions 16 w .. 16 w + 15 (144 MFMAs), the waves
+// agree on the heads' running maxima, then wave w adds the 64 positions'
+// exp(s - m) c into columns 128 w .. 128 w + 127 (128 MFMAs; a 16-byte load of
+// row k gives one B element of eight column tiles, column 8 j + e of tile e).
+// Tokens run from the last (the longest) to the first.
+__global__ __launch_bounds__(kThreads, 2) void mla_kernel(const float* q, const uint16_t* cache,
+                                                          int pos0, double scale, float* oc) {
+    __shared__ MlaLds S;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & (kLanes - 1), i = lane & 15, g = lane >> 4;
+    const int t = (int)gridDim.x - 1 - (int)blockIdx.x, n_pos = pos0 + t + 1;
+    const float4* qs = reinterpret_cast<const float4*>(q + (int64_t)t * kHeads * kQDimC);
+    for (int k = tid; k < kHeads * kQDimC / 4; k += kThreads) {
+        const int h = k / (kQDimC / 4), c = k - h * (kQDimC / 4);
+        *reinterpret_cast<float4*>(&S.q[h][4 * c]) = qs[k];
+    }
+    double m[4], l[4];
+    f64x4 o[8];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) { m[v] = -INFINITY; l[v] = 0.0; }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = f64x4{0.0, 0.0, 0.0, 0.0};
+    __syncthreads();
+    for (int base = 0; base < n_pos; base += 64) {
+        const int pos = base + 16 * wave + i;
+        f64x4 s = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        if (base + 16 * wave < n_pos) {
+            const u32x4* row = reinterpret_cast<const u32x4*>(
+                cache + (int64_t)min(pos, n_pos - 1) * kRowElems) + g;
+            f64x4 a4[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a4[e] = f64x4{0.0, 0.0, 0.0, 0.0};
+            u32x4 b = ld_global(row);
+#pragma unroll 3
+            for (int k = 0; k < kQDimC / 32; ++k) {
+                const u32x4 nb = ld_global(row + (k + 1 < kQDimC / 32 ? 4 * (k + 1) : 0));
+                float qa[8];
+                load8(&S.q[i][32 * k + 8 * g], qa);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) a4[e & 3] = mfma64((double)qa[e], widen(b, e), a4[e & 3]);
+                b = nb;
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                s[v] = pos < n_pos ? ((a4[0][v] + a4[1][v]) + (a4[2][v] + a4[3][v])) * scale : -INFINITY;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const double mv = row_max64(s[v]);
+            if (i == 0) S.mx[wave][4 * v + g] = mv;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            double mn = m[v];
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) mn = fmax(mn, S.mx[w][4 * v + g]);
+            const double f = exp(m[v] - mn), p = exp(s[v] - mn);
+            m[v] = mn;
+            l[v] = fma(l[v], f, p);
+            S.p[4 * v + g][16 * wave + i] = p;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e][v] *= f;
+        }
+        __syncthreads();
+        const int ks = min(16, (n_pos - base + 3) >> 2);
+        const u32x4* col = reinterpret_cast<const u32x4*>(cache + 128 * wave) + i;
+        u32x4 b = ld_global(col + (int64_t)min(base + g, n_pos - 1) * (kRowElems / kChunk));
+        for (int k = 0; k < ks; ++k) {
+            const u32x4 nb = ld_global(col + (int64_t)min(base + 4 * (k + 1) + g, n_pos - 1) *
+                                                 (kRowElems / kChunk));
+            const double a = S.p[i][4 * k + g];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = mfma64(a, widen(b, e), o[e]);
+            b = nb;
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const double s = row_sum64(l[v]);
+        if (i == 0) S.ls[wave][4 * v + g] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int h = 4 * v + g;
+        const double Ls = (S.ls[0][h] + S.ls[1][h]) + (S.ls[2][h] + S.ls[3][h]);
+        float r[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r[e] = (float)(o[e][v] / Ls);
+        store8(oc + ((int64_t)t * kHeads + h) * kLora + 128 * wave + 8 * i, r);
+    }
+}
+
+// Head outputs bf16(W_UV o_c), exact. Grid (token blocks of 32, heads, halves
+// of the 128 rows), a wave per 16 rows.
+__global__ __launch_bounds__(kThreads) void uv_kernel(const float* oc, const uint16_t* kv_b, int T,
+                                                      uint16_t* heads) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
+    const int h = blockIdx.y, row0 = 64 * blockIdx.z + 16 * wave, t0 = 32 * blockIdx.x;
+    const u32x4* wp = reinterpret_cast<const u32x4*>(
+        kv_b + ((int64_t)h * attn::kKvbRowsPerHead + kNope + row0 + perm16(i)) * kLora) + q;
+    const float* xp[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+        xp[n] = oc + ((int64_t)min(t0 + 16 * n + i, T - 1) * kHeads + h) * kLora + 8 * q;
+    f64x4 acc[2] = {f64x4{0.0, 0.0, 0.0, 0.0}, f64x4{0.0, 0.0, 0.0, 0.0}};
+#pragma unroll 2
+    for (int s = 0; s < kLora / 32; ++s) {
+        const u32x4 a = ld_global(wp + 4 * s);
+        float x[2][8];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) load8(xp[n] + 32 * s, x[n]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const double w = widen(a, e);
+#pragma unroll
+            for (int n = 0; n < 2; ++n) acc[n] = mfma64(w, (double)x[n][e], acc[n]);
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        const int t = t0 + 16 * n + i;
+        if (t >= T) continue;
+        *reinterpret_cast<uint2*>(heads + ((int64_t)t * kHeads + h) * kV + row0 + 4 * q) =
+            make_uint2(bf16_bits((float)acc[n][0]) | (bf16_bits((float)acc[n][1]) << 16),
+                       bf16_bits((float)acc[n][2]) | (bf16_bits((float)acc[n][3]) << 16));
+    }
+}
+
+// ---------------------------------------------------------------- experts
+
+// Entries (token * 6 + slot) sorted by expert, one workgroup. The order of an
+// expert's entries does not matter: each entry's results are its own.
+__global__ __launch_bounds__(1024) void table_kernel(const int32_t* ids, int n, Tables* tab,
+                                                     int32_t* ent) {
+    __shared__ int cnt[kRouted], at[kRouted];
+    const int tid = threadIdx.x;
+    if (tid < kRouted) cnt[tid] = 0;
+    __syncthreads();
+    // (clamped: logits that are not numbers can leave an id outside the table)
+    for (int k = tid; k < n; k += 1024) atomicAdd(&cnt[min(max(ids[k], 0), kRouted - 1)], 1);
+    __syncthreads();
+    if (tid < kRouted) {
+        int off = 0, blk = 0;
+        for (int e = 0; e < tid; ++e) {
+            off += cnt[e];
+            blk += (cnt[e] + kTok - 1) / kTok;
+        }
+        at[tid] = off;
+        tab->off[tid] = off;
+        tab->blk[tid] = blk;
+        if (tid == kRouted - 1) {
+            tab->off[kRouted] = off + cnt[tid];
+            tab->blk[kRouted] = blk + (cnt[tid] + kTok - 1) / kTok;
+        }
+    }
+    __syncthreads();
+    for (int k = tid; k < n; k += 1024) ent[atomicAdd(&at[min(max(ids[k], 0), kRouted - 1)], 1)] = k;
+}
+
+struct ExpertParams {
+    const uint16_t* experts;
+    int64_t stride;
+    const uint16_t* shared;
+    const Tables* tab;
+    const int32_t* ent;
+    const float* weights;
+    const uint16_t* xn;     // [T][H]
+    uint16_t* h;            // [T * 6][1408], in sorted order
+    uint16_t* hs;           // [T][2816]
+    uint16_t* part;         // [T][7][H]
+    int T;
+    int routed_wgs;         // workgroups of routed tiles, then those of the shared expert
+};
+
+// This workgroup's token block of a routed expert: workgroups of one XCD
+// (blockIdx % 8) take all row tiles of a block in turn, so a block's token
+// rows are fetched into one L2. False past the last block.
+__device__ __forceinline__ bool routed_block(const Tables* tab, int tiles, int& e, int& tile, int& j0,
+                                             int& m, int& base) {
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
+    const int b = xcd + kXcds * (local / tiles);
+    tile = local % tiles;
+    if (b >= tab->blk[kRouted]) return false;
+    e = __builtin_popcountll(__ballot(tab->blk[lane] <= b)) - 1;   // the last expert starting at or
+    // before b (an expert without tokens starts where the next one does)
+    base = tab->off[e];
+    j0 = kTok * (b - tab->blk[e]);
+    m = min(kTok, tab->off[e + 1] - base - j0);
+    return true;
+}
+
+template <int NT>
+__device__ __forceinline__ void gate_up_tile(const ExpertParams& P, const uint16_t* W, int row0,
+                                             bool shared, int first, int m) {
+    const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
+    const u32x4 *wp[2], *xp[NT];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+        wp[r] = reinterpret_cast<const u32x4*>(W + (int64_t)(row0 + 16 * r + perm16(i)) * kHidden) + q;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int j = first + min(16 * n + i, m - 1);
+        const int t = shared ? j : P.ent[j] / kTopK;
+        xp[n] = reinterpret_cast<const u32x4*>(P.xn + (int64_t)t * kHidden) + q;
+    }
+    f64x4 acc[2][NT];
+    gemm_wave<kHidden, NT>(wp, xp, acc);
+    uint16_t* out = shared ? P.hs : P.h;
+    const int pitch = shared ? kSharedInter : kInter;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        if (16 * n + i >= m) continue;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const f64x4 d = acc[r][n];
+            *reinterpret_cast<uint32_t*>(out + (int64_t)(first + 16 * n + i) * pitch +
+                                         (row0 + 16 * r + 4 * q) / 2) =
+                bf16_bits(swiglu(d[0], d[1])) | (bf16_bits(swiglu(d[2], d[3])) << 16);
+        }
+    }
+}
+
+// gate / up and SwiGLU of every routed entry and of the shared expert.
+__global__ __launch_bounds__(kThreads, 2) void gate_up_kernel(ExpertParams P) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int e = 0, tile = 0, j0 = 0, m = 0, base = 0;
+    const uint16_t* W;
+    const bool shared = (int)blockIdx.x >= P.routed_wgs;
+    if (!shared) {
+        if (!routed_block(P.tab, 2 * kInter / kRows, e, tile, j0, m, base)) return;
+        W = P.experts + (int64_t)e * P.stride;
+    } else {
+        constexpr int kTiles = 2 * kSharedInter / kRows;
+        const int b = (int)blockIdx.x - P.routed_wgs;
+        tile = b % kTiles;
+        j0 = kTok * (b / kTiles);
+        m = min(kTok, P.T - j0);
+        W = P.shared;
+    }
+    const int row0 = kRows * tile + 32 * wave, first = base + j0;
+    if (m <= 16) gate_up_tile<1>(P, W, row0, shared, first, m);
+    else if (m <= 32) gate_up_tile<2>(P, W, row0, shared, first, m);
+    else if (m <= 48) gate_up_tile<3>(P, W, row0, shared, first, m);
+    else gate_up_tile<4>(P, W, row0, shared, first, m);
+}
+
+template <int K, int NT>
+__device__ __forceinline__ void down_tile(const ExpertParams& P, const uint16_t* W, int row0,
+                                          int first, int m) {
+    constexpr bool shared = K == kSharedInter;
+    const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
+    const u32x4 *wp[2], *xp[NT];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+        wp[r] = reinterpret_cast<const u32x4*>(W + (int64_t)(row0 + 16 * r + perm16(i)) * K) + q;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+        xp[n] = reinterpret_cast<const u32x4*>((shared ? P.hs : P.h) +
+                                               (int64_t)(first + min(16 * n + i, m - 1)) * K) + q;
+    f64x4 acc[2][NT];
+    gemm_wave<K, NT>(wp, xp, acc);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        if (16 * n + i >= m) continue;
+        const int j = first + 16 * n + i;
+        int64_t slot;
+        float w = 1.f;
+        if (shared) {
+            slot = (int64_t)j * kSlots + kTopK;
+        } else {
+            const int en = P.ent[j], t = en / kTopK;
+            slot = (int64_t)t * kSlots + (en - t * kTopK);
+            w = P.weights[en];
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const f64x4 d = acc[r][n];
+            uint32_t b[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float y = bf16r((float)d[v]);
+                b[v] = shared ? bf16_bits(y) : bf16_bits(w * y);
+            }
+            *reinterpret_cast<uint2*>(P.part + slot * kHidden + row0 + 16 * r + 4 * q) =
+                make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+        }
+    }
+}
+
+// down and the routing weight of every routed entry, down of the shared expert.
+__global__ __launch_bounds__(kThreads, 2) void down_kernel(ExpertParams P) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int kTiles = kHidden / kRows;
+    int e = 0, tile = 0, j0 = 0, m = 0, base = 0;
+    if ((int)blockIdx.x < P.routed_wgs) {
+        if (!routed_block(P.tab, kTiles, e, tile, j0, m, base)) return;
+        const uint16_t* W = P.experts + (int64_t)e * P.stride + (int64_t)2 * kInter * kHidden;
+        const int row0 = kRows * tile + 32 * wave, first = base + j0;
+        if (m <= 16) down_tile<kInter, 1>(P, W, row0, first, m);
+        else if (m <= 32) down_tile<kInter, 2>(P, W, row0, first, m);
+        else if (m <= 48) down_tile<kInter, 3>(P, W, row0, first, m);
+        else down_tile<kInter, 4>(P, W, row0, first, m);
+        return;
+    }
+    const int b = (int)blockIdx.x - P.routed_wgs;
+    tile = b % kTiles;
+    j0 = kTok * (b / kTiles);
+    m = min(kTok, P.T - j0);
+    const uint16_t* W = P.shared + (int64_t)2 * kSharedInter * kHidden;
+    const int row0 = kRows * tile + 32 * wave;
+    if (m <= 16) down_tile<kSharedInter, 1>(P, W, row0, j0, m);
+    else if (m <= 32) down_tile<kSharedInter, 2>(P, W, row0, j0, m);
+    else if (m <= 48) down_tile<kSharedInter, 3>(P, W, row0, j0, m);
+    else down_tile<kSharedInter, 4>(P, W, row0, j0, m);
+}
+
+// The last token's residual, for the lm_head.
+__global__ __launch_bounds__(kThreads) void copy_row_kernel(const float* x, float* out) {
+    const int k = blockIdx.x * kThreads + threadIdx.x;
+    out[k] = x[k];
+}
+
+// A projection over T tokens: token blocks of 16 while that leaves fewer than
+// four waves per SIMD (1024 workgroups of four waves), else 32.
+template <int K, int EPI>
+static void launch_proj(const uint16_t* W, int n_rows, const uint16_t* X, int T, uint16_t* out,
+                        float* x, hipStream_t s) {
+    const int tiles = (n_rows + kRows - 1) / kRows;
+    if (tiles * ((T + 31) / 32) < 1024)
+        hipLaunchKernelGGL((proj_kernel<K, 1, EPI>), dim3(tiles, (T + 15) / 16), dim3(kThreads), 0,
+                           s, W, n_rows, X, T, out, x);
+    else
+        hipLaunchKernelGGL((proj_kernel<K, 2, EPI>), dim3(tiles, (T + 31) / 32), dim3(kThreads), 0,
+                           s, W, n_rows, X, T, out, x);
+}
+
+}  // namespace pre
+}  // namespace fleet_moe
+
+using namespace fleet_moe;
+
+int fleet_moe_check_dims(const fleet_moe_dims* d);
+int fleet_moe_check_device(int min_cus);
+
+static bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
+
+extern "C" size_t fleet_prefill_workspace_bytes(const fleet_moe_dims* dims) {
+    if (!dims || fleet_moe_check_dims(dims) != 0) return 0;
+    return pre::layout(pre::kDenseInter).total;
+}
+
+extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_layer* layers,
+                             const int32_t* tokens, int32_t n_tokens, int32_t pos0, float* x_out,
+                             uint32_t* status, void* workspace, size_t workspace_bytes,
+                             const fleet_moe_dims* dims, hipStream_t stream) {
+    using namespace pre;
+    if (!model || !layers || !dims) return FLEET_MOE_ERR_ARG;
+    if (int e = fleet_moe_check_dims(dims)) return e;
+    if (model->n_layers < 1 || model->n_layers > FLEET_STEP_MAX_LAYERS || !model->embed ||
+        !model->rope_cos || !model->rope_sin || model->max_pos < 1 ||
+        model->max_pos > attn::kMaxPos || !tokens || !x_out || !status || !workspace ||
+        n_tokens < 1 || pos0 < 0 || n_tokens > model->max_pos - pos0)
+        return FLEET_MOE_ERR_ARG;
+    if (!aligned(model->embed, 16) || !aligned(model->rope_cos, 4) ||
+        !aligned(model->rope_sin, 4) || !aligned(tokens, 4) || !aligned(x_out, 4) ||
+        !aligned(status, 4) || !aligned(workspace, 256))
+        return FLEET_MOE_ERR_ARG;
+    for (int i = 0; i < model->n_layers; ++i) {
+        const fleet_step_layer& l = layers[i];
+        if (!l.attn.qkv || !l.attn.kv_b || !l.attn.o_proj || !l.cache ||
+            (!l.dense && (!l.moe.router || !l.moe.experts || !l.moe.shared)))
+            return FLEET_MOE_ERR_ARG;
+        if (!aligned(l.attn.norm_in, 8) || !aligned(l.attn.qkv, 16) ||
+            !aligned(l.attn.kv_a_norm, 2) || !aligned(l.attn.kv_b, 16) ||
+            !aligned(l.attn.o_proj, 16) || !aligned(l.cache, 16) || !aligned(l.moe.norm, 8) ||
+            !aligned(l.dense, 16) || !aligned(l.moe.router, 16) || !aligned(l.moe.experts, 16) ||
+            !aligned(l.moe.shared, 16))
+            return FLEET_MOE_ERR_ARG;
+        if (!l.dense && (l.moe.expert_stride < kExpertStride || l.moe.expert_stride % kChunk != 0))
+            return FLEET_MOE_ERR_DIMS;
+    }
+    const Layout L = layout(kDenseInter);
+    if (workspace_bytes < L.total) return FLEET_MOE_ERR_WORKSPACE;
+    if (int e = fleet_moe_check_device(1)) return e;
+    char* ws = static_cast<char*>(workspace);
+    Tables* tab = reinterpret_cast<Tables*>(ws + L.tab);
+    int32_t* ent = reinterpret_cast<int32_t*>(ws + L.ent);
+    float* x = reinterpret_cast<float*>(ws + L.x);
+    uint16_t* xn = reinterpret_cast<uint16_t*>(ws + L.xn);
+    float* xnf = reinterpret_cast<float*>(ws + L.xnf);
+    uint16_t* qkv = reinterpret_cast<uint16_t*>(ws + L.qkv);
+    float* q = reinterpret_cast<float*>(ws + L.q);
+    float* oc = reinterpret_cast<float*>(ws + L.oc);
+    uint16_t* heads = reinterpret_cast<uint16_t*>(ws + L.heads);
+    int32_t* ids = reinterpret_cast<int32_t*>(ws + L.ids);
+    float* wts = reinterpret_cast<float*>(ws + L.w);
+    uint16_t* h = reinterpret_cast<uint16_t*>(ws + L.h);
+    uint16_t* hs = reinterpret_cast<uint16_t*>(ws + L.hs);
+    uint16_t* part = reinterpret_cast<uint16_t*>(ws + L.part);
+    const double mm = 0.1 * 0.707 * std::log(40.0) + 1.0;
+    const double scale = std::pow(192.0, -0.5) * mm * mm;
+    const float eps = dims->rms_eps;
+    for (int c0 = 0; c0 < n_tokens; c0 += kChunkTokens) {
+        const int T = n_tokens - c0 < kChunkTokens ? n_tokens - c0 : kChunkTokens;
+        const int p0 = pos0 + c0;
+        hipLaunchKernelGGL(embed_norm_kernel, dim3(T), dim3(kThreads), 0, stream, model->embed,
+                           tokens + c0, layers[0].attn.norm_in, eps, x, xn, status);
+        for (int i = 0; i < model->n_layers; ++i) {
+            const fleet_step_layer& l = layers[i];
+            launch_proj<kHidden, kEpiBf16>(l.attn.qkv, kQkvRows, xn, T, qkv, nullptr, stream);
+            hipLaunchKernelGGL(rope_cache_kernel, dim3(T), dim3(kThreads), 0, stream, qkv,
+                               l.attn.kv_a_norm, eps, model->rope_cos, model->rope_sin, p0,
+                               l.cache, q);
+            hipLaunchKernelGGL(qc_kernel, dim3((T + 15) / 16, kHeads), dim3(kThreads), 0, stream,
+                               qkv, l.attn.kv_b, T, q);
+            hipLaunchKernelGGL(mla_kernel, dim3(T), dim3(kThreads), 0, stream, q, l.cache, p0,
+                               scale, oc);
+            hipLaunchKernelGGL(uv_kernel, dim3((T + 31) / 32, kHeads, 2), dim3(kThreads), 0,
+                               stream, oc, l.attn.kv_b, T, heads);
+            launch_proj<kHeads * kV, kEpiResidual>(l.attn.o_proj, kHidden, heads, T, nullptr, x,
+                                                   stream);
+            hipLaunchKernelGGL(norm_kernel, dim3(T), dim3(kThreads), 0, stream, x, l.moe.norm, eps,
+                               xn, l.dense ? nullptr : xnf);
+            const bool last = i == model->n_layers - 1;
+            const uint16_t* next = last ? nullptr : layers[i + 1].attn.norm_in;
+            if (l.dense) {
+                launch_proj<kHidden, kEpiSwiglu>(l.dense, 2 * kDenseInter, xn, T, hs, nullptr,
+                                                 stream);
+                launch_proj<kDenseInter, kEpiResidual>(
+                    l.dense + (int64_t)2 * kDenseInter * kHidden, kHidden, hs, T, nullptr, x,
+                    stream);
+                if (!last)
+                    hipLaunchKernelGGL(norm_kernel, dim3(T), dim3(kThreads), 0, stream, x, next,
+                                       eps, xn, nullptr);
+                continue;
+            }
+            if (int e = fleet_moe_router_topk(l.moe.router, xnf, T, nullptr, nullptr, ids, wts,
+                                              dims, stream))
+                return e;
+            hipLaunchKernelGGL(table_kernel, dim3(1), dim3(1024), 0, stream, ids, T * kTopK, tab,
+                               ent);
+            ExpertParams P{};
+            P.experts = l.moe.experts;
+            P.stride = l.moe.expert_stride;
+            P.shared = l.moe.shared;
+            P.tab = tab;
+            P.ent = ent;
+            P.weights = wts;
+            P.xn = xn;
+            P.h = h;
+            P.hs = hs;
+            P.part = part;
+            P.T = T;
+            // at most one partly filled block per selected expert
+            const int n = T * kTopK;
+            const int blocks = (n < kRouted ? n : kRouted) + n / kTok;
+            const int bx = (blocks + kXcds - 1) / kXcds * kXcds, sb = (T + kTok - 1) / kTok;
+            P.routed_wgs = bx * (2 * kInter / kRows);
+            hipLaunchKernelGGL(gate_up_kernel,
+                               dim3(P.routed_wgs + sb * (2 * kSharedInter / kRows)),
+                               dim3(kThreads), 0, stream, P);
+            P.routed_wgs = bx * (kHidden / kRows);
+            hipLaunchKernelGGL(down_kernel, dim3(P.routed_wgs + sb * (kHidden / kRows)),
+                               dim3(kThreads), 0, stream, P);
+            hipLaunchKernelGGL(combine_norm_kernel, dim3(T), dim3(kThreads), 0, stream, part, x,
+                               next, eps, last ? nullptr : xn);
+        }
+        if (c0 + T == n_tokens)
+            hipLaunchKernelGGL(copy_row_kernel, dim3(kHidden / kThreads), dim3(kThreads), 0, stream,
+                               x + (int64_t)(T - 1) * kHidden, x_out);
+    }
+    return (int)hipGetLastError();
+}

@@ -94,6 +94,10 @@ SYMBOLS = [
      [POINTER(FleetStepModel), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
       c_void_p, c_size_t, POINTER(FleetMoeDims), c_void_p]),
     ("fleet_decode_step_status", c_int, [c_void_p, POINTER(ctypes.c_uint32), c_void_p]),
+    ("fleet_prefill_workspace_bytes", c_size_t, [POINTER(FleetMoeDims)]),
+    ("fleet_prefill", c_int,
+     [POINTER(FleetStepModel), c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p,
+      c_void_p, c_size_t, POINTER(FleetMoeDims), c_void_p]),
     ("fleet_ffn_column", c_int,
      [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_size_t, POINTER(FleetMoeDims),
       c_void_p]),

@@ -287,6 +287,25 @@ int fleet_decode_step(const fleet_step_model* model, const int32_t* token, int32
                       void* workspace, size_t workspace_bytes, const fleet_moe_dims* dims,
                       hipStream_t stream);
 
+/* Workspace bytes fleet_prefill needs (one buffer; about 90 MB). */
+size_t fleet_prefill_workspace_bytes(const fleet_moe_dims* dims);
+
+/* n_tokens prompt tokens (device int32) at positions pos0 .. through every
+ * layer, all of a chunk's tokens at once: cache rows pos0 .. pos0 + n_tokens -
+ * 1 of every layer and x_out (fp32[hidden], the last token's residual before
+ * the final norm) are what n_tokens calls of fleet_decode_step leave, bit for
+ * bit; no logits and no pick. layers: the HOST copy of model->layers (its
+ * pointers are kernel arguments); model->lm_head and final_norm are not read.
+ * Every projection is the exact dot product rounded once, as in the decode
+ * kernels. status: a device uint32; a token outside the vocabulary sets
+ * FLEET_MOE_ABORT_TOKEN there and counts as a zero row (as in fleet_embed).
+ * pos0 + n_tokens <= max_pos is checked here. No two workgroups wait for each
+ * other; the workspace needs no clearing. */
+int fleet_prefill(const fleet_step_model* model, const fleet_step_layer* layers,
+                  const int32_t* tokens, int32_t n_tokens, int32_t pos0, float* x_out,
+                  uint32_t* status, void* workspace, size_t workspace_bytes,
+                  const fleet_moe_dims* dims, hipStream_t stream);
+
 /* The FLEET_MOE_ABORT_* bits recorded in a fleet_decode_step workspace (the
  * OR over its stages), read synchronously on `stream`. */
 int fleet_decode_step_status(const void* workspace, uint32_t* status, hipStream_t stream);
