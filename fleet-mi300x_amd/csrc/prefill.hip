@@ -9,10 +9,11 @@
 // as in the decode kernels.
 //
 // Stepping reads every weight once per token (1.36 ms a step, 515 ms for 384
-// tokens); here a weight is read once per chunk (384 tokens: 50.7 ms). The dot products run on the fp64 matrix cores
-// (v_mfma_f64_16x16x4): a product of two bf16 values is exact in fp64 and so,
-// for these operands, is their sum, so the order of the additions does not
-// matter and no error bound has to be checked.
+// tokens); here a weight is read once per chunk (384 tokens: 26 ms). The projections run as exact
+// integer products of digits (digit_gemm.h), which keeps up with HBM; the
+// attention's own products (q_c, scores, the weighted sum, W_UV), whose operands
+// are fp32 or fp64, run on the fp64 matrix cores (v_mfma_f64_16x16x4): their
+// products and sums are exact, or fp64 as in the decode kernels.
 //
 // Operand layout of every fp64 MFMA below: lane l holds A[i = l % 16][k = l /
 // 16] and B[k = l / 16][j = l % 16], and D[4 v + l / 16][l % 16] in register
@@ -22,6 +23,7 @@
 #include <cmath>
 
 #include "attn_body.h"
+#include "digit_gemm.h"
 
 namespace fleet_moe {
 namespace pre {
@@ -37,9 +39,7 @@ using attn::kV;
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kLanes;
-constexpr int kChunkTokens = 512;       // tokens per chunk: h, partials and q of a chunk stay resident
-constexpr int kTok = 64;                // tokens per workgroup of an expert GEMM
-constexpr int kRows = 128;              // weight rows per workgroup (32 per wave)
+constexpr int kChunkTokens = 528;       // tokens per chunk: h, partials and q of a chunk stay resident
 constexpr int kQDimC = kLora + kRope;   // 576: q_c and q_pe of a head
 constexpr int kSlots = kTopK + 1;
 constexpr int kXcds = 8;
@@ -62,11 +62,14 @@ __device__ __forceinline__ int perm16(int i) { return 4 * (i & 3) + (i >> 2); }
 
 struct Tables {
     int32_t off[kRouted + 1];     // first sorted entry of an expert
-    int32_t blk[kRouted + 1];     // first token block (kTok tokens) of an expert
+    int32_t blk[kRouted + 1];     // first token block of an expert
 };
 
 struct Layout {
-    size_t tab, ent, x, xn, xnf, qkv, q, oc, heads, ids, w, h, hs, part, total;
+    size_t tab, ent, x, xn, xnf, qkv, q, oc, heads, ids, w, h, hs, part;
+    size_t xd, headsd, hd, hsd;             // digit rows, 3 bytes a value
+    size_t xm, headsm, hm, hsm;             // their exponents and error constants
+    size_t total;
 };
 
 __host__ __device__ constexpr size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -89,7 +92,15 @@ __host__ constexpr Layout layout(int dense_inter) {
     L.h = L.w + up256(T * kTopK * 4);
     L.hs = L.h + T * kTopK * kInter * 2;
     L.part = L.hs + up256(T * hs * 2);
-    L.total = L.part + T * kSlots * kHidden * 2;
+    L.xd = L.part + T * kSlots * kHidden * 2;
+    L.headsd = L.xd + T * kHidden * 3;
+    L.hd = L.headsd + T * kHeads * kV * 3;
+    L.hsd = L.hd + T * kTopK * kInter * 3;
+    L.xm = L.hsd + up256(T * hs * 3);
+    L.headsm = L.xm + up256(T * sizeof(digit::Meta));
+    L.hm = L.headsm + up256(T * sizeof(digit::Meta));
+    L.hsm = L.hm + up256(T * kTopK * sizeof(digit::Meta));
+    L.total = L.hsm + up256(T * sizeof(digit::Meta));
     return L;
 }
 constexpr int kDenseInter = 10944;
@@ -98,6 +109,15 @@ constexpr int kDenseInter = 10944;
 
 struct NormLds {
     double red[kWaves];
+    uint32_t mx[kWaves];
+    float sb[kWaves], rs[kWaves];
+};
+
+// A normed row's outputs: bf16, and its digits for the projections.
+struct NormOut {
+    uint16_t* xn;          // [T][H], or null (nothing follows)
+    uint8_t* xd;           // [T][3 H]
+    digit::Meta* xm;       // [T]
 };
 
 // RMSNorm of one 2048-vector held eight per thread (256 threads), the decode
@@ -147,12 +167,36 @@ __device__ __forceinline__ void widen8(const u32x4& c, float (&v)[8]) {
     }
 }
 
+// Row t's normed chunk of this thread, and the row's digits.
+__device__ void put_normed(const NormOut& O, int t, const u32x4& o, NormLds& S) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & (kLanes - 1);
+    reinterpret_cast<u32x4*>(O.xn + (int64_t)t * kHidden)[tid] = o;
+    const uint32_t w = digit::wave_umax(digit::absmax16(o));
+    if (lane == 0) S.mx[wave] = w;
+    __syncthreads();
+    const uint32_t mx = max(max(S.mx[0], S.mx[1]), max(S.mx[2], S.mx[3]));
+    int sx;
+    const bool ok = digit::row_exponent(mx, sx);
+    float sb0 = 0.f, res = 0.f;
+    if (ok) digit::put_digits(O.xd + (int64_t)t * 3 * kHidden, tid, o, sx, sb0, res);
+    sb0 = wave_sum(sb0);
+    res = wave_sum(res);
+    if (lane == 0) {
+        S.sb[wave] = sb0;
+        S.rs[wave] = res;
+    }
+    __syncthreads();
+    if (tid == 0)
+        O.xm[t] = digit::make_meta(mx, ok, sx, (S.sb[0] + S.sb[1]) + (S.sb[2] + S.sb[3]),
+                                   (S.rs[0] + S.rs[1]) + (S.rs[2] + S.rs[3]));
+}
+
 // x = embed[token] (zeros and FLEET_MOE_ABORT_TOKEN outside the vocabulary,
 // as fleet_embed), then layer 0's first norm. One workgroup per token.
 __global__ __launch_bounds__(kThreads) void embed_norm_kernel(const uint16_t* embed,
                                                               const int32_t* tokens,
                                                               const uint16_t* gamma, float eps,
-                                                              float* x, uint16_t* xn,
+                                                              float* x, NormOut O,
                                                               uint32_t* status) {
     __shared__ NormLds S;
     const int t = blockIdx.x, tid = threadIdx.x;
@@ -167,19 +211,19 @@ __global__ __launch_bounds__(kThreads) void embed_norm_kernel(const uint16_t* em
     float v[8];
     widen8(c, v);
     store8(x + (int64_t)t * kHidden + 8 * tid, v);
-    reinterpret_cast<u32x4*>(xn + (int64_t)t * kHidden)[tid] = norm_row(v, gamma, eps, S);
+    put_normed(O, t, norm_row(v, gamma, eps, S), S);
 }
 
-// xn = norm(x), also widened to fp32 for the router when xnf is not null.
+// The normed row of x, also widened to fp32 for the router when xnf is not null.
 __global__ __launch_bounds__(kThreads) void norm_kernel(const float* x, const uint16_t* gamma,
-                                                        float eps, uint16_t* xn, float* xnf) {
+                                                        float eps, NormOut O, float* xnf) {
     __shared__ NormLds S;
     const int64_t at = (int64_t)blockIdx.x * kHidden;
     const int tid = threadIdx.x;
     float v[8];
     load8(x + at + 8 * tid, v);
     const u32x4 o = norm_row(v, gamma, eps, S);
-    reinterpret_cast<u32x4*>(xn + at)[tid] = o;
+    put_normed(O, blockIdx.x, o, S);
     if (xnf) {
         widen8(o, v);
         store8(xnf + at + 8 * tid, v);
@@ -188,10 +232,10 @@ __global__ __launch_bounds__(kThreads) void norm_kernel(const float* x, const ui
 
 // The MoE layer's combine of one token, x = bf16(x + bf16(bf16(sum_k part_k) +
 // shared)) with the routed terms in slot order, then the next layer's first
-// norm (xn null after the last layer).
+// norm (O.xn null after the last layer).
 __global__ __launch_bounds__(kThreads) void combine_norm_kernel(const uint16_t* part, float* x,
                                                                 const uint16_t* gamma, float eps,
-                                                                uint16_t* xn) {
+                                                                NormOut O) {
     __shared__ NormLds S;
     const int t = blockIdx.x, tid = threadIdx.x;
     float v[8], y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -211,58 +255,45 @@ __global__ __launch_bounds__(kThreads) void combine_norm_kernel(const uint16_t* 
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = bf16r(v[i] + bf16r(bf16r(y[i]) + p[i]));
     store8(x + (int64_t)t * kHidden + 8 * tid, v);
-    if (xn) reinterpret_cast<u32x4*>(xn + (int64_t)t * kHidden)[tid] = norm_row(v, gamma, eps, S);
+    if (O.xn) put_normed(O, t, norm_row(v, gamma, eps, S), S);
 }
 
-// ---------------------------------------------------------------- exact GEMMs
+// ---------------------------------------------------------------- projections
 
-// One wave: 32 weight rows (two A tiles) x 16 NT tokens, K products each, all
-// exact. wp / xp: each lane's rows, offset to its lane group's first chunk
-// (lane l: chunk l / 16 of every four). The next step's chunks are in flight
-// while the current one's 16 NT MFMAs run (64 cycles each: the loads, 2 + NT
-// per step, and the widening are hidden behind them).
-template <int K, int NT>
-__device__ __forceinline__ void gemm_wave(const u32x4* const (&wp)[2], const u32x4* const (&xp)[NT],
-                                          f64x4 (&acc)[2][NT]) {
-    static_assert(K % 32 == 0, "whole steps");
-    constexpr int S = K / 32;
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int n = 0; n < NT; ++n) acc[r][n] = f64x4{0.0, 0.0, 0.0, 0.0};
-    u32x4 a[2], b[NT];
-#pragma unroll
-    for (int r = 0; r < 2; ++r) a[r] = ld_stream(wp[r]);
-#pragma unroll
-    for (int n = 0; n < NT; ++n) b[n] = ld_global(xp[n]);
-#pragma unroll 2
-    for (int s = 0; s < S; ++s) {
-        const int nx = s + 1 < S ? 4 * (s + 1) : 0;
-        u32x4 a2[2], b2[NT];
-#pragma unroll
-        for (int r = 0; r < 2; ++r) a2[r] = ld_stream(wp[r] + nx);
-#pragma unroll
-        for (int n = 0; n < NT; ++n) b2[n] = ld_global(xp[n] + nx);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const double a0 = widen(a[0], e), a1 = widen(a[1], e);
-#pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                const double x = widen(b[n], e);
-                acc[0][n] = mfma64(a0, x, acc[0][n]);
-                acc[1][n] = mfma64(a1, x, acc[1][n]);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 2; ++r) a[r] = a2[r];
-#pragma unroll
-        for (int n = 0; n < NT; ++n) b[n] = b2[n];
-    }
+// h = bf16(bf16(silu(g)) * u) of bf16 values
+__device__ __forceinline__ float swiglu(float g, float u) { return bf16r(bf16r(silu_rn(g)) * u); }
+
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+    return bf16_bits(a) | (bf16_bits(b) << 16);
 }
 
-// h = bf16(bf16(silu(bf16 g)) * bf16 u)
-__device__ __forceinline__ float swiglu(double g, double u) {
-    return bf16r(bf16r(silu_rn(bf16r((float)g))) * bf16r((float)u));
+// A GEMM's token operand: bf16 rows of K values, their digits and exponents.
+struct Rows {
+    const uint16_t* x;
+    const uint8_t* d;
+    const digit::Meta* m;
+};
+
+// One workgroup: bf16 of its rows from `row0` of W x the tokens row(0 .. m - 1) of
+// X. Returns the first of this wave's 16 rows, or -1 where another wave of the
+// row tile holds the result. Waves past n_rows repeat the last rows.
+template <int K, int NT, int KS, int NW, class Row>
+__device__ __forceinline__ int product(const uint16_t* W, int row0, int n_rows, const Rows& X,
+                                       int m, Row&& row,
+                                       typename digit::Shape<NT, KS, NW>::Lds& L, float (&y)[NT][4]) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = threadIdx.x & 15, first = row0 + 16 * (wave / KS);
+    const uint16_t* w = W + (int64_t)min(first, n_rows - 16) * K;
+    digit::Acc<NT> acc;
+    digit::gemm<K, NT, KS, NW>(w + (int64_t)j * K,
+                           [&](int i) { return X.d + (int64_t)row(min(i, m - 1)) * 3 * K; }, L,
+                           acc);
+    if (wave % KS != 0 || first >= n_rows) return -1;
+    digit::Meta meta[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) meta[n] = X.m[row(min(16 * n + j, m - 1))];
+    digit::finish<K, NT>(acc, meta, m, w, [&](int i) { return X.x + (int64_t)row(i) * K; }, y);
+    return first;
 }
 
 enum Epi { kEpiBf16, kEpiResidual, kEpiSwiglu };
@@ -270,46 +301,34 @@ enum Epi { kEpiBf16, kEpiResidual, kEpiSwiglu };
 // Rows x tokens of a plain projection: out[t][row] = bf16 (kEpiBf16, pitch
 // n_rows), x[t][row] = bf16(x + bf16(d)) (kEpiResidual, in place on fp32 x),
 // or the SwiGLU of row pairs (kEpiSwiglu, pitch n_rows / 2). Grid (row tiles,
-// token blocks of 16 NT).
-template <int K, int NT, int EPI>
-__global__ __launch_bounds__(kThreads, 2) void proj_kernel(const uint16_t* W, int n_rows,
-                                                           const uint16_t* X, int T,
-                                                           uint16_t* out, float* x) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// token blocks of 16 NT); n_rows is a multiple of 16.
+template <int K, int NT, int KS, int EPI>
+__global__ __launch_bounds__(512) void proj_kernel(const uint16_t* W, int n_rows, Rows X, int T,
+                                                   uint16_t* out, float* x) {
+    using Sh = digit::Shape<NT, KS, 8>;
+    __shared__ typename Sh::Lds L;
     const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
-    const int row0 = kRows * blockIdx.x + 32 * wave, t0 = 16 * NT * blockIdx.y;
-    if (row0 >= n_rows) return;                       // n_rows is a multiple of 32
-    const u32x4 *wp[2], *xp[NT];
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-        wp[r] = reinterpret_cast<const u32x4*>(W + (int64_t)(row0 + 16 * r + perm16(i)) * K) + q;
-#pragma unroll
-    for (int n = 0; n < NT; ++n)
-        xp[n] = reinterpret_cast<const u32x4*>(X + (int64_t)min(t0 + 16 * n + i, T - 1) * K) + q;
-    f64x4 acc[2][NT];
-    gemm_wave<K, NT>(wp, xp, acc);
+    const int t0 = Sh::kTok * blockIdx.y, m = min(Sh::kTok, T - t0);
+    float y[NT][4];
+    const int row0 = product<K, NT, KS, 8>(W, Sh::kRows * blockIdx.x, n_rows, X, m,
+                                        [&](int k) { return t0 + k; }, L, y);
+    if (row0 < 0) return;
+    const int row = row0 + 4 * q;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
+        if (16 * n + i >= m) continue;
         const int t = t0 + 16 * n + i;
-        if (t >= T) continue;
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const f64x4 d = acc[r][n];
-            const int row = row0 + 16 * r + 4 * q;
-            if constexpr (EPI == kEpiSwiglu) {
-                const float h0 = swiglu(d[0], d[1]), h1 = swiglu(d[2], d[3]);
-                *reinterpret_cast<uint32_t*>(out + (int64_t)t * (n_rows / 2) + row / 2) =
-                    bf16_bits(h0) | (bf16_bits(h1) << 16);
-            } else if constexpr (EPI == kEpiResidual) {
-                float4* p = reinterpret_cast<float4*>(x + (int64_t)t * n_rows + row);
-                const float4 a = *p;
-                *p = make_float4(bf16r(a.x + bf16r((float)d[0])), bf16r(a.y + bf16r((float)d[1])),
-                                 bf16r(a.z + bf16r((float)d[2])), bf16r(a.w + bf16r((float)d[3])));
-            } else {
-                *reinterpret_cast<uint2*>(out + (int64_t)t * n_rows + row) =
-                    make_uint2(bf16_bits((float)d[0]) | (bf16_bits((float)d[1]) << 16),
-                               bf16_bits((float)d[2]) | (bf16_bits((float)d[3]) << 16));
-            }
+        if constexpr (EPI == kEpiSwiglu) {
+            *reinterpret_cast<uint32_t*>(out + (int64_t)t * (n_rows / 2) + row / 2) =
+                pack2(swiglu(y[n][0], y[n][1]), swiglu(y[n][2], y[n][3]));
+        } else if constexpr (EPI == kEpiResidual) {
+            float4* p = reinterpret_cast<float4*>(x + (int64_t)t * n_rows + row);
+            const float4 a = *p;
+            *p = make_float4(bf16r(a.x + y[n][0]), bf16r(a.y + y[n][1]), bf16r(a.z + y[n][2]),
+                             bf16r(a.w + y[n][3]));
+        } else {
+            *reinterpret_cast<uint2*>(out + (int64_t)t * n_rows + row) =
+                make_uint2(pack2(y[n][0], y[n][1]), pack2(y[n][2], y[n][3]));
         }
     }
 }
@@ -550,10 +569,11 @@ __global__ __launch_bounds__(kThreads) void uv_kernel(const float* oc, const uin
 
 // ---------------------------------------------------------------- experts
 
-// Entries (token * 6 + slot) sorted by expert, one workgroup. The order of an
+// Entries (token * 6 + slot) sorted by expert and each expert's blocks of `tok`
+// tokens, one workgroup. The order of an
 // expert's entries does not matter: each entry's results are its own.
-__global__ __launch_bounds__(1024) void table_kernel(const int32_t* ids, int n, Tables* tab,
-                                                     int32_t* ent) {
+__global__ __launch_bounds__(1024) void table_kernel(const int32_t* ids, int n, int tok,
+                                                     Tables* tab, int32_t* ent) {
     __shared__ int cnt[kRouted], at[kRouted];
     const int tid = threadIdx.x;
     if (tid < kRouted) cnt[tid] = 0;
@@ -565,14 +585,14 @@ __global__ __launch_bounds__(1024) void table_kernel(const int32_t* ids, int n, 
         int off = 0, blk = 0;
         for (int e = 0; e < tid; ++e) {
             off += cnt[e];
-            blk += (cnt[e] + kTok - 1) / kTok;
+            blk += (cnt[e] + tok - 1) / tok;
         }
         at[tid] = off;
         tab->off[tid] = off;
         tab->blk[tid] = blk;
         if (tid == kRouted - 1) {
             tab->off[kRouted] = off + cnt[tid];
-            tab->blk[kRouted] = blk + (cnt[tid] + kTok - 1) / kTok;
+            tab->blk[kRouted] = blk + (cnt[tid] + tok - 1) / tok;
         }
     }
     __syncthreads();
@@ -586,9 +606,11 @@ struct ExpertParams {
     const Tables* tab;
     const int32_t* ent;
     const float* weights;
-    const uint16_t* xn;     // [T][H]
-    uint16_t* h;            // [T * 6][1408], in sorted order
-    uint16_t* hs;           // [T][2816]
+    Rows xn;                // [T][H]
+    Rows hr;                // [T * 6][1408], in sorted order
+    Rows hsr;               // [T][2816]
+    uint16_t* h;            // hr's and hsr's bf16 rows, written by gate / up
+    uint16_t* hs;
     uint16_t* part;         // [T][7][H]
     int T;
     int routed_wgs;         // workgroups of routed tiles, then those of the shared expert
@@ -597,8 +619,8 @@ struct ExpertParams {
 // This workgroup's token block of a routed expert: workgroups of one XCD
 // (blockIdx % 8) take all row tiles of a block in turn, so a block's token
 // rows are fetched into one L2. False past the last block.
-__device__ __forceinline__ bool routed_block(const Tables* tab, int tiles, int& e, int& tile, int& j0,
-                                             int& m, int& base) {
+__device__ __forceinline__ bool routed_block(const Tables* tab, int tok, int tiles, int& e,
+                                             int& tile, int& j0, int& m, int& base) {
     const int lane = threadIdx.x & (kLanes - 1);
     const int xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
     const int b = xcd + kXcds * (local / tiles);
@@ -607,81 +629,71 @@ __device__ __forceinline__ bool routed_block(const Tables* tab, int tiles, int& 
     e = __builtin_popcountll(__ballot(tab->blk[lane] <= b)) - 1;   // the last expert starting at or
     // before b (an expert without tokens starts where the next one does)
     base = tab->off[e];
-    j0 = kTok * (b - tab->blk[e]);
-    m = min(kTok, tab->off[e + 1] - base - j0);
+    j0 = tok * (b - tab->blk[e]);
+    m = min(tok, tab->off[e + 1] - base - j0);
     return true;
 }
 
-template <int NT>
-__device__ __forceinline__ void gate_up_tile(const ExpertParams& P, const uint16_t* W, int row0,
-                                             bool shared, int first, int m) {
+template <int NT, int KS, int NW>
+__device__ __forceinline__ void gate_up_tile(const ExpertParams& P, const uint16_t* W, int tile,
+                                             bool shared, int first, int m, void* lds) {
+    using Sh = digit::Shape<NT, KS, NW>;
     const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
-    const u32x4 *wp[2], *xp[NT];
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-        wp[r] = reinterpret_cast<const u32x4*>(W + (int64_t)(row0 + 16 * r + perm16(i)) * kHidden) + q;
-#pragma unroll
-    for (int n = 0; n < NT; ++n) {
-        const int j = first + min(16 * n + i, m - 1);
-        const int t = shared ? j : P.ent[j] / kTopK;
-        xp[n] = reinterpret_cast<const u32x4*>(P.xn + (int64_t)t * kHidden) + q;
-    }
-    f64x4 acc[2][NT];
-    gemm_wave<kHidden, NT>(wp, xp, acc);
-    uint16_t* out = shared ? P.hs : P.h;
+    float y[NT][4];
     const int pitch = shared ? kSharedInter : kInter;
+    const int row0 = product<kHidden, NT, KS, NW>(
+        W, Sh::kRows * tile, 2 * pitch, P.xn, m,
+        [&](int k) { return shared ? first + k : P.ent[first + k] / kTopK; },
+        *static_cast<typename Sh::Lds*>(lds), y);
+    if (row0 < 0) return;
+    uint16_t* out = shared ? P.hs : P.h;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-        if (16 * n + i >= m) continue;
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const f64x4 d = acc[r][n];
+    for (int n = 0; n < NT; ++n)
+        if (16 * n + i < m)
             *reinterpret_cast<uint32_t*>(out + (int64_t)(first + 16 * n + i) * pitch +
-                                         (row0 + 16 * r + 4 * q) / 2) =
-                bf16_bits(swiglu(d[0], d[1])) | (bf16_bits(swiglu(d[2], d[3])) << 16);
-        }
-    }
+                                         (row0 + 4 * q) / 2) =
+                pack2(swiglu(y[n][0], y[n][1]), swiglu(y[n][2], y[n][3]));
 }
 
-// gate / up and SwiGLU of every routed entry and of the shared expert.
-__global__ __launch_bounds__(kThreads, 2) void gate_up_kernel(ExpertParams P) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// gate / up and SwiGLU of every routed entry and of the shared expert, in
+// blocks of at most 16 NTM tokens.
+template <int NTM, int KS, int NW>
+__global__ __launch_bounds__(64 * NW, NTM == 1 ? 3 : 2) void gate_up_kernel(ExpertParams P) {
+    using Sh = digit::Shape<NTM, KS, NW>;
+    __shared__ typename Sh::Lds L;
     int e = 0, tile = 0, j0 = 0, m = 0, base = 0;
     const uint16_t* W;
     const bool shared = (int)blockIdx.x >= P.routed_wgs;
     if (!shared) {
-        if (!routed_block(P.tab, 2 * kInter / kRows, e, tile, j0, m, base)) return;
+        if (!routed_block(P.tab, Sh::kTok, 2 * kInter / Sh::kRows, e, tile, j0, m, base)) return;
         W = P.experts + (int64_t)e * P.stride;
     } else {
-        constexpr int kTiles = 2 * kSharedInter / kRows;
+        constexpr int kTiles = 2 * kSharedInter / Sh::kRows;
         const int b = (int)blockIdx.x - P.routed_wgs;
         tile = b % kTiles;
-        j0 = kTok * (b / kTiles);
-        m = min(kTok, P.T - j0);
+        j0 = Sh::kTok * (b / kTiles);
+        m = min(Sh::kTok, P.T - j0);
         W = P.shared;
     }
-    const int row0 = kRows * tile + 32 * wave, first = base + j0;
-    if (m <= 16) gate_up_tile<1>(P, W, row0, shared, first, m);
-    else if (m <= 32) gate_up_tile<2>(P, W, row0, shared, first, m);
-    else if (m <= 48) gate_up_tile<3>(P, W, row0, shared, first, m);
-    else gate_up_tile<4>(P, W, row0, shared, first, m);
+    const int first = base + j0;
+    if constexpr (NTM > 1) {
+        if (m <= 16) return gate_up_tile<1, KS, NW>(P, W, tile, shared, first, m, &L);
+        if (m <= 32) return gate_up_tile<2, KS, NW>(P, W, tile, shared, first, m, &L);
+    }
+    gate_up_tile<NTM, KS, NW>(P, W, tile, shared, first, m, &L);
 }
 
-template <int K, int NT>
-__device__ __forceinline__ void down_tile(const ExpertParams& P, const uint16_t* W, int row0,
-                                          int first, int m) {
+template <int K, int NT, int KS, int NW>
+__device__ __forceinline__ void down_tile(const ExpertParams& P, const uint16_t* W, int tile,
+                                          int first, int m, void* lds) {
+    using Sh = digit::Shape<NT, KS, NW>;
     constexpr bool shared = K == kSharedInter;
     const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
-    const u32x4 *wp[2], *xp[NT];
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-        wp[r] = reinterpret_cast<const u32x4*>(W + (int64_t)(row0 + 16 * r + perm16(i)) * K) + q;
-#pragma unroll
-    for (int n = 0; n < NT; ++n)
-        xp[n] = reinterpret_cast<const u32x4*>((shared ? P.hs : P.h) +
-                                               (int64_t)(first + min(16 * n + i, m - 1)) * K) + q;
-    f64x4 acc[2][NT];
-    gemm_wave<K, NT>(wp, xp, acc);
+    float y[NT][4];
+    const int row0 = product<K, NT, KS, NW>(W, Sh::kRows * tile, kHidden, shared ? P.hsr : P.hr, m,
+                                        [&](int k) { return first + k; },
+                                        *static_cast<typename Sh::Lds*>(lds), y);
+    if (row0 < 0) return;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         if (16 * n + i >= m) continue;
@@ -695,46 +707,64 @@ __device__ __forceinline__ void down_tile(const ExpertParams& P, const uint16_t*
             slot = (int64_t)t * kSlots + (en - t * kTopK);
             w = P.weights[en];
         }
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const f64x4 d = acc[r][n];
-            uint32_t b[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float y = bf16r((float)d[v]);
-                b[v] = shared ? bf16_bits(y) : bf16_bits(w * y);
-            }
-            *reinterpret_cast<uint2*>(P.part + slot * kHidden + row0 + 16 * r + 4 * q) =
-                make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
-        }
+        *reinterpret_cast<uint2*>(P.part + slot * kHidden + row0 + 4 * q) =
+            make_uint2(pack2(w * y[n][0], w * y[n][1]), pack2(w * y[n][2], w * y[n][3]));
     }
 }
 
+template <int K, int NTM, int KS, int NW>
+__device__ __forceinline__ void down_block(const ExpertParams& P, const uint16_t* W, int tile,
+                                           int first, int m, void* lds) {
+    if constexpr (NTM > 1) {
+        if (m <= 16) return down_tile<K, 1, KS, NW>(P, W, tile, first, m, lds);
+        if (m <= 32) return down_tile<K, 2, KS, NW>(P, W, tile, first, m, lds);
+    }
+    down_tile<K, NTM, KS, NW>(P, W, tile, first, m, lds);
+}
+
 // down and the routing weight of every routed entry, down of the shared expert.
-__global__ __launch_bounds__(kThreads, 2) void down_kernel(ExpertParams P) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    constexpr int kTiles = kHidden / kRows;
+template <int NTM, int KS, int NW>
+__global__ __launch_bounds__(64 * NW, NTM == 1 ? 3 : 2) void down_kernel(ExpertParams P) {
+    using Sh = digit::Shape<NTM, KS, NW>;
+    __shared__ typename Sh::Lds L;
+    constexpr int kTiles = kHidden / Sh::kRows;
     int e = 0, tile = 0, j0 = 0, m = 0, base = 0;
     if ((int)blockIdx.x < P.routed_wgs) {
-        if (!routed_block(P.tab, kTiles, e, tile, j0, m, base)) return;
-        const uint16_t* W = P.experts + (int64_t)e * P.stride + (int64_t)2 * kInter * kHidden;
-        const int row0 = kRows * tile + 32 * wave, first = base + j0;
-        if (m <= 16) down_tile<kInter, 1>(P, W, row0, first, m);
-        else if (m <= 32) down_tile<kInter, 2>(P, W, row0, first, m);
-        else if (m <= 48) down_tile<kInter, 3>(P, W, row0, first, m);
-        else down_tile<kInter, 4>(P, W, row0, first, m);
+        if (!routed_block(P.tab, Sh::kTok, kTiles, e, tile, j0, m, base)) return;
+        down_block<kInter, NTM, KS, NW>(P, P.experts + (int64_t)e * P.stride +
+                                           (int64_t)2 * kInter * kHidden,
+                                    tile, base + j0, m, &L);
         return;
     }
     const int b = (int)blockIdx.x - P.routed_wgs;
     tile = b % kTiles;
-    j0 = kTok * (b / kTiles);
-    m = min(kTok, P.T - j0);
-    const uint16_t* W = P.shared + (int64_t)2 * kSharedInter * kHidden;
-    const int row0 = kRows * tile + 32 * wave;
-    if (m <= 16) down_tile<kSharedInter, 1>(P, W, row0, j0, m);
-    else if (m <= 32) down_tile<kSharedInter, 2>(P, W, row0, j0, m);
-    else if (m <= 48) down_tile<kSharedInter, 3>(P, W, row0, j0, m);
-    else down_tile<kSharedInter, 4>(P, W, row0, j0, m);
+    j0 = Sh::kTok * (b / kTiles);
+    m = min(Sh::kTok, P.T - j0);
+    down_block<kSharedInter, NTM, KS, NW>(P, P.shared + (int64_t)2 * kSharedInter * kHidden, tile, j0,
+                                      m, &L);
+}
+
+// The two expert launches and the digits between them. `n` entries; at most one
+// partly filled block per selected expert.
+template <int NTM, int KG, int KD, int NW>
+static void launch_experts(ExpertParams P, int n, uint8_t* hd, digit::Meta* hm, uint8_t* hsd,
+                           digit::Meta* hsm, hipStream_t s) {
+    constexpr int kTok = 16 * NTM;
+    const int blocks = (n < kRouted ? n : kRouted) + n / kTok;
+    const int bx = (blocks + kXcds - 1) / kXcds * kXcds, sb = (P.T + kTok - 1) / kTok;
+    constexpr int kGRows = digit::Shape<NTM, KG, NW>::kRows;
+    constexpr int kDRows = digit::Shape<NTM, KD, NW>::kRows;
+    P.routed_wgs = bx * (2 * kInter / kGRows);
+    hipLaunchKernelGGL((gate_up_kernel<NTM, KG, NW>),
+                       dim3(P.routed_wgs + sb * (2 * kSharedInter / kGRows)),
+                       dim3(64 * NW), 0, s, P);
+    hipLaunchKernelGGL((digit::digits_kernel<kInter>), dim3((n + 3) / 4), dim3(256), 0, s, P.h, n,
+                       hd, hm);
+    hipLaunchKernelGGL((digit::digits_kernel<kSharedInter>), dim3((P.T + 3) / 4), dim3(256), 0, s,
+                       P.hs, P.T, hsd, hsm);
+    P.routed_wgs = bx * (kHidden / kDRows);
+    hipLaunchKernelGGL((down_kernel<NTM, KD, NW>), dim3(P.routed_wgs + sb * (kHidden / kDRows)),
+                       dim3(64 * NW), 0, s, P);
 }
 
 // The last token's residual, for the lm_head.
@@ -743,18 +773,30 @@ __global__ __launch_bounds__(kThreads) void copy_row_kernel(const float* x, floa
     out[k] = x[k];
 }
 
-// A projection over T tokens: token blocks of 16 while that leaves fewer than
-// four waves per SIMD (1024 workgroups of four waves), else 32.
+template <int K, int NT, int KS, int EPI>
+static void launch_proj_as(const uint16_t* W, int n_rows, const Rows& X, int T, uint16_t* out,
+                           float* x, hipStream_t s) {
+    using Sh = digit::Shape<NT, KS, 8>;
+    hipLaunchKernelGGL((proj_kernel<K, NT, KS, EPI>),
+                       dim3((n_rows + Sh::kRows - 1) / Sh::kRows, (T + Sh::kTok - 1) / Sh::kTok),
+                       dim3(512), 0, s, W, n_rows, X, T, out, x);
+}
+
+// A projection over T tokens. Few tokens leave few workgroups, so four waves
+// share a row tile's K (16 KB of weights each instead of 64: at 8 tokens qkv
+// 33 -> 13 us, o_proj 29 -> 13); many give the CUs enough to do without.
 template <int K, int EPI>
-static void launch_proj(const uint16_t* W, int n_rows, const uint16_t* X, int T, uint16_t* out,
+static void launch_proj(const uint16_t* W, int n_rows, const Rows& X, int T, uint16_t* out,
                         float* x, hipStream_t s) {
-    const int tiles = (n_rows + kRows - 1) / kRows;
-    if (tiles * ((T + 31) / 32) < 1024)
-        hipLaunchKernelGGL((proj_kernel<K, 1, EPI>), dim3(tiles, (T + 15) / 16), dim3(kThreads), 0,
-                           s, W, n_rows, X, T, out, x);
-    else
-        hipLaunchKernelGGL((proj_kernel<K, 2, EPI>), dim3(tiles, (T + 31) / 32), dim3(kThreads), 0,
-                           s, W, n_rows, X, T, out, x);
+    if (T <= 64) launch_proj_as<K, 1, 4, EPI>(W, n_rows, X, T, out, x, s);
+    else if (T <= 192) launch_proj_as<K, 2, 2, EPI>(W, n_rows, X, T, out, x, s);
+    else launch_proj_as<K, 3, 1, EPI>(W, n_rows, X, T, out, x, s);
+}
+
+template <int K>
+static void launch_digits(const uint16_t* x, int rows, uint8_t* d, digit::Meta* m, hipStream_t s) {
+    hipLaunchKernelGGL((digit::digits_kernel<K>), dim3((rows + 3) / 4), dim3(256), 0, s, x, rows, d,
+                       m);
 }
 
 }  // namespace pre
@@ -820,17 +862,29 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
     uint16_t* h = reinterpret_cast<uint16_t*>(ws + L.h);
     uint16_t* hs = reinterpret_cast<uint16_t*>(ws + L.hs);
     uint16_t* part = reinterpret_cast<uint16_t*>(ws + L.part);
+    auto bytes = [&](size_t o) { return reinterpret_cast<uint8_t*>(ws + o); };
+    auto metas = [&](size_t o) { return reinterpret_cast<digit::Meta*>(ws + o); };
+    const NormOut norm_out{xn, bytes(L.xd), metas(L.xm)}, no_out{nullptr, nullptr, nullptr};
+    const Rows xr{xn, bytes(L.xd), metas(L.xm)}, headsr{heads, bytes(L.headsd), metas(L.headsm)},
+        hr{h, bytes(L.hd), metas(L.hm)}, hsr{hs, bytes(L.hsd), metas(L.hsm)};
     const double mm = 0.1 * 0.707 * std::log(40.0) + 1.0;
     const double scale = std::pow(192.0, -0.5) * mm * mm;
     const float eps = dims->rms_eps;
-    for (int c0 = 0; c0 < n_tokens; c0 += kChunkTokens) {
-        const int T = n_tokens - c0 < kChunkTokens ? n_tokens - c0 : kChunkTokens;
+    const int n_chunks = (n_tokens + kChunkTokens - 1) / kChunkTokens;
+    const int chunk = (n_tokens + n_chunks - 1) / n_chunks;       // even chunks
+    for (int c0 = 0; c0 < n_tokens; c0 += chunk) {
+        const int T = n_tokens - c0 < chunk ? n_tokens - c0 : chunk;
         const int p0 = pos0 + c0;
+        // Up to 160 tokens an expert has 15 or fewer on average: blocks of 16 and
+        // workgroups of four waves, three to a CU (128 tokens: 16.2 ms, 17.2 in
+        // blocks of 48); beyond, blocks of 48, which split a weight once for all
+        // of them (256 tokens: 21.8 ms, 384: 26.3; in blocks of 32 21.9 and 27.8)
+        const bool small = T <= 160;
         hipLaunchKernelGGL(embed_norm_kernel, dim3(T), dim3(kThreads), 0, stream, model->embed,
-                           tokens + c0, layers[0].attn.norm_in, eps, x, xn, status);
+                           tokens + c0, layers[0].attn.norm_in, eps, x, norm_out, status);
         for (int i = 0; i < model->n_layers; ++i) {
             const fleet_step_layer& l = layers[i];
-            launch_proj<kHidden, kEpiBf16>(l.attn.qkv, kQkvRows, xn, T, qkv, nullptr, stream);
+            launch_proj<kHidden, kEpiBf16>(l.attn.qkv, kQkvRows, xr, T, qkv, nullptr, stream);
             hipLaunchKernelGGL(rope_cache_kernel, dim3(T), dim3(kThreads), 0, stream, qkv,
                                l.attn.kv_a_norm, eps, model->rope_cos, model->rope_sin, p0,
                                l.cache, q);
@@ -840,28 +894,30 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
                                scale, oc);
             hipLaunchKernelGGL(uv_kernel, dim3((T + 31) / 32, kHeads, 2), dim3(kThreads), 0,
                                stream, oc, l.attn.kv_b, T, heads);
-            launch_proj<kHeads * kV, kEpiResidual>(l.attn.o_proj, kHidden, heads, T, nullptr, x,
+            launch_digits<kHeads * kV>(heads, T, bytes(L.headsd), metas(L.headsm), stream);
+            launch_proj<kHeads * kV, kEpiResidual>(l.attn.o_proj, kHidden, headsr, T, nullptr, x,
                                                    stream);
             hipLaunchKernelGGL(norm_kernel, dim3(T), dim3(kThreads), 0, stream, x, l.moe.norm, eps,
-                               xn, l.dense ? nullptr : xnf);
+                               norm_out, l.dense ? nullptr : xnf);
             const bool last = i == model->n_layers - 1;
             const uint16_t* next = last ? nullptr : layers[i + 1].attn.norm_in;
             if (l.dense) {
-                launch_proj<kHidden, kEpiSwiglu>(l.dense, 2 * kDenseInter, xn, T, hs, nullptr,
+                launch_proj<kHidden, kEpiSwiglu>(l.dense, 2 * kDenseInter, xr, T, hs, nullptr,
                                                  stream);
+                launch_digits<kDenseInter>(hs, T, bytes(L.hsd), metas(L.hsm), stream);
                 launch_proj<kDenseInter, kEpiResidual>(
-                    l.dense + (int64_t)2 * kDenseInter * kHidden, kHidden, hs, T, nullptr, x,
+                    l.dense + (int64_t)2 * kDenseInter * kHidden, kHidden, hsr, T, nullptr, x,
                     stream);
                 if (!last)
                     hipLaunchKernelGGL(norm_kernel, dim3(T), dim3(kThreads), 0, stream, x, next,
-                                       eps, xn, nullptr);
+                                       eps, norm_out, nullptr);
                 continue;
             }
             if (int e = fleet_moe_router_topk(l.moe.router, xnf, T, nullptr, nullptr, ids, wts,
                                               dims, stream))
                 return e;
-            hipLaunchKernelGGL(table_kernel, dim3(1), dim3(1024), 0, stream, ids, T * kTopK, tab,
-                               ent);
+            hipLaunchKernelGGL(table_kernel, dim3(1), dim3(1024), 0, stream, ids, T * kTopK,
+                               small ? 16 : 48, tab, ent);
             ExpertParams P{};
             P.experts = l.moe.experts;
             P.stride = l.moe.expert_stride;
@@ -869,24 +925,21 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
             P.tab = tab;
             P.ent = ent;
             P.weights = wts;
-            P.xn = xn;
+            P.xn = xr;
+            P.hr = hr;
+            P.hsr = hsr;
             P.h = h;
             P.hs = hs;
             P.part = part;
             P.T = T;
-            // at most one partly filled block per selected expert
-            const int n = T * kTopK;
-            const int blocks = (n < kRouted ? n : kRouted) + n / kTok;
-            const int bx = (blocks + kXcds - 1) / kXcds * kXcds, sb = (T + kTok - 1) / kTok;
-            P.routed_wgs = bx * (2 * kInter / kRows);
-            hipLaunchKernelGGL(gate_up_kernel,
-                               dim3(P.routed_wgs + sb * (2 * kSharedInter / kRows)),
-                               dim3(kThreads), 0, stream, P);
-            P.routed_wgs = bx * (kHidden / kRows);
-            hipLaunchKernelGGL(down_kernel, dim3(P.routed_wgs + sb * (kHidden / kRows)),
-                               dim3(kThreads), 0, stream, P);
+            if (small)
+                launch_experts<1, 1, 1, 4>(P, T * kTopK, bytes(L.hd), metas(L.hm), bytes(L.hsd),
+                                        metas(L.hsm), stream);
+            else
+                launch_experts<3, 1, 1, 8>(P, T * kTopK, bytes(L.hd), metas(L.hm), bytes(L.hsd),
+                                        metas(L.hsm), stream);
             hipLaunchKernelGGL(combine_norm_kernel, dim3(T), dim3(kThreads), 0, stream, part, x,
-                               next, eps, last ? nullptr : xn);
+                               next, eps, last ? no_out : norm_out);
         }
         if (c0 + T == n_tokens)
             hipLaunchKernelGGL(copy_row_kernel, dim3(kHidden / kThreads), dim3(kThreads), 0, stream,

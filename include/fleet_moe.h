@@ -287,7 +287,7 @@ int fleet_decode_step(const fleet_step_model* model, const int32_t* token, int32
                       void* workspace, size_t workspace_bytes, const fleet_moe_dims* dims,
                       hipStream_t stream);
 
-/* Workspace bytes fleet_prefill needs (one buffer; about 90 MB). */
+/* Workspace bytes fleet_prefill needs (one buffer; about 130 MB). */
 size_t fleet_prefill_workspace_bytes(const fleet_moe_dims* dims);
 
 /* n_tokens prompt tokens (device int32) at positions pos0 .. through every

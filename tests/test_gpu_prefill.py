@@ -2,8 +2,8 @@
 teacher-forced decode steps leave, bit for bit: every cache row, the last
 token's residual, the pick and the position. The steps themselves are checked
 against the oracle in test_gpu_decode_model.py and test_gpu_step.py, so no
-tolerance is needed. Lengths around the 16-token tiles, the 64-token blocks
-and the 512-token chunk."""
+tolerance is needed. Lengths around the 16-token tiles, the 48-token blocks,
+the changes of shape (65, 161, 193) and the 528-token chunk."""
 from __future__ import annotations
 
 import pytest
@@ -62,12 +62,42 @@ def check(pair, tokens):
         assert d == 0.0, f"{k}: {d:.2e} of the values differ"
 
 
-@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 33, 64, 65, 130, 512, 530])
+@pytest.mark.parametrize("n", [1, 5, 6, 16, 17, 48, 49, 65, 160, 161, 193, 528, 530])
 def test_prefill_equals_steps(pair, n):
     g = torch.Generator(device="cuda").manual_seed(n)
     tokens = torch.randint(0, lay_mod.VOCAB, (n,), generator=g, device="cuda", dtype=torch.int32)
     check(pair, tokens)
     assert pair[0].status() == 0 and pair[1].status() == 0
+
+
+def test_wide_exponents_and_zero_rows(pair):
+    """Weights whose magnitudes span 2^40 within a row, zero rows, rows far
+    below 2^-87 and norms of 0: where a dot product cannot be certified from
+    its leading digits, the fp64 path decides, and the bits stay the steps'."""
+    got, want = pair
+    blob, lay = got.blob, got.layout
+    kept = blob.clone()
+    g = torch.Generator(device="cuda").manual_seed(9)
+    words = blob.view(torch.bfloat16)
+    for name, t in lay.tensors.items():
+        v = words[t.offset // 2: (t.offset + t.nbytes) // 2]
+        if name.endswith(("qkv", "o_proj", "dense", "shared", "experts")):
+            for part in v.split(1 << 26):
+                e = torch.randint(-34, 7, part.shape, generator=g, device="cuda")
+                part.mul_(torch.exp2(e.float()).bfloat16())
+            rows = v[: v.numel() // 2048 * 2048].view(-1, 2048)
+            rows[3::40] = 0
+            rows[5::40] *= 1e-35
+        elif name.endswith("norm_post"):
+            v[::7] = 0
+    try:
+        n = 40
+        tokens = torch.randint(0, lay_mod.VOCAB, (n,), generator=g, device="cuda",
+                               dtype=torch.int32)
+        check(pair, tokens)
+        assert bool(torch.isfinite(got.x).all())
+    finally:
+        blob.copy_(kept)
 
 
 def test_one_token_repeated(pair):
