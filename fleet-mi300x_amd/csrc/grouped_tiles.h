@@ -1,0 +1,398 @@
+// The grouped step's kernels for many tokens (launch_grouped draws the line):
+// every unit -- the shared expert, each selected expert -- is cut into
+// workgroups of 16 R W weight rows x up to 16 NT tokens, bf16 MFMA 16x16x32.
+//
+// HBM bound: 17.3 MB per selected expert and 34.6 MB for the shared one, at 31
+// FLOP per byte and 256 tokens. A wave's weights go from HBM into registers (16
+// R rows x 256 K, refilled for the next slice as they are used), so every weight
+// byte is written to and read from LDS once, by its own wave, whatever the number
+// of tokens; the token rows pass through LDS, two slices in turn, each read by
+// the workgroup's four waves. Sums: 8 MFMAs in a chain per 256-K slice, the
+// slices' sums added in fp32 (error against 64 bits 2.0e-4 at 256 tokens, 2.2e-4
+// in the other plan, which chains 32).
+//
+// R = 2, NT = 4 (128 KB of weights in flight per CU): 256 tokens in 285 us; with
+// R = 1 and NT = 3: 335; NT = 2, R = 2: 292, but 332 against 272 under Zipf
+// routing, whose popular experts fill blocks of 64. Persistent workgroups that
+// carry the stream across tiles: 358. The start's plan: 468.
+//
+// Launches: the tables (one workgroup), gate / up + SwiGLU, down + routing weight,
+// combine; data crosses them as plain memory.
+#pragma once
+
+namespace fleet_moe {
+namespace grouped {
+namespace tiles {
+
+constexpr int kSteps = 8;                     // MFMA steps (32 K) per slice
+constexpr int kSliceK = 32 * kSteps;          // 256
+constexpr int kPitch = kSliceK * 2 + 16;      // LDS bytes per token: 16 tokens' chunks hit 64 banks
+constexpr int kXcds = 8;
+
+// Entries sorted by expert, and the first entry and token block of each.
+struct Table {
+    int32_t off[kRouted + 1];
+    int32_t blk[kRouted + 1];
+    int16_t ent[kMaxEntries];
+};
+static_assert(sizeof(Table) <= kTabBytes, "shares the place of the other plan's tables");
+
+struct Params {
+    const uint16_t* experts;
+    const uint16_t* shared;
+    int64_t stride;
+    const float* weights;
+    const uint16_t* x;
+    const Table* tab;
+    uint16_t* h;            // [T * 6][1408] in sorted order, then [T][2816]
+    uint16_t* part;         // [T][7][H]: bf16(w bf16(d)) per slot, the shared expert's bf16(d)
+    uint16_t* out;
+    int T;
+    int routed_wgs;         // workgroups of routed tiles, then those of the shared expert
+};
+
+// One workgroup; ids outside [0, 64) are clamped and reported, as in the other
+// plan. The order of an expert's entries does not reach any result.
+__global__ __launch_bounds__(1024) void table_kernel(const int32_t* ids, int n, int tok, Header* hdr,
+                                                     Table* tab) {
+    __shared__ int cnt[kRouted], at[kRouted];
+    const int tid = threadIdx.x;
+    if (tid < kRouted) cnt[tid] = 0;
+    __syncthreads();
+    int id[2];
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int k = tid + 1024 * r;
+        const int raw = k < n ? ids[k] : 0;
+        id[r] = min(max(raw, 0), kRouted - 1);
+        bad |= raw != id[r];
+        if (k < n) atomicAdd(&cnt[id[r]], 1);
+    }
+    if (__ballot(bad) && (tid & (kLanes - 1)) == 0) flag_abort(hdr, FLEET_MOE_ABORT_BAD_ID);
+    __syncthreads();
+    if (tid < kLanes) {
+        const int c = cnt[tid], b = (c + tok - 1) / tok;
+        const int oi = wave_incl_scan(c), bi = wave_incl_scan(b);
+        at[tid] = oi - c;
+        tab->off[tid] = oi - c;
+        tab->blk[tid] = bi - b;
+        if (tid == kRouted - 1) {
+            tab->off[kRouted] = oi;
+            tab->blk[kRouted] = bi;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int k = tid + 1024 * r;
+        if (k < n) tab->ent[atomicAdd(&at[id[r]], 1)] = (int16_t)k;
+    }
+}
+static_assert(kMaxEntries <= 2048, "two entries per thread");
+
+// LDS of a workgroup: two slices of its tokens' rows, and per wave the turn buffer
+// (two steps of 16 rows).
+constexpr int kTurnPitch = 128 + 16;
+template <int NT, int W>
+struct Lds {
+    alignas(16) uint8_t x[2][16 * NT * kPitch];
+    alignas(16) uint8_t turn[W][16 * kTurnPitch];
+};
+
+// y[n][v] = row 4 q + v of the wave's 16 rows (from `w`) x token 16 n + l % 16;
+// xrow(i): the bf16 row of the workgroup's i-th token.
+// A weight load takes eight rows' 128-byte lines, eight lanes to a line. (In the
+// MFMA's own layout, lane l = row l % 16, the four lanes of a row are 16 apart:
+// every 16 lanes touch 16 lines, 64 bytes of each per load, and the stream stops
+// at 4.9 TB/s.) Two such loads, 16 rows x two steps, change to the MFMA's layout
+// through LDS.
+template <int K, int NT, int R, int W, class XRow>
+__device__ __forceinline__ void gemm(const uint16_t* w, XRow&& xrow, Lds<NT, W>& L,
+                                     f32x4 (&y)[R][NT]) {
+    constexpr int kChunks = K / kChunk;                  // 16-byte chunks per row
+    constexpr int kTokChunks = kSliceK / kChunk;         // 32 per slice
+    constexpr int P = 16 * NT * kTokChunks / (64 * W);
+    static_assert(16 * NT * kTokChunks % (64 * W) == 0 && K % 64 == 0, "whole chunks, whole lines");
+    const int tid = threadIdx.x, lane = tid & (kLanes - 1), j = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const u32x4* wp = reinterpret_cast<const u32x4*>(w) + (lane >> 3) * kChunks + (lane & 7);
+    uint8_t* const turn = L.turn[wave];
+    uint8_t* const tw = turn + (lane >> 3) * kTurnPitch + 16 * (lane & 7);
+    const uint8_t* const tr = turn + j * kTurnPitch + 16 * q;
+    const u32x4* src[P];
+    const int c = tid % kTokChunks;                      // 64 W is a multiple of 32
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+        src[i] = reinterpret_cast<const u32x4*>(xrow((tid + 64 * W * i) / kTokChunks)) + c;
+    const int dst = (tid / kTokChunks) * kPitch + 16 * c;
+    constexpr int kDst = 64 * W / kTokChunks * kPitch;
+    u32x4 raw[R][kSteps / 2][2], xs[P];
+    auto load_w = [&](int p, int c0) {                   // steps 2 p, 2 p + 1 of the slice at c0
+        if (c0 + 8 * p < kChunks)                        // uniform
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    raw[r][p][h] = ld_stream(wp + (16 * r + 8 * h) * kChunks + c0 + 8 * p);
+    };
+    auto load_x = [&](int c0) {
+        if (c0 + c < kChunks)
+#pragma unroll
+            for (int i = 0; i < P; ++i) xs[i] = ld_global(src[i] + c0);
+    };
+    auto put = [&](int buf, int c0) {
+        if (c0 + c < kChunks)
+#pragma unroll
+            for (int i = 0; i < P; ++i)
+                *reinterpret_cast<u32x4*>(L.x[buf] + dst + i * kDst) = xs[i];
+    };
+    auto barrier = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    // Workgroups start at different slices: rows are 4 KB (2816 B) apart, and all
+    // waves walking them from the left would meet in the same memory channels.
+    constexpr int kSlices = (kChunks + kTokChunks - 1) / kTokChunks;
+    int c0 = (int)(blockIdx.x / kXcds % kSlices) * kTokChunks;
+    load_x(c0);
+#pragma unroll
+    for (int p = 0; p < kSteps / 2; ++p) load_w(p, c0);
+    put(0, c0);
+    barrier();
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) y[r][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int it = 0; it < kSlices; ++it) {
+        const bool more = it + 1 < kSlices;
+        const int buf = it & 1, nx = c0 + kTokChunks < kChunks ? c0 + kTokChunks : 0;
+        if (more) load_x(nx);                            // uniform but for the tail's chunks
+        const uint8_t* xp = L.x[buf] + j * kPitch + 16 * q;
+        f32x4 t[R][NT];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) t[r][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < kSteps / 2; ++p) {
+            if (c0 + 8 * p < kChunks) {                  // uniform
+                u32x4 a[R][2];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        *reinterpret_cast<u32x4*>(tw + 8 * h * kTurnPitch) = raw[r][p][h];
+                    lds_wave_sync();
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        a[r][h] = *reinterpret_cast<const u32x4*>(tr + 64 * h);
+                    lds_wave_sync();
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        const u32x4 b = *reinterpret_cast<const u32x4*>(xp + 16 * n * kPitch +
+                                                                       64 * (2 * p + h));
+#pragma unroll
+                        for (int r = 0; r < R; ++r) t[r][n] = mfma16(a[r][h], b, t[r][n]);
+                    }
+            }
+            if (p == kSteps / 4 && more) put(buf ^ 1, nx);
+            if (more) load_w(p, nx);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) y[r][n] += t[r][n];
+        c0 = nx;
+        barrier();
+    }
+}
+
+// This workgroup's token block of a routed expert (row tile `tile` of `tiles`,
+// entries [first, first + m)): the workgroups of one XCD (blockIdx % 8) take a
+// block's row tiles in turn, so its token rows are fetched into one L2. False
+// past the last block.
+__device__ __forceinline__ bool routed_block(const Table* tab, int tok, int tiles, int& e, int& tile,
+                                             int& first, int& m) {
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int local = blockIdx.x / kXcds, b = blockIdx.x % kXcds + kXcds * (local / tiles);
+    tile = local % tiles;
+    if (b >= tab->blk[kRouted]) return false;
+    // the last expert that starts at or before b (one without tokens starts
+    // where the next does)
+    e = __builtin_popcountll(__ballot(tab->blk[lane] <= b)) - 1;
+    const int j0 = tok * (b - tab->blk[e]);
+    first = tab->off[e] + j0;
+    m = min(tok, tab->off[e + 1] - first);
+    return true;
+}
+
+template <int NT, int R, int W>
+__device__ __forceinline__ void g_tile(const Params& P, const uint16_t* wt, int tile, bool shared,
+                                       int first, int m, void* lds) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
+    const int row0 = 16 * R * (W * tile + wave);
+    f32x4 y[R][NT];
+    gemm<kHidden, NT, R, W>(wt + (int64_t)row0 * kHidden, [&](int k) {
+        const int j = first + min(k, m - 1);
+        return P.x + (int64_t)(shared ? j : P.tab->ent[j] / kTopK) * kHidden;
+    }, *static_cast<Lds<NT, W>*>(lds), y);
+    uint16_t* out = shared ? P.h + (int64_t)P.T * kTopK * kInter : P.h;
+    const int pitch = shared ? kSharedInter : kInter;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+        if (16 * n + i < m)
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const f32x4 d = y[r][n];
+                *reinterpret_cast<uint32_t*>(out + (int64_t)(first + 16 * n + i) * pitch +
+                                             (row0 + 16 * r + 4 * q) / 2) =
+                    pack_bf16(bf16r(bf16r(silu_rn(bf16r(d[0]))) * bf16r(d[1])),
+                              bf16r(bf16r(silu_rn(bf16r(d[2]))) * bf16r(d[3])));
+            }
+}
+
+template <int NTM, int R, int W>
+__global__ __launch_bounds__(64 * W, 2) void g_kernel(Params P) {
+    __shared__ Lds<NTM, W> S;
+    void* lds = &S;
+    int e = 0, tile = 0, first = 0, m = 0;
+    const uint16_t* wt;
+    const bool shared = (int)blockIdx.x >= P.routed_wgs;
+    if (!shared) {
+        if (!routed_block(P.tab, 16 * NTM, 2 * kInter / (16 * R * W), e, tile, first, m)) return;
+        wt = P.experts + (int64_t)e * P.stride;
+    } else {
+        constexpr int kTiles = 2 * kSharedInter / (16 * R * W);
+        const int b = (int)blockIdx.x - P.routed_wgs;
+        tile = b % kTiles;
+        first = 16 * NTM * (b / kTiles);
+        m = min(16 * NTM, P.T - first);
+        wt = P.shared;
+    }
+    if constexpr (NTM > 1)
+        if (m <= 16) return g_tile<1, R, W>(P, wt, tile, shared, first, m, lds);
+    if constexpr (NTM > 2)
+        if (m <= 32) return g_tile<2, R, W>(P, wt, tile, shared, first, m, lds);
+    if constexpr (NTM > 3)
+        if (m <= 48) return g_tile<3, R, W>(P, wt, tile, shared, first, m, lds);
+    g_tile<NTM, R, W>(P, wt, tile, shared, first, m, lds);
+}
+
+template <int K, int NT, int R, int W>
+__device__ __forceinline__ void d_tile(const Params& P, const uint16_t* wt, int tile, int first,
+                                       int m, void* lds) {
+    constexpr bool shared = K == kSharedInter;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
+    const int row0 = 16 * R * (W * tile + wave);
+    const uint16_t* h = shared ? P.h + (int64_t)P.T * kTopK * kInter : P.h;
+    f32x4 y[R][NT];
+    gemm<K, NT, R, W>(wt + (int64_t)row0 * K,
+                   [&](int k) { return h + (int64_t)(first + min(k, m - 1)) * K; },
+                   *static_cast<Lds<NT, W>*>(lds), y);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        if (16 * n + i >= m) continue;
+        const int j = first + 16 * n + i;
+        int64_t slot;
+        float w = 1.f;
+        if (shared) {
+            slot = (int64_t)j * kSlots + kTopK;
+        } else {
+            const int en = P.tab->ent[j], t = en / kTopK;
+            slot = (int64_t)t * kSlots + (en - t * kTopK);
+            w = P.weights[en];
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const f32x4 d = y[r][n];
+            *reinterpret_cast<uint2*>(P.part + slot * kHidden + row0 + 16 * r + 4 * q) =
+                make_uint2(pack_bf16(w * bf16r(d[0]), w * bf16r(d[1])),
+                           pack_bf16(w * bf16r(d[2]), w * bf16r(d[3])));
+        }
+    }
+}
+
+template <int K, int NTM, int R, int W>
+__device__ __forceinline__ void d_block(const Params& P, const uint16_t* wt, int tile, int first,
+                                        int m, void* lds) {
+    if constexpr (NTM > 1)
+        if (m <= 16) return d_tile<K, 1, R, W>(P, wt, tile, first, m, lds);
+    if constexpr (NTM > 2)
+        if (m <= 32) return d_tile<K, 2, R, W>(P, wt, tile, first, m, lds);
+    if constexpr (NTM > 3)
+        if (m <= 48) return d_tile<K, 3, R, W>(P, wt, tile, first, m, lds);
+    d_tile<K, NTM, R, W>(P, wt, tile, first, m, lds);
+}
+
+template <int NTM, int R, int W>
+__global__ __launch_bounds__(64 * W, 2) void d_kernel(Params P) {
+    __shared__ Lds<NTM, W> S;
+    void* lds = &S;
+    constexpr int kTiles = kHidden / (16 * R * W);
+    int e = 0, tile = 0, first = 0, m = 0;
+    if ((int)blockIdx.x < P.routed_wgs) {
+        if (!routed_block(P.tab, 16 * NTM, kTiles, e, tile, first, m)) return;
+        d_block<kInter, NTM, R, W>(P, P.experts + (int64_t)e * P.stride + (int64_t)2 * kInter * kHidden,
+                                tile, first, m, lds);
+        return;
+    }
+    const int b = (int)blockIdx.x - P.routed_wgs;
+    tile = b % kTiles;
+    first = 16 * NTM * (b / kTiles);
+    m = min(16 * NTM, P.T - first);
+    d_block<kSharedInter, NTM, R, W>(P, P.shared + (int64_t)2 * kSharedInter * kHidden, tile, first, m,
+                                  lds);
+}
+
+// out[t] = bf16(bf16(sum_k part[t][k]) + part[t][6]), k in slot order. A
+// workgroup per token.
+__global__ __launch_bounds__(256) void combine_kernel(const uint16_t* part, uint16_t* out) {
+    const int t = blockIdx.x, tid = threadIdx.x;
+    u32x4 c[kSlots];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s)
+        c[s] = reinterpret_cast<const u32x4*>(part + ((int64_t)t * kSlots + s) * kHidden)[tid];
+    u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = 0.f, b = 0.f;
+#pragma unroll
+        for (int s = 0; s < kTopK; ++s) {
+            a += bf_lo(c[s][i]);
+            b += bf_hi(c[s][i]);
+        }
+        o[i] = pack_bf16(bf16r(bf16r(a) + bf_lo(c[kTopK][i])), bf16r(bf16r(b) + bf_hi(c[kTopK][i])));
+    }
+    uint32_t* p = reinterpret_cast<uint32_t*>(out + (int64_t)t * kHidden) + 4 * tid;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p[i] = o[i];          // out is 4-byte aligned
+}
+
+template <int NTM, int R, int W>
+static void launch(Params P, const int32_t* ids, Header* hdr, Table* tab, hipStream_t s) {
+    constexpr int kTok = 16 * NTM;
+    const int n = P.T * kTopK;
+    hipLaunchKernelGGL(table_kernel, dim3(1), dim3(1024), 0, s, ids, n, kTok, hdr, tab);
+    // at most one partly filled block per selected expert
+    const int blocks = (n < kRouted ? n : kRouted) + n / kTok;
+    const int bx = (blocks + kXcds - 1) / kXcds * kXcds, sb = (P.T + kTok - 1) / kTok;
+    P.routed_wgs = bx * (2 * kInter / (16 * R * W));
+    hipLaunchKernelGGL((g_kernel<NTM, R, W>), dim3(P.routed_wgs + sb * (2 * kSharedInter / (16 * R * W))),
+                       dim3(64 * W), 0, s, P);
+    P.routed_wgs = bx * (kHidden / (16 * R * W));
+    hipLaunchKernelGGL((d_kernel<NTM, R, W>), dim3(P.routed_wgs + sb * (kHidden / (16 * R * W))),
+                       dim3(64 * W), 0, s, P);
+    hipLaunchKernelGGL(combine_kernel, dim3(P.T), dim3(256), 0, s, P.part, P.out);
+}
+
+}  // namespace tiles
+}  // namespace grouped
+}  // namespace fleet_moe

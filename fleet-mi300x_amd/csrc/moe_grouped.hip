@@ -31,6 +31,7 @@
 //   (epoch << 32 | payload, device-scope stores and loads; no grid barrier).
 // T > 8: two launches on the stream, G, then D + C; h crosses the kernel
 //   boundary as plain bf16.
+// T >= kTileTokens (84): grouped_tiles.h.
 // Partials bf16(w * bf16(d)) (shared: bf16(d), or with two launches the two
 // fp32 K-half sums) are published per (token, slot) as tagged words; phase C
 // sums them in slot order: out[t] = bf16(bf16(sum_k part[t][k]) + shared[t]).
@@ -94,8 +95,17 @@ static_assert(offsetof(Header, abort) == 8, "status word offset");
 constexpr int kTabBytes = 16 + kUnitsMax * 6 * 4 + kMaxEntries * 2;
 
 struct Layout {
-    size_t tab, h, hp, part, sp, total;
+    size_t tab, h, hp, part, sp, pp, pe, total;
 };
+
+// From this many tokens on, the step runs as tiles (grouped_tiles.h). Above 64
+// tokens the shared expert takes a second pass of the MFMA items here, each
+// reading its weights anew, and every 32-row item of an expert with few tokens
+// leaves waves idle (uniform / Zipf(1.1) routing, us): 80 tokens 294 / 179 here,
+// 241 / 179 as tiles; 96: 330 / 209 and 234 / 188; 128: 421 / 266 and 243 / 211;
+// 256: 468 / 390 and 285 / 272. At 72 tokens the Zipf step is still faster here
+// (168 and 177).
+constexpr int kTileTokens = 84;
 
 __host__ __device__ constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
@@ -106,7 +116,12 @@ __host__ __device__ constexpr Layout layout(int max_tokens) {
     L.hp = L.h + align256((size_t)(max_tokens < kVMax ? max_tokens : kVMax) * kHWordsPerToken * 8);
     L.part = L.hp + align256((size_t)max_tokens * kHWordsPerToken * 4);
     L.sp = L.part + align256((size_t)max_tokens * kSlots * kPartWords * 8);
-    L.total = L.sp + align256((size_t)max_tokens * 2 * kHidden * 8);
+    L.pp = L.sp + align256((size_t)max_tokens * 2 * kHidden * 8);
+    // plain partials of the tiles: a place of their own, as the tagged words
+    // must never hold anything but tagged words
+    const size_t tiled = max_tokens < kTileTokens ? 0 : (size_t)max_tokens;
+    L.pe = L.pp + tiled * kSlots * kHidden * 2;
+    L.total = L.pe + align256(tiled * kTopK * 8);
     return L;
 }
 
@@ -1140,6 +1155,8 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_dc_kernel(Params P) {
 }  // namespace grouped
 }  // namespace fleet_moe
 
+#include "grouped_tiles.h"
+
 using namespace fleet_moe;
 
 int fleet_moe_check_dims(const fleet_moe_dims* d);
@@ -1190,6 +1207,23 @@ static int launch_grouped(const fleet_moe_layer* layer, int32_t n_tokens, const 
                           const float* weights, const uint16_t* x_norm, uint16_t* out,
                           char* ws, int max_tokens, hipStream_t stream) {
     const grouped::Layout L = grouped::layout(max_tokens);
+    if (n_tokens >= grouped::kTileTokens && max_tokens >= grouped::kTileTokens) {
+        grouped::tiles::Params Q{};
+        Q.experts = layer->experts;
+        Q.shared = layer->shared;
+        Q.stride = layer->expert_stride;
+        Q.weights = weights;
+        Q.x = x_norm;
+        grouped::tiles::Table* tab = reinterpret_cast<grouped::tiles::Table*>(ws + L.tab);
+        Q.tab = tab;
+        Q.h = reinterpret_cast<uint16_t*>(ws + L.hp);
+        Q.part = reinterpret_cast<uint16_t*>(ws + L.pp);
+        Q.out = out;
+        Q.T = n_tokens;
+        grouped::tiles::launch<4, 2, 4>(Q, ids, reinterpret_cast<grouped::Header*>(ws), tab,
+                                        stream);
+        return (int)hipGetLastError();
+    }
     grouped::Params P;
     P.experts = layer->experts;
     P.shared = layer->shared;

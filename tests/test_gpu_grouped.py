@@ -195,3 +195,81 @@ def test_grouped_call_count_wrap_restarts_a_clean_workspace(dev):
         else:           # the call numbered 2^32 - 1 (n = 1) restarted the count at 0
             assert head == [n - 1, 256 * (n - 1)]
     assert runner.status() == 0
+
+
+@pytest.mark.parametrize("T, routing", [(83, "uniform"), (84, "uniform"), (84, "zipf"),
+                                        (97, "hot"), (129, "zipf"), (193, "uniform"),
+                                        (255, "hot"), (256, "zipf"), (256, "one")])
+def test_grouped_tiles(dev, T, routing):
+    """The tiled plan from its first token count (84) to the largest, at block
+    edges (m = 1 mod 16, 64 + 1, 256): uniform and Zipf routing, the same six
+    experts for all (blocks of 64 of one expert), and one expert six times
+    per token (24 blocks). bf16 tolerance, as for the other plans. (The oracle
+    counts a token once per expert, so it has no value for "one": that is
+    compared with the same tokens in steps of 64, the other plan.)"""
+    layer, pl = dev
+    runner = ops.GroupedRunner(T, DSV2_LITE)
+    xn = orc.rms_norm(synth.hidden_inputs(150 + T, T))
+    bias = synth.zipf_logit_bias(2) if routing == "zipf" else None
+    _, ids, ws = orc.route(pl.router_f32(), xn, logit_bias=bias)
+    if routing in ("hot", "one"):
+        ids = np.tile(np.array([5, 17, 3, 63, 0, 41] if routing == "hot" else [9] * 6, np.int32),
+                      (T, 1))
+    say(f"grouped tiles T={T} {routing}")
+    a = (torch.from_numpy(orc.bf16_bits(xn).view(np.int16)).cuda(),
+         torch.from_numpy(ids).cuda(), torch.from_numpy(ws).cuda())
+    out = runner.run(layer, *a)
+    torch.cuda.synchronize()
+    got = ops.bf16_bits_to_f32(out).cpu().numpy()
+    if routing == "one":
+        parts = [runner.run(layer, *(v[k: k + 64].contiguous() for v in a)) for k in range(0, T, 64)]
+        want = ops.bf16_bits_to_f32(torch.cat(parts)).cpu().numpy()
+    else:
+        want = orc.moe_grouped(pl, xn, ids, ws)["out"]
+    assert rel_err(got, want) <= 1e-2
+    assert np.mean(got == want) > 0.95
+    assert runner.status() == 0
+
+
+def test_grouped_plans_share_a_workspace(dev):
+    """Tiled and tagged-word steps in turn on one workspace, a tile step with
+    ids out of range, and both under graph capture: every result equals that
+    of a workspace of its own."""
+    layer, pl = dev
+    from fleet_moe import _lib
+    runner = ops.GroupedRunner(256, DSV2_LITE)
+    calls = []
+    for n, T in enumerate((256, 4, 84, 64, 8, 100, 16)):
+        xn = orc.rms_norm(synth.hidden_inputs(210 + n, T))
+        _, ids, ws = orc.route(pl.router_f32(), xn)
+        a = (torch.from_numpy(orc.bf16_bits(xn).view(np.int16)).cuda(),
+             torch.from_numpy(ids).cuda(), torch.from_numpy(ws).cuda())
+        calls.append((a, ops.GroupedRunner(256, DSV2_LITE).run(layer, *a)))
+    for n, (a, want) in enumerate(calls):
+        say(f"shared workspace call {n}")
+        assert torch.equal(runner.run(layer, *a), want), n
+    outs = [torch.empty_like(w) for _, w in calls]
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    say("capture")
+    with torch.cuda.stream(s), torch.cuda.graph(graph, stream=s):
+        for (a, _), o in zip(calls, outs):
+            runner.run_into(layer, *a, o)
+    torch.cuda.current_stream().wait_stream(s)
+    for _ in range(3):
+        for o in outs:
+            o.zero_()
+        graph.replay()
+        runner.run(layer, *calls[1][0])
+        torch.cuda.synchronize()
+        for (_, want), o in zip(calls, outs):
+            assert torch.equal(o, want)
+    assert runner.status() == 0
+    (x, ids, ws), _ = calls[2]
+    bad = ids.clone()
+    bad[70, 2], bad[3, 0] = 64, -5
+    say("tile step with ids out of range")
+    runner.run(layer, x, bad, ws)
+    torch.cuda.synchronize()
+    assert runner.status() == _lib.ABORT_BAD_ID
