@@ -11,8 +11,10 @@
 // (v_mfma_f64_16x16x4); here the eight digit products that matter take 160, and
 // splitting 16 x 64 weights about 500 cycles of the vector ALU (v_perm_b32 and
 // v_cvt_i32_f32 issue every 6 to 8 cycles), whatever the number of tokens. A SIMD's
-// share of HBM delivers those weights in 770. The 27-layer prompt of 384 tokens
-// went from 50.7 ms on the fp64 cores to 26.3, 64 tokens from 24.0 to 12.8.
+// share of HBM delivers those weights in 770: up to 16 tokens per expert the
+// stream runs at 5 TB/s, beyond that the vector ALU and the matrix cores bound it.
+// The 27-layer prompt of 384 tokens went from 50.7 ms on the fp64 cores to 24.0,
+// 64 tokens from 24.0 to 10.7.
 //
 //   x (a token's row, K values): ix = round(x 2^sx), |ix| < 2^22, digits b2 b1
 //     b0 (ix = b2 2^16 + b1 2^8 + b0, |b2| <= 64, |b1|, |b0| <= 128), one
@@ -39,6 +41,9 @@ constexpr int kSliceSteps = 4;        // steps that share a weight exponent
 constexpr int kSliceBytes = kSliceSteps * kStepBytes;         // a token's digits of a slice
 constexpr int kSliceChunks = kSliceBytes / 16;
 
+// A wave's turn buffer: 16 rows x one step (128 bytes, spread over the banks).
+constexpr int kTurnPitch = 2 * kStepK + 16;
+
 // A workgroup's shape: 16 NT tokens x 16 W / KS weight rows, W waves, KS of them
 // sharing 16 rows' K slices (slice s is wave s % KS's). LDS holds two rounds of KS
 // slices of the tokens' digits; the pitch spreads 16 tokens' chunks over all
@@ -51,6 +56,7 @@ struct Shape {
     static constexpr int kRows = 16 * kWaves / KS;
     static constexpr int kPitch = KS * kSliceBytes + 16;
     struct Lds {
+        alignas(16) uint8_t turn[W][16 * kTurnPitch];
         union {
             alignas(16) uint8_t x[2][kTok * kPitch];
             struct {
@@ -216,31 +222,69 @@ __device__ __forceinline__ void split_weights(const u32x4& lo, const u32x4& hi, 
 
 // Sums of one wave's 16 weight rows x 16 NT tokens: lane (j = l % 16, q = l / 16)
 // holds rows 4 q + v of tokens 16 n + j in units of 2^(8 - sx), and per row the
-// error terms es (sum of 2^-sw over the slices) and er (w's own).
+// error terms es (largest 2^-sw of the slices: times a token's constant it bounds
+// the sum over the slices) and er (w's own).
 template <int NT>
 struct Acc {
     f64x4 s[NT];
-    f32x4 es, er;      // fp32 sums of positive terms; finish() covers their rounding
+    f32x4 es, er;      // er: an fp32 sum of positive terms; finish() covers its rounding
 };
 
-// One slice (up to four steps): split the weights in `raw`, multiply with the
-// tokens' digits at `x` in LDS, fold the levels into A.
-// hook(s) runs once step s's registers are split (to refill them).
+// Orders a wave's own LDS accesses.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// Max over the eight lanes of each aligned group of 8.
+__device__ __forceinline__ uint32_t max8_lanes(uint32_t v) {
+    v = max(v, (uint32_t)FLEET_DPP((int)v, 0xB1));
+    v = max(v, (uint32_t)FLEET_DPP((int)v, 0x4E));
+    return max(v, (uint32_t)FLEET_DPP((int)v, 0x141));
+}
+
+// One slice: split the weights in `raw`, multiply with the tokens' digits at `x`
+// in LDS, fold the levels into A. raw[s][h]: step s of row 8 h + l / 8, chunk
+// l % 8 (a load takes eight rows' 128-byte lines; in the MFMA's layout 16 lanes
+// would touch 16 lines); a step's rows change to the MFMA's layout through the
+// wave's turn buffer, one step ahead of their use. hook(s) runs once step s's
+// registers are used (to refill them). Straight-line code: steps past the row's
+// end hold zero weights, whose digits are zero.
 template <int NT, int kPitch, class Hook>
-__device__ __forceinline__ void slice(u32x4 (&raw)[kSliceSteps][2], int n_steps, const uint8_t* x,
-                                      Acc<NT>& A, Hook&& hook) {
+__device__ __forceinline__ void slice(u32x4 (&raw)[kSliceSteps][2], const uint8_t* x,
+                                      uint8_t* turn, Acc<NT>& A, Hook&& hook) {
     const int lane = threadIdx.x & (kLanes - 1), j = lane & 15, q = lane >> 4;
-    // the slice's largest |w| per row
-    u16x2 m2 = {0, 0};
+    uint8_t* const tw = turn + (lane >> 3) * kTurnPitch + 16 * (lane & 7);
+    const uint8_t* const tr = turn + j * kTurnPitch + 16 * q;
+    u32x4 w[2];
+    auto turn_step = [&](int s) {
+        *reinterpret_cast<u32x4*>(tw) = raw[s][0];
+        *reinterpret_cast<u32x4*>(tw + 8 * kTurnPitch) = raw[s][1];
+        wave_sync();
+        w[0] = *reinterpret_cast<const u32x4*>(tr);
+        w[1] = *reinterpret_cast<const u32x4*>(tr + 64);
+        wave_sync();
+    };
+    // the slice's largest |w| per row: of rows 8 h + l / 8, then of row j
+    uint32_t mx;
+    {
+        u16x2 m2[2] = {{0, 0}, {0, 0}};
 #pragma unroll
-    for (int s = 0; s < kSliceSteps; ++s)
+        for (int s = 0; s < kSliceSteps; ++s)
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int d = 0; d < 4; ++d)
-                m2 = __builtin_elementwise_max(
-                    m2, __builtin_bit_cast(u16x2, raw[s][c][d] & 0x7fff7fffu));
-    const uint32_t mx = xor_rows_max(max((uint32_t)m2[0], (uint32_t)m2[1]));
+                for (int d = 0; d < 4; ++d)
+                    m2[h] = __builtin_elementwise_max(
+                        m2[h], __builtin_bit_cast(u16x2, raw[s][h][d] & 0x7fff7fffu));
+        const uint32_t m0 = max8_lanes(max((uint32_t)m2[0][0], (uint32_t)m2[0][1]));
+        const uint32_t m1 = max8_lanes(max((uint32_t)m2[1][0], (uint32_t)m2[1][1]));
+        const int src = (j & 7) << 5;                     // lane 8 (j % 8)
+        const uint32_t b0 = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)m0);
+        const uint32_t b1 = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)m1);
+        mx = j < 8 ? b0 : b1;
+    }
     const int e = (int)(mx >> 7);
     const bool ok = e >= 40 && e < 255;
     // |w| < 2^(e - 126): sw30 = 156 - e
@@ -249,34 +293,32 @@ __device__ __forceinline__ void slice(u32x4 (&raw)[kSliceSteps][2], int n_steps,
 #pragma unroll
     for (int n = 0; n < NT; ++n) l4[n] = l3[n] = l2[n] = l1[n] = i32x4{0, 0, 0, 0};
     uint32_t low = 0;
+    turn_step(0);
     const uint8_t* xp = x + j * kPitch + 16 * q;
 #pragma unroll
     for (int s = 0; s < kSliceSteps; ++s) {
         // (the barrier keeps the scheduler from splitting every step's weights
         // first, which spills)
         __builtin_amdgcn_sched_barrier(0);
-        if (s < n_steps) {
-            u32x4 a[3];
-            split_weights(raw[s][0], raw[s][1], sc, a, low);
-            hook(s);
+        u32x4 a[3];
+        split_weights(w[0], w[1], sc, a, low);
+        hook(s);
+        if (s + 1 < kSliceSteps) turn_step(s + 1);
 #pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                u32x4 b[3];
+        for (int n = 0; n < NT; ++n) {
+            u32x4 b[3];
 #pragma unroll
-                for (int d = 0; d < 3; ++d)
-                    b[d] = *reinterpret_cast<const u32x4*>(xp + 16 * n * kPitch + s * kStepBytes +
-                                                          d * kStepK);
-                l4[n] = mfma8(a[2], b[2], l4[n]);
-                l3[n] = mfma8(a[2], b[1], l3[n]);
-                l2[n] = mfma8(a[2], b[0], l2[n]);
-                l1[n] = mfma8(a[1], b[0], l1[n]);
-                l3[n] = mfma8(a[1], b[2], l3[n]);
-                l2[n] = mfma8(a[1], b[1], l2[n]);
-                l1[n] = mfma8(a[0], b[1], l1[n]);
-                l2[n] = mfma8(a[0], b[2], l2[n]);
-            }
-        } else {
-            hook(s);
+            for (int d = 0; d < 3; ++d)
+                b[d] = *reinterpret_cast<const u32x4*>(xp + 16 * n * kPitch + s * kStepBytes +
+                                                      d * kStepK);
+            l4[n] = mfma8(a[2], b[2], l4[n]);
+            l3[n] = mfma8(a[2], b[1], l3[n]);
+            l2[n] = mfma8(a[2], b[0], l2[n]);
+            l1[n] = mfma8(a[1], b[0], l1[n]);
+            l3[n] = mfma8(a[1], b[2], l3[n]);
+            l2[n] = mfma8(a[1], b[1], l2[n]);
+            l1[n] = mfma8(a[0], b[1], l1[n]);
+            l2[n] = mfma8(a[0], b[2], l2[n]);
         }
     }
     // fold: rows 4 q + v have their exponents in lanes 4 q + v
@@ -290,7 +332,7 @@ __device__ __forceinline__ void slice(u32x4 (&raw)[kSliceSteps][2], int n_steps,
         const bool okr = er >= 40 && er < 255;
         const double u = okr ? pow2(er - 148) : 0.0;        // 2^-(sw30 - 8)
         const float uf = okr ? __uint_as_float((uint32_t)(er - 21) << 23) : 0.f;
-        A.es[v] += mr != 0 && !okr ? INFINITY : uf;
+        A.es[v] = fmaxf(A.es[v], mr != 0 && !okr ? INFINITY : uf);
         A.er[v] += uf * (16384.f * (float)(lr + kSliceSteps * kStepK));
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
@@ -301,15 +343,14 @@ __device__ __forceinline__ void slice(u32x4 (&raw)[kSliceSteps][2], int n_steps,
     }
 }
 
-// The whole workgroup: wrow is this lane's weight row (l % 16 of its wave's 16
-// rows), xd(i) the digit row of the workgroup's i-th token (i < 16 NT). While a
+// The whole workgroup: w is the first of its wave's 16 weight rows, xd(i) the digit row of the workgroup's i-th token (i < 16 NT). While a
 // round of KS slices is multiplied, the next one's weights (registers) and
 // digits (registers, then the other LDS buffer) are on their way: a wave's
 // loads complete in order, so digits loaded straight from memory would wait for
 // the weights issued before them. The KS waves of a row tile add their sums in
 // LDS; A is complete in those with wave % KS == 0.
 template <int K, int NT, int KS, int W, class XD>
-__device__ __forceinline__ void gemm(const uint16_t* wrow, XD&& xd,
+__device__ __forceinline__ void gemm(const uint16_t* w, XD&& xd,
                                      typename Shape<NT, KS, W>::Lds& L, Acc<NT>& A) {
     using Sh = Shape<NT, KS, W>;
     constexpr int kThreads = Sh::kThreads;
@@ -318,64 +359,71 @@ __device__ __forceinline__ void gemm(const uint16_t* wrow, XD&& xd,
     constexpr int R = KS * kSliceSteps;                  // steps per round
     constexpr int kTokChunks = KS * kSliceChunks;
     constexpr int kChunks = Sh::kTok * kTokChunks, P = (kChunks + kThreads - 1) / kThreads;
-    const int tid = threadIdx.x, lane = tid & (kLanes - 1), q = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ks = wave % KS;
-    const u32x4* wp = reinterpret_cast<const u32x4*>(wrow) + q;
-    // this thread's digit chunks of a round: chunk c of token t
+    // the 16 rows as a buffer: a load past it returns zeros and reads nothing
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(w), 0, 16 * K * 2, 0x00020000);
+    const int wat = (lane >> 3) * (K * 2) + 16 * (lane & 7);
+    // this thread's digit chunks of a round: chunk c of token t; threads without
+    // one write to the padding
     const uint8_t* src[P];
-    int at[P];       // LDS offset | step of the round << 20
+    int at[P], col[P];       // LDS offset, offset within a round
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         const int p = tid + kThreads * i, t = p / kTokChunks, c = p - t * kTokChunks;
         const bool have = p < kChunks;
-        src[i] = xd(have ? t : 0) + 16 * c;
-        at[i] = t * Sh::kPitch + 16 * c + ((have ? c / (kStepBytes / 16) : S) << 20);
+        src[i] = xd(have ? t : 0);
+        at[i] = have ? t * Sh::kPitch + 16 * c : Sh::kPitch - 16;
+        col[i] = 16 * c;
     }
 #pragma unroll
     for (int n = 0; n < NT; ++n) A.s[n] = f64x4{0.0, 0.0, 0.0, 0.0};
     A.es = A.er = f32x4{0.f, 0.f, 0.f, 0.f};
     u32x4 raw[kSliceSteps][2], xs[P];
     auto load = [&](int s, int step) {          // step s of the slice, `step` of the row
+        const int off = wat + (step < S ? step * 2 * kStepK : 1 << 30);
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
-            raw[s][c] = step < S ? ld_stream(wp + 8 * step + 4 * c) : u32x4{0u, 0u, 0u, 0u};
+        for (int h = 0; h < 2; ++h)
+            raw[s][h] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 * h * K, 0, 2);
     };
+    // (a chunk past the row's end is never used: any of the row's stands in)
     auto load_x = [&](int s0) {
 #pragma unroll
         for (int i = 0; i < P; ++i)
-            if (s0 + (at[i] >> 20) < S)
-                xs[i] = ld_global(reinterpret_cast<const u32x4*>(src[i] + s0 * kStepBytes));
+            xs[i] = ld_global(reinterpret_cast<const u32x4*>(
+                src[i] + min(s0 * kStepBytes + col[i], S * kStepBytes - 16)));
     };
-    auto put = [&](int buf, int s0) {
+    auto put = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < P; ++i)
-            if (s0 + (at[i] >> 20) < S)
-                *reinterpret_cast<u32x4*>(L.x[buf] + (at[i] & 0xfffff)) = xs[i];
+        for (int i = 0; i < P; ++i) *reinterpret_cast<u32x4*>(L.x[buf] + at[i]) = xs[i];
     };
     auto barrier = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
-    load_x(0);
+    // Workgroups start at different rounds: rows are 4 KB (2816 B) apart, and all
+    // waves walking them from the left would meet in the same memory channels.
+    constexpr int kRounds = (S + R - 1) / R;
+    int s0 = (int)(blockIdx.x / 8 % kRounds) * R;
+    load_x(s0);
 #pragma unroll
-    for (int s = 0; s < kSliceSteps; ++s) load(s, ks * kSliceSteps + s);
-    put(0, 0);
+    for (int s = 0; s < kSliceSteps; ++s) load(s, s0 + ks * kSliceSteps + s);
+    put(0);
     barrier();
-    int buf = 0;
 #pragma unroll 1
-    for (int s0 = 0; s0 < S; s0 += R, buf ^= 1) {
-        const int mine = s0 + ks * kSliceSteps, nx = s0 + R;
-        if (nx < S) load_x(nx);                             // uniform
-        // (the digits go to LDS half way, which frees their registers)
-        if (mine < S)                                       // uniform
-            slice<NT, Sh::kPitch>(raw, min(kSliceSteps, S - mine), L.x[buf] + ks * kSliceBytes, A,
-                                  [&](int s) {
-                                      if (s == kSliceSteps / 2 && nx < S) put(buf ^ 1, nx);
-                                      load(s, mine + R + s);
-                                  });
-        else if (nx < S)
-            put(buf ^ 1, nx);
+    for (int it = 0; it < kRounds; ++it) {
+        const bool more = it + 1 < kRounds;
+        const int buf = it & 1, nx = s0 + R < S ? s0 + R : 0;
+        load_x(nx);
+        // (the digits go to LDS half way, which frees their registers; after the
+        // last round nothing reads them)
+        slice<NT, Sh::kPitch>(raw, L.x[buf] + ks * kSliceBytes, L.turn[wave], A, [&](int s) {
+            if (s == kSliceSteps / 2) put(buf ^ 1);
+            load(s, more ? nx + ks * kSliceSteps + s : S);
+        });
+        s0 = nx;
         barrier();
     }
     if constexpr (KS > 1) {
@@ -396,7 +444,7 @@ __device__ __forceinline__ void gemm(const uint16_t* wrow, XD&& xd,
                 for (int v = 0; v < 4; ++v) {
 #pragma unroll
                     for (int n = 0; n < NT; ++n) A.s[n][v] += L.part.s[wave + k][n][v][lane];
-                    A.es[v] += L.part.e[wave + k][0][v][lane];
+                    A.es[v] = fmaxf(A.es[v], L.part.e[wave + k][0][v][lane]);
                     A.er[v] += L.part.e[wave + k][1][v][lane];
                 }
         }

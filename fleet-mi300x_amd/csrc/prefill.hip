@@ -9,7 +9,7 @@
 // as in the decode kernels.
 //
 // Stepping reads every weight once per token (1.36 ms a step, 515 ms for 384
-// tokens); here a weight is read once per chunk (384 tokens: 26 ms). The projections run as exact
+// tokens); here a weight is read once per chunk (384 tokens: 24 ms). The projections run as exact
 // integer products of digits (digit_gemm.h), which keeps up with HBM; the
 // attention's own products (q_c, scores, the weighted sum, W_UV), whose operands
 // are fp32 or fp64, run on the fp64 matrix cores (v_mfma_f64_16x16x4): their
@@ -285,8 +285,7 @@ __device__ __forceinline__ int product(const uint16_t* W, int row0, int n_rows, 
     const int j = threadIdx.x & 15, first = row0 + 16 * (wave / KS);
     const uint16_t* w = W + (int64_t)min(first, n_rows - 16) * K;
     digit::Acc<NT> acc;
-    digit::gemm<K, NT, KS, NW>(w + (int64_t)j * K,
-                           [&](int i) { return X.d + (int64_t)row(min(i, m - 1)) * 3 * K; }, L,
+    digit::gemm<K, NT, KS, NW>(w, [&](int i) { return X.d + (int64_t)row(min(i, m - 1)) * 3 * K; }, L,
                            acc);
     if (wave % KS != 0 || first >= n_rows) return -1;
     digit::Meta meta[NT];
@@ -789,7 +788,7 @@ template <int K, int EPI>
 static void launch_proj(const uint16_t* W, int n_rows, const Rows& X, int T, uint16_t* out,
                         float* x, hipStream_t s) {
     if (T <= 64) launch_proj_as<K, 1, 4, EPI>(W, n_rows, X, T, out, x, s);
-    else if (T <= 192) launch_proj_as<K, 2, 2, EPI>(W, n_rows, X, T, out, x, s);
+    else if (T <= 256 || K > kHidden) launch_proj_as<K, 2, 2, EPI>(W, n_rows, X, T, out, x, s);
     else launch_proj_as<K, 3, 1, EPI>(W, n_rows, X, T, out, x, s);
 }
 
@@ -875,11 +874,12 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
     for (int c0 = 0; c0 < n_tokens; c0 += chunk) {
         const int T = n_tokens - c0 < chunk ? n_tokens - c0 : chunk;
         const int p0 = pos0 + c0;
-        // Up to 160 tokens an expert has 15 or fewer on average: blocks of 16 and
-        // workgroups of four waves, three to a CU (128 tokens: 16.2 ms, 17.2 in
-        // blocks of 48); beyond, blocks of 48, which split a weight once for all
-        // of them (256 tokens: 21.8 ms, 384: 26.3; in blocks of 32 21.9 and 27.8)
-        const bool small = T <= 160;
+        // Tokens per block of an expert. Narrow blocks take few registers and
+        // little LDS, so three (16) or two (32) workgroups of four waves share a
+        // CU; wide ones split a weight once for more tokens. Blocks of 16 / 32 /
+        // 48, ms: 128 tokens 13.9 / 14.8 / 15.4, 192: 17.5 / 17.3, 256: 21.4 / 20.3 /
+        // 21.0, 384: 27.9 / 25.7 / 25.7, 528: 37.7 / 33.4 / 32.5
+        const int block = T <= 176 ? 16 : T <= 400 ? 32 : 48;
         hipLaunchKernelGGL(embed_norm_kernel, dim3(T), dim3(kThreads), 0, stream, model->embed,
                            tokens + c0, layers[0].attn.norm_in, eps, x, norm_out, status);
         for (int i = 0; i < model->n_layers; ++i) {
@@ -917,7 +917,7 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
                                               dims, stream))
                 return e;
             hipLaunchKernelGGL(table_kernel, dim3(1), dim3(1024), 0, stream, ids, T * kTopK,
-                               small ? 16 : 48, tab, ent);
+                               block, tab, ent);
             ExpertParams P{};
             P.experts = l.moe.experts;
             P.stride = l.moe.expert_stride;
@@ -932,12 +932,12 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
             P.hs = hs;
             P.part = part;
             P.T = T;
-            if (small)
-                launch_experts<1, 1, 1, 4>(P, T * kTopK, bytes(L.hd), metas(L.hm), bytes(L.hsd),
-                                        metas(L.hsm), stream);
-            else
-                launch_experts<3, 1, 1, 8>(P, T * kTopK, bytes(L.hd), metas(L.hm), bytes(L.hsd),
-                                        metas(L.hsm), stream);
+            auto experts = [&](auto launch) {
+                launch(P, T * kTopK, bytes(L.hd), metas(L.hm), bytes(L.hsd), metas(L.hsm), stream);
+            };
+            if (block == 16) experts(launch_experts<1, 1, 1, 4>);
+            else if (block == 32) experts(launch_experts<2, 1, 1, 4>);
+            else experts(launch_experts<3, 1, 1, 8>);
             hipLaunchKernelGGL(combine_norm_kernel, dim3(T), dim3(kThreads), 0, stream, part, x,
                                next, eps, last ? no_out : norm_out);
         }

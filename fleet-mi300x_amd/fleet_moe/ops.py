@@ -481,10 +481,10 @@ class Decoder:
         self.reset(0)
         done = 0
         n = min(tokens.numel(), self.max_pos)
-        # from 6 tokens on: 4 take 6.5 ms together and 5.4 as steps, 8 take 7.8
-        # and 10.9, 384 take 26 and 515 (few tokens select nearly as many
-        # experts' weights, and leave most of a 16-token tile empty)
-        if self.fused and tokens.dim() == 1 and n >= 6:
+        # from 5 tokens on: 4 take 5.8 ms together and 5.2 as steps, 5 take 6.0
+        # and 6.4, 8 take 6.8 and 10.3, 384 take 24 and 515 (few tokens select
+        # nearly as many experts' weights, and leave most of a 16-token tile empty)
+        if self.fused and tokens.dim() == 1 and n >= 5:
             t = tokens[:n].to(device=self.blob.device, dtype=torch.int32).contiguous()
             rc = _lib.load().fleet_prefill(
                 ctypes.byref(self.step_model), self.step_rows, _ptr(t), n, 0, _ptr(self.x),
