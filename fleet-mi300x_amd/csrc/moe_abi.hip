@@ -1,17 +1,17 @@
 // C-ABI plumbing shared by the entry points, and the standalone router.
 //
 // fleet_moe_router_topk runs the router GEMV and the greedy top-k for any
-// number of tokens: one workgroup per token, four waves, 16 router rows per
-// wave with fp64 accumulation of the exact bf16 x bf16 products (so the logits
-// are the correctly rounded fp32 values and the routing is reproducible bit
-// for bit), then softmax + top-k on wave 0 with ties to the lowest index.
+// number of tokens: one workgroup per token, fp64 accumulation of the exact
+// bf16 x bf16 products (so the logits are the correctly rounded fp32 values and
+// the routing is reproducible bit for bit), then softmax + top-k on wave 0 with
+// ties to the lowest index.
 #include <stdio.h>
 #include <string.h>
 
 #include <mutex>
 #include <vector>
 
-#include "moe_common.h"
+#include "attn_body.h"
 
 namespace fleet_moe {
 
@@ -89,9 +89,15 @@ int check_resident_impl(const void* fn, int threads, int grid) {
 
 namespace router {
 
-constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / kLanes;
-constexpr int kRowsPerWave = kRouted / kWaves;   // 16
+// 131,072 products of fp64 accumulation per token bound it (a product, a
+// widening and an addition, ~17 cycles per 64 of them: 3.6 us on one CU), so
+// the workgroup fills the CU: 16 waves, wave w rows 8 (w / 2) .. + 7, half w % 2
+// of K, every load issued before the first product, and one reduction of eight
+// sums per wave. (Four waves of 16 rows, a load and a reduction at a time: 9.2
+// us for one token.)
+constexpr int kThreads = 1024;
+constexpr int kRowsPerWave = 8;
+constexpr int kHalf = kHidden / 2;
 
 struct Params {
     const u32x4* router;
@@ -100,44 +106,62 @@ struct Params {
     float* logits;           // fp32[T][64] or null
     int32_t* ids;            // int32[T][6]
     float* weights;          // fp32[T][6]
+    uint16_t* xb;            // bf16 bits of x [T][H], or null
     float scaling;
 };
 
 __global__ __launch_bounds__(kThreads) void router_topk_kernel(Params P) {
-    __shared__ float s_logit[kRouted];
+    __shared__ double s_part[2][kRouted];
     __shared__ int s_ids[8];
     __shared__ float s_w[8];
     const int t = blockIdx.x;
-    const int wave = threadIdx.x >> 6;
+    const int wave = threadIdx.x >> 6, half = wave & 1, row0 = kRowsPerWave * (wave >> 1);
     const int lane = threadIdx.x & (kLanes - 1);
-    const float* xt = P.x + (int64_t)t * kHidden;
-    float xr[4][8];
+    // lane: chunks lane and lane + 64 of its half
+    const float* xt = P.x + (int64_t)t * kHidden + half * kHalf;
+    float xr[2][8];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const float4 a = reinterpret_cast<const float4*>(xt)[2 * (lane + kLanes * m)];
-        const float4 b = reinterpret_cast<const float4*>(xt)[2 * (lane + kLanes * m) + 1];
+    for (int m = 0; m < 2; ++m) {
+        const float4* p = reinterpret_cast<const float4*>(xt) + 2 * (lane + kLanes * m);
+        const float4 a = p[0], b = p[1];
         xr[m][0] = a.x; xr[m][1] = a.y; xr[m][2] = a.z; xr[m][3] = a.w;
         xr[m][4] = b.x; xr[m][5] = b.y; xr[m][6] = b.z; xr[m][7] = b.w;
     }
-    for (int r = wave * kRowsPerWave; r < (wave + 1) * kRowsPerWave; ++r) {
-        const u32x4* row = P.router + (int64_t)r * kRowChunks;
-        double acc = 0.0;
+    u32x4 w[kRowsPerWave][2];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const u32x4 w = row[lane + kLanes * m];
-            const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
+    for (int r = 0; r < kRowsPerWave; ++r)
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+            w[r][m] = P.router[(int64_t)(row0 + r) * kRowChunks + half * (kRowChunks / 2) + lane +
+                               kLanes * m];
+    if (P.xb && row0 == 0) {
+        u32x4* o = reinterpret_cast<u32x4*>(P.xb + (int64_t)t * kHidden + half * kHalf);
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            u32x4 v;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                v[q] = bf16_bits(xr[m][2 * q]) | (bf16_bits(xr[m][2 * q + 1]) << 16);
+            o[lane + kLanes * m] = v;
+        }
+    }
+    double acc[kRowsPerWave];
+#pragma unroll
+    for (int r = 0; r < kRowsPerWave; ++r) {
+        acc[r] = 0.0;
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                acc += (double)(bf_lo(wv[q]) * xr[m][2 * q]);
-                acc += (double)(bf_hi(wv[q]) * xr[m][2 * q + 1]);
+                acc[r] += (double)(bf_lo(w[r][m][q]) * xr[m][2 * q]);
+                acc[r] += (double)(bf_hi(w[r][m][q]) * xr[m][2 * q + 1]);
             }
-        }
-        acc = wave_sum64(acc);
-        if (lane == 0) s_logit[r] = (float)acc;
     }
+    const double tot = attn::wave_msum64<kRowsPerWave>(acc);
+    s_part[half][row0 + msum_index<kRowsPerWave>(lane)] = tot;   // lanes of an index agree
     __syncthreads();
     if (wave == 0) {
-        const float l = s_logit[lane];
+        const float l = (float)(s_part[0][lane] + s_part[1][lane]);
         if (P.logits) P.logits[(int64_t)t * kRouted + lane] = l;
         wave_softmax_topk(l, kRouted, kTopK, P.scaling, s_ids, s_w, P.bias);
         // lanes < k read slots written by other lanes of this same wave
@@ -207,16 +231,15 @@ int fleet_moe_check_resident(const void* fn, int threads, int grid) {
 
 static bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
-extern "C" int fleet_moe_router_topk(const uint16_t* w_router, const float* x_norm,
-                                     int32_t n_tokens, const float* logit_bias, float* logits,
-                                     int32_t* ids, float* weights, const fleet_moe_dims* dims,
-                                     hipStream_t stream) {
+static int launch_router(const uint16_t* w_router, const float* x_norm, int32_t n_tokens,
+                         const float* logit_bias, float* logits, int32_t* ids, float* weights,
+                         uint16_t* x_bf16, const fleet_moe_dims* dims, hipStream_t stream) {
     if (int e = check_dims_impl(dims)) return e;
     if (!w_router || !x_norm || !ids || !weights || n_tokens < 1 || n_tokens > 65535)
         return FLEET_MOE_ERR_ARG;
     if (!aligned(w_router, 16) || !aligned(x_norm, 16) || !aligned(ids, 4) ||
         !aligned(weights, 4) || (logits && !aligned(logits, 4)) ||
-        (logit_bias && !aligned(logit_bias, 4)))
+        (logit_bias && !aligned(logit_bias, 4)) || (x_bf16 && !aligned(x_bf16, 16)))
         return FLEET_MOE_ERR_ARG;
     if (int e = check_device_impl(1)) return e;
     router::Params P;
@@ -226,10 +249,29 @@ extern "C" int fleet_moe_router_topk(const uint16_t* w_router, const float* x_no
     P.logits = logits;
     P.ids = ids;
     P.weights = weights;
+    P.xb = x_bf16;
     P.scaling = dims->routed_scaling;
     hipLaunchKernelGGL(router::router_topk_kernel, dim3(n_tokens), dim3(router::kThreads), 0,
                        stream, P);
     return (int)hipGetLastError();
+}
+
+extern "C" int fleet_moe_router_topk(const uint16_t* w_router, const float* x_norm,
+                                     int32_t n_tokens, const float* logit_bias, float* logits,
+                                     int32_t* ids, float* weights, const fleet_moe_dims* dims,
+                                     hipStream_t stream) {
+    return launch_router(w_router, x_norm, n_tokens, logit_bias, logits, ids, weights, nullptr, dims,
+                         stream);
+}
+
+extern "C" int fleet_moe_router_topk_bf16(const uint16_t* w_router, const float* x_norm,
+                                          int32_t n_tokens, const float* logit_bias,
+                                          float* logits, int32_t* ids, float* weights,
+                                          uint16_t* x_bf16, const fleet_moe_dims* dims,
+                                          hipStream_t stream) {
+    if (!x_bf16) return FLEET_MOE_ERR_ARG;
+    return launch_router(w_router, x_norm, n_tokens, logit_bias, logits, ids, weights, x_bf16, dims,
+                         stream);
 }
 
 extern "C" int fleet_moe_residual_fold(const float* x, const float* partials, int32_t n_partials,

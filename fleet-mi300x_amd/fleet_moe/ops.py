@@ -75,6 +75,13 @@ def route(layer: DeviceLayer, x_norm: torch.Tensor, logit_bias: torch.Tensor | N
           stream=None):
     """Router logits + greedy top-k for x_norm fp32 [T, H] (bf16-valued).
     Returns (logits fp32 [T, E], ids int32 [T, k], weights fp32 [T, k])."""
+    return _route(layer, x_norm, logit_bias, None, stream)
+
+
+def _route(layer: DeviceLayer, x_norm: torch.Tensor, logit_bias: torch.Tensor | None,
+           x_bits: torch.Tensor | None, stream):
+    """route(), which with `x_bits` (int16 [T, H]) also writes x_norm's bf16
+    bits there, in the same launch."""
     d = layer.dims
     T = x_norm.shape[0]
     _need(x_norm, torch.float32, (T, d.hidden), "x_norm")
@@ -85,10 +92,16 @@ def route(layer: DeviceLayer, x_norm: torch.Tensor, logit_bias: torch.Tensor | N
     ids = torch.empty((T, d.top_k), dtype=torch.int32, device=dev)
     ws = torch.empty((T, d.top_k), dtype=torch.float32, device=dev)
     dims = c_dims(d)
-    rc = _lib.load().fleet_moe_router_topk(layer.router_u16(), _ptr(x_norm), T, _ptr(logit_bias),
-                                           _ptr(logits), _ptr(ids), _ptr(ws), ctypes.byref(dims),
-                                           _stream(stream))
-    _lib.check(rc, "fleet_moe_router_topk")
+    lib = _lib.load()
+    args = (layer.router_u16(), _ptr(x_norm), T, _ptr(logit_bias), _ptr(logits), _ptr(ids),
+            _ptr(ws))
+    if x_bits is None:
+        rc = lib.fleet_moe_router_topk(*args, ctypes.byref(dims), _stream(stream))
+        _lib.check(rc, "fleet_moe_router_topk")
+    else:
+        rc = lib.fleet_moe_router_topk_bf16(*args, _ptr(x_bits), ctypes.byref(dims),
+                                            _stream(stream))
+        _lib.check(rc, "fleet_moe_router_topk_bf16")
     return logits, ids, ws
 
 
@@ -204,8 +217,9 @@ def f32_to_bf16_bits(t: torch.Tensor) -> torch.Tensor:
 def moe(layer: DeviceLayer, x_norm: torch.Tensor, runner: GroupedRunner, stream=None) -> dict:
     """reference_decode.moe for pre-normed tokens x_norm fp32 [T, H]: route,
     then the grouped product. Returns dict(logits, ids, weights, out bf16 bits)."""
-    logits, ids, ws = route(layer, x_norm, stream=stream)
-    out = runner.run(layer, f32_to_bf16_bits(x_norm), ids, ws, stream)
+    x_bits = torch.empty(x_norm.shape, dtype=torch.int16, device=x_norm.device)
+    logits, ids, ws = _route(layer, x_norm, None, x_bits, stream)
+    out = runner.run(layer, x_bits, ids, ws, stream)
     return {"logits": logits, "ids": ids, "weights": ws, "out": out}
 
 

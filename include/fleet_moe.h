@@ -80,6 +80,13 @@ int fleet_moe_router_topk(const uint16_t* router, const float* x_norm, int32_t n
                           const float* logit_bias, float* logits, int32_t* ids,
                           float* weights, const fleet_moe_dims* dims, hipStream_t stream);
 
+/* The same, and x_bf16 (bf16[n_tokens][hidden], 16-byte aligned) = x_norm rounded
+ * to bf16: the grouped step's input, from the launch that has x_norm at hand. */
+int fleet_moe_router_topk_bf16(const uint16_t* router, const float* x_norm, int32_t n_tokens,
+                               const float* logit_bias, float* logits, int32_t* ids,
+                               float* weights, uint16_t* x_bf16, const fleet_moe_dims* dims,
+                               hipStream_t stream);
+
 /* The residual fold of the NORM_ROUTER prologue (stage_residual_f32,
  * src/kernels/fleet_kernel.hip:107-144, called at :405-425): the post-
  * attention residual x[1] = bf16(x[0] + bf16(p_0 + ... + p_{n-1})) from the

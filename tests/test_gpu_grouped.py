@@ -273,3 +273,27 @@ def test_grouped_plans_share_a_workspace(dev):
     runner.run(layer, x, bad, ws)
     torch.cuda.synchronize()
     assert runner.status() == _lib.ABORT_BAD_ID
+
+
+@pytest.mark.parametrize("T", [1, 5, 84])
+def test_moe_equals_its_parts(dev, T):
+    """ops.moe (router, bf16 rounding in the router's launch, grouped step)
+    equals route + f32_to_bf16_bits + run bit for bit; the rounding also on
+    ties, signs, subnormals and non-finite values."""
+    layer, pl = dev
+    runner = ops.GroupedRunner(T, DSV2_LITE)
+    x = torch.from_numpy(orc.rms_norm(synth.hidden_inputs(300 + T, T))).cuda()
+    logits, ids, ws = ops.route(layer, x)
+    want = runner.run(layer, ops.f32_to_bf16_bits(x), ids, ws)
+    r = ops.moe(layer, x, runner)
+    torch.cuda.synchronize()
+    for a, b in ((r["logits"], logits), (r["ids"], ids), (r["weights"], ws), (r["out"], want)):
+        assert torch.equal(a, b)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    odd = torch.randint(-2**31, 2**31 - 1, (T, 2048), generator=g, device="cuda",
+                        dtype=torch.int64).to(torch.int32).view(torch.float32)
+    bits = torch.empty((T, 2048), dtype=torch.int16, device="cuda")
+    say("bf16 bits of arbitrary fp32 patterns")
+    ops._route(layer, odd, None, bits, None)
+    torch.cuda.synchronize()
+    assert torch.equal(bits, ops.f32_to_bf16_bits(odd))
