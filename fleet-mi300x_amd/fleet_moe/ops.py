@@ -21,9 +21,17 @@ from . import _lib
 from .layout import DSV2_LITE, Layout, MoeDims
 
 
+# The current stream's handle without a Stream object (0.1 us instead of 2.8,
+# of the 13 a routing call spent on the host); None where torch has no GPU.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream=None) -> int:
-    s = torch.cuda.current_stream() if stream is None else stream
-    return int(s.cuda_stream)
+    if stream is None:
+        if _raw_stream is not None:
+            return _raw_stream(torch.cuda.current_device())
+        stream = torch.cuda.current_stream()
+    return int(stream.cuda_stream)
 
 
 def c_dims(d: MoeDims) -> _lib.FleetMoeDims:
@@ -87,10 +95,9 @@ def _route(layer: DeviceLayer, x_norm: torch.Tensor, logit_bias: torch.Tensor | 
     _need(x_norm, torch.float32, (T, d.hidden), "x_norm")
     if logit_bias is not None:
         _need(logit_bias, torch.float32, (d.n_routed,), "logit_bias")
-    dev = x_norm.device
-    logits = torch.empty((T, d.n_routed), dtype=torch.float32, device=dev)
-    ids = torch.empty((T, d.top_k), dtype=torch.int32, device=dev)
-    ws = torch.empty((T, d.top_k), dtype=torch.float32, device=dev)
+    logits = x_norm.new_empty((T, d.n_routed))
+    ids = x_norm.new_empty((T, d.top_k), dtype=torch.int32)
+    ws = x_norm.new_empty((T, d.top_k))
     dims = c_dims(d)
     lib = _lib.load()
     args = (layer.router_u16(), _ptr(x_norm), T, _ptr(logit_bias), _ptr(logits), _ptr(ids),
