@@ -13,8 +13,8 @@
 // v_cvt_i32_f32 issue every 6 to 8 cycles), whatever the number of tokens. A SIMD's
 // share of HBM delivers those weights in 770: up to 16 tokens per expert the
 // stream runs at 5 TB/s, beyond that the vector ALU and the matrix cores bound it.
-// The 27-layer prompt of 384 tokens went from 50.7 ms on the fp64 cores to 24.0,
-// 64 tokens from 24.0 to 10.7.
+// The 27-layer prompt of 384 tokens went from 50.7 ms on the fp64 cores to 23.5,
+// 64 tokens from 24.0 to 10.0.
 //
 //   x (a token's row, K values): ix = round(x 2^sx), |ix| < 2^22, digits b2 b1
 //     b0 (ix = b2 2^16 + b1 2^8 + b0, |b2| <= 64, |b1|, |b0| <= 128), one

@@ -9,7 +9,7 @@
 // as in the decode kernels.
 //
 // Stepping reads every weight once per token (1.36 ms a step, 515 ms for 384
-// tokens); here a weight is read once per chunk (384 tokens: 24 ms). The projections run as exact
+// tokens); here a weight is read once per chunk (384 tokens: 23.5 ms). The projections run as exact
 // integer products of digits (digit_gemm.h), which keeps up with HBM; the
 // attention's own products (q_c, scores, the weighted sum, W_UV), whose operands
 // are fp32 or fp64, run on the fp64 matrix cores (v_mfma_f64_16x16x4): their
@@ -412,11 +412,14 @@ __global__ __launch_bounds__(kThreads) void qc_kernel(const uint16_t* qkv, const
     }
 }
 
+constexpr int kMlaWaves = 8;
+constexpr int kMlaPos = 16 * kMlaWaves;         // positions per round
+constexpr int kMlaCols = kLora / kMlaWaves;     // columns of c per wave: 64
 struct MlaLds {
     alignas(16) float q[kHeads][kQDimC + 4];
-    double p[kHeads][64 + 2];
-    double mx[kWaves][kHeads];
-    double ls[kWaves][kHeads];
+    double p[kHeads][kMlaPos + 2];
+    double mx[kMlaWaves][kHeads];
+    double ls[kMlaWaves][kHeads];
 };
 
 __device__ __forceinline__ double row_max64(double v) {
@@ -433,32 +436,35 @@ __device__ __forceinline__ double row_sum64(double v) {
 }
 
 // One token's 16 heads against cache rows 0 .. pos, all fp64 (the heads share
-// the cached rows, so they are the 16 rows of A). Per 64 positions: wave w
+// the cached rows, so they are the 16 rows of A). Per 128 positions: wave w
 // takes the scores of positions 16 w .. 16 w + 15 (144 MFMAs), the waves
-// agree on the heads' running maxima, then wave w adds the 64 positions'
-// exp(s - m) c into columns 128 w .. 128 w + 127 (128 MFMAs; a 16-byte load of
-// row k gives one B element of eight column tiles, column 8 j + e of tile e).
-// Tokens run from the last (the longest) to the first.
-__global__ __launch_bounds__(kThreads, 2) void mla_kernel(const float* q, const uint16_t* cache,
-                                                          int pos0, double scale, float* oc) {
+// agree on the heads' running maxima, then wave w adds the positions'
+// exp(s - m) c into columns 64 w .. 64 w + 63 (128 MFMAs; an 8-byte load of
+// row k gives one B element of four column tiles, column 4 j + e of tile e).
+// Tokens run from the last (the longest) to the first. A token is a serial
+// chain of rounds, and up to a few hundred tokens leave matrix cores free: eight
+// waves to a token instead of four halve its rounds (384 tokens: 99 -> 88 us).
+__global__ __launch_bounds__(64 * kMlaWaves, 2) void mla_kernel(const float* q,
+                                                                const uint16_t* cache, int pos0,
+                                                                double scale, float* oc) {
     __shared__ MlaLds S;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & (kLanes - 1), i = lane & 15, g = lane >> 4;
     const int t = (int)gridDim.x - 1 - (int)blockIdx.x, n_pos = pos0 + t + 1;
     const float4* qs = reinterpret_cast<const float4*>(q + (int64_t)t * kHeads * kQDimC);
-    for (int k = tid; k < kHeads * kQDimC / 4; k += kThreads) {
+    for (int k = tid; k < kHeads * kQDimC / 4; k += 64 * kMlaWaves) {
         const int h = k / (kQDimC / 4), c = k - h * (kQDimC / 4);
         *reinterpret_cast<float4*>(&S.q[h][4 * c]) = qs[k];
     }
     double m[4], l[4];
-    f64x4 o[8];
+    f64x4 o[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) { m[v] = -INFINITY; l[v] = 0.0; }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int e = 0; e < 4; ++e) o[e] = f64x4{0.0, 0.0, 0.0, 0.0};
     __syncthreads();
-    for (int base = 0; base < n_pos; base += 64) {
+    for (int base = 0; base < n_pos; base += kMlaPos) {
         const int pos = base + 16 * wave + i;
         f64x4 s = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
         if (base + 16 * wave < n_pos) {
@@ -491,24 +497,26 @@ __global__ __launch_bounds__(kThreads, 2) void mla_kernel(const float* q, const 
         for (int v = 0; v < 4; ++v) {
             double mn = m[v];
 #pragma unroll
-            for (int w = 0; w < kWaves; ++w) mn = fmax(mn, S.mx[w][4 * v + g]);
+            for (int w = 0; w < kMlaWaves; ++w) mn = fmax(mn, S.mx[w][4 * v + g]);
             const double f = exp(m[v] - mn), p = exp(s[v] - mn);
             m[v] = mn;
             l[v] = fma(l[v], f, p);
             S.p[4 * v + g][16 * wave + i] = p;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) o[e][v] *= f;
+            for (int e = 0; e < 4; ++e) o[e][v] *= f;
         }
         __syncthreads();
-        const int ks = min(16, (n_pos - base + 3) >> 2);
-        const u32x4* col = reinterpret_cast<const u32x4*>(cache + 128 * wave) + i;
-        u32x4 b = ld_global(col + (int64_t)min(base + g, n_pos - 1) * (kRowElems / kChunk));
+        const int ks = min(kMlaPos / 4, (n_pos - base + 3) >> 2);
+        const uint16_t* col = cache + kMlaCols * wave;
+        uint2 b = ld_global_u2(col + (int64_t)min(base + g, n_pos - 1) * kRowElems, i);
         for (int k = 0; k < ks; ++k) {
-            const u32x4 nb = ld_global(col + (int64_t)min(base + 4 * (k + 1) + g, n_pos - 1) *
-                                                 (kRowElems / kChunk));
+            const uint2 nb =
+                ld_global_u2(col + (int64_t)min(base + 4 * (k + 1) + g, n_pos - 1) * kRowElems, i);
             const double a = S.p[i][4 * k + g];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = mfma64(a, widen(b, e), o[e]);
+            o[0] = mfma64(a, (double)bf_lo(b.x), o[0]);
+            o[1] = mfma64(a, (double)bf_hi(b.x), o[1]);
+            o[2] = mfma64(a, (double)bf_lo(b.y), o[2]);
+            o[3] = mfma64(a, (double)bf_hi(b.y), o[3]);
             b = nb;
         }
     }
@@ -521,49 +529,42 @@ __global__ __launch_bounds__(kThreads, 2) void mla_kernel(const float* q, const 
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         const int h = 4 * v + g;
-        const double Ls = (S.ls[0][h] + S.ls[1][h]) + (S.ls[2][h] + S.ls[3][h]);
-        float r[8];
+        double Ls = 0.0;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) r[e] = (float)(o[e][v] / Ls);
-        store8(oc + ((int64_t)t * kHeads + h) * kLora + 128 * wave + 8 * i, r);
+        for (int w = 0; w < kMlaWaves; ++w) Ls += S.ls[w][h];
+        *reinterpret_cast<float4*>(oc + ((int64_t)t * kHeads + h) * kLora + kMlaCols * wave + 4 * i) =
+            make_float4((float)(o[0][v] / Ls), (float)(o[1][v] / Ls), (float)(o[2][v] / Ls),
+                        (float)(o[3][v] / Ls));
     }
 }
 
-// Head outputs bf16(W_UV o_c), exact. Grid (token blocks of 32, heads, halves
-// of the 128 rows), a wave per 16 rows.
+// Head outputs bf16(W_UV o_c), exact. Grid (token blocks of 16, heads, halves
+// of the 128 rows), a wave per 16 rows; bound by the chain of its MFMAs, so
+// even and odd k add into sums of their own, and blocks are small (384 tokens:
+// 25 us with blocks of 32, now 20).
 __global__ __launch_bounds__(kThreads) void uv_kernel(const float* oc, const uint16_t* kv_b, int T,
                                                       uint16_t* heads) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
-    const int h = blockIdx.y, row0 = 64 * blockIdx.z + 16 * wave, t0 = 32 * blockIdx.x;
+    const int h = blockIdx.y, row0 = 64 * blockIdx.z + 16 * wave, t = 16 * blockIdx.x + i;
     const u32x4* wp = reinterpret_cast<const u32x4*>(
         kv_b + ((int64_t)h * attn::kKvbRowsPerHead + kNope + row0 + perm16(i)) * kLora) + q;
-    const float* xp[2];
-#pragma unroll
-    for (int n = 0; n < 2; ++n)
-        xp[n] = oc + ((int64_t)min(t0 + 16 * n + i, T - 1) * kHeads + h) * kLora + 8 * q;
+    const float* xp = oc + ((int64_t)min(t, T - 1) * kHeads + h) * kLora + 8 * q;
     f64x4 acc[2] = {f64x4{0.0, 0.0, 0.0, 0.0}, f64x4{0.0, 0.0, 0.0, 0.0}};
-#pragma unroll 2
+#pragma unroll 4
     for (int s = 0; s < kLora / 32; ++s) {
         const u32x4 a = ld_global(wp + 4 * s);
-        float x[2][8];
+        float x[8];
+        load8(xp + 32 * s, x);
 #pragma unroll
-        for (int n = 0; n < 2; ++n) load8(xp[n] + 32 * s, x[n]);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const double w = widen(a, e);
-#pragma unroll
-            for (int n = 0; n < 2; ++n) acc[n] = mfma64(w, (double)x[n][e], acc[n]);
-        }
+        for (int e = 0; e < 8; ++e) acc[e & 1] = mfma64(widen(a, e), (double)x[e], acc[e & 1]);
     }
+    if (t >= T) return;
+    float d[4];
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {
-        const int t = t0 + 16 * n + i;
-        if (t >= T) continue;
-        *reinterpret_cast<uint2*>(heads + ((int64_t)t * kHeads + h) * kV + row0 + 4 * q) =
-            make_uint2(bf16_bits((float)acc[n][0]) | (bf16_bits((float)acc[n][1]) << 16),
-                       bf16_bits((float)acc[n][2]) | (bf16_bits((float)acc[n][3]) << 16));
-    }
+    for (int v = 0; v < 4; ++v) d[v] = (float)(acc[0][v] + acc[1][v]);
+    *reinterpret_cast<uint2*>(heads + ((int64_t)t * kHeads + h) * kV + row0 + 4 * q) =
+        make_uint2(pack2(d[0], d[1]), pack2(d[2], d[3]));
 }
 
 // ---------------------------------------------------------------- experts
@@ -783,11 +784,15 @@ static void launch_proj_as(const uint16_t* W, int n_rows, const Rows& X, int T, 
 
 // A projection over T tokens. Few tokens leave few workgroups, so four waves
 // share a row tile's K (16 KB of weights each instead of 64: at 8 tokens qkv
-// 33 -> 13 us, o_proj 29 -> 13); many give the CUs enough to do without.
+// 33 -> 13 us, o_proj 29 -> 13); many give the CUs enough to do without. With
+// 33 to 64 tokens, 2 waves suit the wide ones (qkv 25 -> 20 us at 64), 4 the
+// 2048 rows of o_proj and down (14 against 18).
 template <int K, int EPI>
 static void launch_proj(const uint16_t* W, int n_rows, const Rows& X, int T, uint16_t* out,
                         float* x, hipStream_t s) {
-    if (T <= 64) launch_proj_as<K, 1, 4, EPI>(W, n_rows, X, T, out, x, s);
+    if (T <= 32 || (T <= 64 && n_rows <= kHidden))
+        launch_proj_as<K, 1, 4, EPI>(W, n_rows, X, T, out, x, s);
+    else if (T <= 64) launch_proj_as<K, 1, 2, EPI>(W, n_rows, X, T, out, x, s);
     else if (T <= 256 || K > kHidden) launch_proj_as<K, 2, 2, EPI>(W, n_rows, X, T, out, x, s);
     else launch_proj_as<K, 3, 1, EPI>(W, n_rows, X, T, out, x, s);
 }
@@ -890,9 +895,9 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
                                l.cache, q);
             hipLaunchKernelGGL(qc_kernel, dim3((T + 15) / 16, kHeads), dim3(kThreads), 0, stream,
                                qkv, l.attn.kv_b, T, q);
-            hipLaunchKernelGGL(mla_kernel, dim3(T), dim3(kThreads), 0, stream, q, l.cache, p0,
+            hipLaunchKernelGGL(mla_kernel, dim3(T), dim3(64 * kMlaWaves), 0, stream, q, l.cache, p0,
                                scale, oc);
-            hipLaunchKernelGGL(uv_kernel, dim3((T + 31) / 32, kHeads, 2), dim3(kThreads), 0,
+            hipLaunchKernelGGL(uv_kernel, dim3((T + 15) / 16, kHeads, 2), dim3(kThreads), 0,
                                stream, oc, l.attn.kv_b, T, heads);
             launch_digits<kHeads * kV>(heads, T, bytes(L.headsd), metas(L.headsm), stream);
             launch_proj<kHeads * kV, kEpiResidual>(l.attn.o_proj, kHidden, headsr, T, nullptr, x,
