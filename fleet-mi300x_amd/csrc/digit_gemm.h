@@ -13,8 +13,8 @@
 // v_cvt_i32_f32 issue every 6 to 8 cycles), whatever the number of tokens. A SIMD's
 // share of HBM delivers those weights in 770: up to 16 tokens per expert the
 // stream runs at 5 TB/s, beyond that the vector ALU and the matrix cores bound it.
-// The 27-layer prompt of 384 tokens went from 50.7 ms on the fp64 cores to 23.5,
-// 64 tokens from 24.0 to 10.0.
+// The 27-layer prompt of 384 tokens went from 50.7 ms on the fp64 cores to 23.2,
+// 64 tokens from 24.0 to 9.5.
 //
 //   x (a token's row, K values): ix = round(x 2^sx), |ix| < 2^22, digits b2 b1
 //     b0 (ix = b2 2^16 + b1 2^8 + b0, |b2| <= 64, |b1|, |b0| <= 128), one
@@ -143,13 +143,11 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
     return v;
 }
 
-// One wave per row of K values.
+// The digits of one row of K values, by one wave.
 template <int K>
-__global__ __launch_bounds__(256) void digits_kernel(const uint16_t* x, int rows, uint8_t* out,
-                                                     Meta* meta) {
+__device__ __forceinline__ void digits_of_row(const uint16_t* x, int row, uint8_t* out, Meta* meta) {
     constexpr int C = K / kChunk, G = (C + kLanes - 1) / kLanes;
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & (kLanes - 1);
-    if (row >= rows) return;
+    const int lane = threadIdx.x & (kLanes - 1);
     const u32x4* src = reinterpret_cast<const u32x4*>(x + (int64_t)row * K);
     u32x4 c[G];
     uint32_t mx = 0;
@@ -173,6 +171,29 @@ __global__ __launch_bounds__(256) void digits_kernel(const uint16_t* x, int rows
     sb0 = wave_sum(sb0);
     res = wave_sum(res);
     if (lane == 0) meta[row] = make_meta(mx, ok, sx, sb0, res);
+}
+
+// Four rows of K values per workgroup.
+template <int K>
+__global__ __launch_bounds__(256) void digits_kernel(const uint16_t* x, int rows, uint8_t* out,
+                                                     Meta* meta) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row < rows) digits_of_row<K>(x, row, out, meta);
+}
+
+// Two operands in one launch, workgroups of a's rows first: either alone is
+// the 5 us that an empty launch takes here.
+struct Operand {
+    const uint16_t* x;
+    int rows;
+    uint8_t* d;
+    Meta* m;
+};
+template <int KA, int KB>
+__global__ __launch_bounds__(256) void digits2_kernel(Operand a, Operand b) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), rows_a = (a.rows + 3) & ~3;
+    if (row < a.rows) digits_of_row<KA>(a.x, row, a.d, a.m);
+    else if (row >= rows_a && row - rows_a < b.rows) digits_of_row<KB>(b.x, row - rows_a, b.d, b.m);
 }
 
 // ---------------------------------------------------------------- the GEMM

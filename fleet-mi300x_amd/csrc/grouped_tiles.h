@@ -14,7 +14,8 @@
 // R = 2, NT = 4 (128 KB of weights in flight per CU): 256 tokens in 285 us; with
 // R = 1 and NT = 3: 335; NT = 2, R = 2: 292, but 332 against 272 under Zipf
 // routing, whose popular experts fill blocks of 64. Persistent workgroups that
-// carry the stream across tiles: 358. The start's plan: 468.
+// carry the stream across tiles: 358. The plan for fewer tokens: 468. With one K
+// step ahead (R = 1) in the down launch alone: 300.
 //
 // Launches: the tables (one workgroup), gate / up + SwiGLU, down + routing weight,
 // combine; data crosses them as plain memory.

@@ -9,7 +9,7 @@
 // as in the decode kernels.
 //
 // Stepping reads every weight once per token (1.36 ms a step, 515 ms for 384
-// tokens); here a weight is read once per chunk (384 tokens: 23.5 ms). The projections run as exact
+// tokens); here a weight is read once per chunk (384 tokens: 23.2 ms). The projections run as exact
 // integer products of digits (digit_gemm.h), which keeps up with HBM; the
 // attention's own products (q_c, scores, the weighted sum, W_UV), whose operands
 // are fp32 or fp64, run on the fp64 matrix cores (v_mfma_f64_16x16x4): their
@@ -335,13 +335,15 @@ __global__ __launch_bounds__(512) void proj_kernel(const uint16_t* W, int n_rows
 // ---------------------------------------------------------------- attention
 
 // Per token: the cache row (kv_a_layernorm of c, RoPE of k_pe) and q_pe.
-__global__ __launch_bounds__(kThreads) void rope_cache_kernel(const uint16_t* qkv,
-                                                              const uint16_t* gamma, float eps,
-                                                              const float* cos, const float* sin,
-                                                              int pos0, uint16_t* cache, float* q) {
-    __shared__ float v[kQkvRows];
-    __shared__ double red[kWaves];
-    const int t = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & (kLanes - 1);
+struct RopeLds {
+    float v[kQkvRows];
+    double red[kWaves];
+};
+__device__ void rope_cache(int t, const uint16_t* qkv, const uint16_t* gamma, float eps,
+                           const float* cos, const float* sin, int pos0, uint16_t* cache, float* q,
+                           RopeLds& S) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & (kLanes - 1);
+    float* v = S.v;
     const int64_t pos = pos0 + t;
     const uint16_t* src = qkv + (int64_t)t * kQkvRows;
     for (int k = tid; k < kQkvRows / 2; k += kThreads) {
@@ -353,11 +355,11 @@ __global__ __launch_bounds__(kThreads) void rope_cache_kernel(const uint16_t* qk
     uint16_t* row = cache + pos * kRowElems;
     const float c0 = v[kQDim + tid], c1 = v[kQDim + kThreads + tid];
     const double ss = wave_sum64((double)c0 * c0 + (double)c1 * c1);
-    if (lane == 0) red[wave] = ss;
+    if (lane == 0) S.red[wave] = ss;
     __syncthreads();
     double ssq = 0.0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) ssq += red[w];
+    for (int w = 0; w < kWaves; ++w) ssq += S.red[w];
     const float inv = __fdiv_rn(1.0f, sqrt_rn((float)(ssq / (double)kLora) + eps));
     const float g0 = gamma ? bf_lo(gamma[tid]) : 1.f, g1 = gamma ? bf_lo(gamma[kThreads + tid]) : 1.f;
     row[tid] = (uint16_t)bf16_bits(bf16r(bf16r(c0 * inv) * g0));
@@ -372,44 +374,55 @@ __global__ __launch_bounds__(kThreads) void rope_cache_kernel(const uint16_t* qk
     }
 }
 
-// q_c = W_UK^T q_nope, exact, rounded once to fp32. A wave: 128 columns of one
-// head x 16 tokens; lane group q sums k = 32 q .. 32 q + 31, a 16-byte load of
-// row k gives one A element of eight column tiles (column 8 i + e of tile e).
-// Grid (token blocks of 16, heads), a wave per 128 columns.
-__global__ __launch_bounds__(kThreads) void qc_kernel(const uint16_t* qkv, const uint16_t* kv_b,
-                                                      int T, float* q_out) {
+// q_c = W_UK^T q_nope, exact, rounded once to fp32. A wave: 64 columns of one
+// head x 16 tokens; lane group q sums k = 32 q .. 32 q + 31, an 8-byte load of
+// row k gives one A element of four column tiles (column 4 i + e of tile e).
+// A workgroup: half of one head's columns for token block `block`. Bound by a
+// wave's chain of MFMAs (64 cycles each), so a wave has 128 of them and all its
+// weights in flight (8 / 384 tokens, with the launch of rope_cache: 16.0 / 27.1 us
+// with 128 columns a wave, now 8.3 / 21.4).
+__device__ void qc_block(int block, int h, int half, const uint16_t* qkv, const uint16_t* kv_b,
+                         int T, float* q_out) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
-    const int h = blockIdx.y, t = 16 * blockIdx.x + i;
+    const int t = 16 * block + i, col = kLora / 2 * half + 64 * wave;
+    const uint16_t* wk = kv_b + ((int64_t)h * attn::kKvbRowsPerHead + 32 * q) * kLora + col;
+    uint2 a[32];
+#pragma unroll
+    for (int k = 0; k < 32; ++k) a[k] = ld_global_u2(wk + k * kLora, i);
     const uint16_t* xq = qkv + (int64_t)min(t, T - 1) * kQkvRows + h * (kNope + kRope) + 32 * q;
     u32x4 b[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) b[m] = reinterpret_cast<const u32x4*>(xq)[m];
-    const u32x4* wk = reinterpret_cast<const u32x4*>(
-        kv_b + ((int64_t)h * attn::kKvbRowsPerHead + 32 * q) * kLora + 128 * wave) + i;
-    f64x4 acc[8];
+    __builtin_amdgcn_sched_barrier(0);
+    f64x4 acc[4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int e = 0; e < 4; ++e) acc[e] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        u32x4 a[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) a[e] = ld_global(wk + (8 * m + e) * (kLora / kChunk));
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const double x = widen(b[m], k);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[e] = mfma64(widen(a[k], e), x, acc[e]);
-        }
+    for (int k = 0; k < 32; ++k) {
+        const double x = widen(b[k / 8], k % 8);
+        acc[0] = mfma64((double)bf_lo(a[k].x), x, acc[0]);
+        acc[1] = mfma64((double)bf_hi(a[k].x), x, acc[1]);
+        acc[2] = mfma64((double)bf_lo(a[k].y), x, acc[2]);
+        acc[3] = mfma64((double)bf_hi(a[k].y), x, acc[3]);
     }
     if (t >= T) return;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        float o[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = (float)acc[e][v];
-        store8(q_out + ((int64_t)t * kHeads + h) * kQDimC + 128 * wave + 8 * (4 * v + q), o);
-    }
+    for (int v = 0; v < 4; ++v)
+        *reinterpret_cast<float4*>(q_out + ((int64_t)t * kHeads + h) * kQDimC + col + 4 * (4 * v + q)) =
+            make_float4((float)acc[0][v], (float)acc[1][v], (float)acc[2][v], (float)acc[3][v]);
+}
+
+// Both read the projection only, so they share a launch (rope_cache alone is
+// the 5 us of an empty one): workgroups of q_c first, then one per token.
+__global__ __launch_bounds__(kThreads, 2) void qc_rope_kernel(const uint16_t* qkv, const uint16_t* kv_b,
+                                                           const uint16_t* gamma, float eps,
+                                                           const float* cos, const float* sin, int T,
+                                                           int pos0, uint16_t* cache, float* q) {
+    __shared__ RopeLds S;
+    const int n_qc = (T + 15) / 16 * 2 * kHeads, b = blockIdx.x;
+    if (b < n_qc) qc_block(b / (2 * kHeads), b % kHeads, b / kHeads % 2, qkv, kv_b, T, q);
+    else rope_cache(b - n_qc, qkv, gamma, eps, cos, sin, pos0, cache, q, S);
 }
 
 constexpr int kMlaWaves = 8;
@@ -538,31 +551,45 @@ __global__ __launch_bounds__(64 * kMlaWaves, 2) void mla_kernel(const float* q,
     }
 }
 
-// Head outputs bf16(W_UV o_c), exact. Grid (token blocks of 16, heads, halves
-// of the 128 rows), a wave per 16 rows; bound by the chain of its MFMAs, so
-// even and odd k add into sums of their own, and blocks are small (384 tokens:
-// 25 us with blocks of 32, now 20).
+// Head outputs bf16(W_UV o_c), exact. Grid (token blocks of 16, heads, quarters
+// of the 128 rows), two waves per 16 rows, each with half of K: bound by the
+// wave's chain of MFMAs (64 of 64 cycles each), all of whose operands are in
+// flight at once (8 / 64 / 384 tokens: 12.4 / 12.9 / 20.1 us with two K halves
+// in one wave and a few loads in flight, now 6.0 / 6.8 / 22.2).
 __global__ __launch_bounds__(kThreads) void uv_kernel(const float* oc, const uint16_t* kv_b, int T,
                                                       uint16_t* heads) {
+    __shared__ double part[2][4][kLanes];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
-    const int h = blockIdx.y, row0 = 64 * blockIdx.z + 16 * wave, t = 16 * blockIdx.x + i;
+    const int h = blockIdx.y, row0 = 32 * blockIdx.z + 16 * (wave & 1), half = wave >> 1;
+    const int t = 16 * blockIdx.x + i;
+    constexpr int kN = kLora / 64;          // 32-K loads per wave
     const u32x4* wp = reinterpret_cast<const u32x4*>(
-        kv_b + ((int64_t)h * attn::kKvbRowsPerHead + kNope + row0 + perm16(i)) * kLora) + q;
-    const float* xp = oc + ((int64_t)min(t, T - 1) * kHeads + h) * kLora + 8 * q;
-    f64x4 acc[2] = {f64x4{0.0, 0.0, 0.0, 0.0}, f64x4{0.0, 0.0, 0.0, 0.0}};
-#pragma unroll 4
-    for (int s = 0; s < kLora / 32; ++s) {
-        const u32x4 a = ld_global(wp + 4 * s);
-        float x[8];
-        load8(xp + 32 * s, x);
+        kv_b + ((int64_t)h * attn::kKvbRowsPerHead + kNope + row0 + perm16(i)) * kLora +
+        kLora / 2 * half) + q;
+    const float* xp = oc + ((int64_t)min(t, T - 1) * kHeads + h) * kLora + kLora / 2 * half + 8 * q;
+    u32x4 a[kN];
+    float x[kN][8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e & 1] = mfma64(widen(a, e), (double)x[e], acc[e & 1]);
+    for (int s = 0; s < kN; ++s) {
+        a[s] = ld_global(wp + 4 * s);
+        load8(xp + 32 * s, x[s]);
     }
-    if (t >= T) return;
+    __builtin_amdgcn_sched_barrier(0);
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < kN; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc = mfma64(widen(a[s], e), (double)x[s][e], acc);
+    if (half == 1) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) part[wave & 1][v][lane] = acc[v];
+    }
+    __syncthreads();
+    if (half == 1 || t >= T) return;
     float d[4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) d[v] = (float)(acc[0][v] + acc[1][v]);
+    for (int v = 0; v < 4; ++v) d[v] = (float)(acc[v] + part[wave][v][lane]);
     *reinterpret_cast<uint2*>(heads + ((int64_t)t * kHeads + h) * kV + row0 + 4 * q) =
         make_uint2(pack2(d[0], d[1]), pack2(d[2], d[3]));
 }
@@ -758,10 +785,9 @@ static void launch_experts(ExpertParams P, int n, uint8_t* hd, digit::Meta* hm, 
     hipLaunchKernelGGL((gate_up_kernel<NTM, KG, NW>),
                        dim3(P.routed_wgs + sb * (2 * kSharedInter / kGRows)),
                        dim3(64 * NW), 0, s, P);
-    hipLaunchKernelGGL((digit::digits_kernel<kInter>), dim3((n + 3) / 4), dim3(256), 0, s, P.h, n,
-                       hd, hm);
-    hipLaunchKernelGGL((digit::digits_kernel<kSharedInter>), dim3((P.T + 3) / 4), dim3(256), 0, s,
-                       P.hs, P.T, hsd, hsm);
+    hipLaunchKernelGGL((digit::digits2_kernel<kInter, kSharedInter>),
+                       dim3((n + 3) / 4 + (P.T + 3) / 4), dim3(256), 0, s,
+                       digit::Operand{P.h, n, hd, hm}, digit::Operand{P.hs, P.T, hsd, hsm});
     P.routed_wgs = bx * (kHidden / kDRows);
     hipLaunchKernelGGL((down_kernel<NTM, KD, NW>), dim3(P.routed_wgs + sb * (kHidden / kDRows)),
                        dim3(64 * NW), 0, s, P);
@@ -890,14 +916,12 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
         for (int i = 0; i < model->n_layers; ++i) {
             const fleet_step_layer& l = layers[i];
             launch_proj<kHidden, kEpiBf16>(l.attn.qkv, kQkvRows, xr, T, qkv, nullptr, stream);
-            hipLaunchKernelGGL(rope_cache_kernel, dim3(T), dim3(kThreads), 0, stream, qkv,
-                               l.attn.kv_a_norm, eps, model->rope_cos, model->rope_sin, p0,
-                               l.cache, q);
-            hipLaunchKernelGGL(qc_kernel, dim3((T + 15) / 16, kHeads), dim3(kThreads), 0, stream,
-                               qkv, l.attn.kv_b, T, q);
+            hipLaunchKernelGGL(qc_rope_kernel, dim3((T + 15) / 16 * 2 * kHeads + T), dim3(kThreads), 0,
+                               stream, qkv, l.attn.kv_b, l.attn.kv_a_norm, eps, model->rope_cos,
+                               model->rope_sin, T, p0, l.cache, q);
             hipLaunchKernelGGL(mla_kernel, dim3(T), dim3(64 * kMlaWaves), 0, stream, q, l.cache, p0,
                                scale, oc);
-            hipLaunchKernelGGL(uv_kernel, dim3((T + 15) / 16, kHeads, 2), dim3(kThreads), 0,
+            hipLaunchKernelGGL(uv_kernel, dim3((T + 15) / 16, kHeads, 4), dim3(kThreads), 0,
                                stream, oc, l.attn.kv_b, T, heads);
             launch_digits<kHeads * kV>(heads, T, bytes(L.headsd), metas(L.headsm), stream);
             launch_proj<kHeads * kV, kEpiResidual>(l.attn.o_proj, kHidden, headsr, T, nullptr, x,
