@@ -425,6 +425,7 @@ __global__ __launch_bounds__(kThreads, 2) void qc_rope_kernel(const uint16_t* qk
     else rope_cache(b - n_qc, qkv, gamma, eps, cos, sin, pos0, cache, q, S);
 }
 
+constexpr int kCus = 256;
 constexpr int kMlaWaves = 8;
 constexpr int kMlaPos = 16 * kMlaWaves;         // positions per round
 constexpr int kMlaCols = kLora / kMlaWaves;     // columns of c per wave: 64
@@ -454,9 +455,12 @@ __device__ __forceinline__ double row_sum64(double v) {
 // agree on the heads' running maxima, then wave w adds the positions'
 // exp(s - m) c into columns 64 w .. 64 w + 63 (128 MFMAs; an 8-byte load of
 // row k gives one B element of four column tiles, column 4 j + e of tile e).
-// Tokens run from the last (the longest) to the first. A token is a serial
+// Tokens run from the last (the longest) to the first up to 256. A token is a serial
 // chain of rounds, and up to a few hundred tokens leave matrix cores free: eight
 // waves to a token instead of four halve its rounds (384 tokens: 99 -> 88 us).
+// Past one token per CU, the workgroups that start second are the shortest and
+// join CUs that hold middling ones; the longest have theirs alone (88 -> 76; 528
+// tokens of a prompt 29.9 -> 29.0 ms).
 __global__ __launch_bounds__(64 * kMlaWaves, 2) void mla_kernel(const float* q,
                                                                 const uint16_t* cache, int pos0,
                                                                 double scale, float* oc) {
@@ -464,7 +468,8 @@ __global__ __launch_bounds__(64 * kMlaWaves, 2) void mla_kernel(const float* q,
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & (kLanes - 1), i = lane & 15, g = lane >> 4;
-    const int t = (int)gridDim.x - 1 - (int)blockIdx.x, n_pos = pos0 + t + 1;
+    const int T = (int)gridDim.x, b = blockIdx.x;
+    const int t = T > kCus && b < kCus ? T - kCus + b : T - 1 - b, n_pos = pos0 + t + 1;
     const float4* qs = reinterpret_cast<const float4*>(q + (int64_t)t * kHeads * kQDimC);
     for (int k = tid; k < kHeads * kQDimC / 4; k += 64 * kMlaWaves) {
         const int h = k / (kQDimC / 4), c = k - h * (kQDimC / 4);
