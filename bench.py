@@ -489,9 +489,9 @@ def bench_column(torch, dev, stream, dims, n_tok: int = 32, warm: int = 4):
 def bench_decode(torch, dev, stream, dims, prompt_len: int = 1024, n_gen: int = 32):
     """Config 4: the full 27-layer model (absorbed-MLA attention, dense layer
     0, 26 MoE layers, lm_head + greedy argmax) at batch 1, weights drawn on the
-    device. The KV cache is prefilled by teacher-forced steps over a seeded
-    uniform prompt of 1024 tokens, then 32 greedy tokens are generated; each
-    step is one replay of the captured HIP graph of the step (the token and
+    device. The KV cache is prefilled with a seeded uniform prompt of 1024
+    tokens (Decoder.prefill, whose rows equal those of steps), then 32 greedy
+    tokens are generated; each step is one replay of the captured HIP graph of the step (the token and
     the position live on the device, the argmax feeds both forward). The step
     is one launch (fleet_decode_step); the same 32 tokens are also timed with
     one launch per stage (embed, per layer attention and FFN, lm_head,
