@@ -502,10 +502,10 @@ class Decoder:
         self.reset(0)
         done = 0
         n = min(tokens.numel(), self.max_pos)
-        # from 5 tokens on: 4 take 5.8 ms together and 5.2 as steps, 5 take 6.0
-        # and 6.4, 8 take 6.8 and 10.3, 384 take 24 and 515 (few tokens select
+        # from 4 tokens on: 3 take 4.7 ms together and 3.9 as steps, 4 take 5.0
+        # and 5.2, 8 take 6.0 and 10.4, 384 take 23 and 514 (few tokens select
         # nearly as many experts' weights, and leave most of a 16-token tile empty)
-        if self.fused and tokens.dim() == 1 and n >= 5:
+        if self.fused and tokens.dim() == 1 and n >= 4:
             t = tokens[:n].to(device=self.blob.device, dtype=torch.int32).contiguous()
             rc = _lib.load().fleet_prefill(
                 ctypes.byref(self.step_model), self.step_rows, _ptr(t), n, 0, _ptr(self.x),
