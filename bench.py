@@ -491,9 +491,9 @@ def bench_decode(torch, dev, stream, dims, prompt_len: int = 1024, n_gen: int = 
     0, 26 MoE layers, lm_head + greedy argmax) at batch 1, weights drawn on the
     device. The KV cache is prefilled with a seeded uniform prompt of 1024
     tokens (Decoder.prefill, whose rows equal those of steps), then 32 greedy
-    tokens are generated; each step is one replay of the captured HIP graph of the step (the token and
-    the position live on the device, the argmax feeds both forward). The step
-    is one launch (fleet_decode_step); the same 32 tokens are also timed with
+    tokens are generated; each step is one replay of the captured HIP graph of
+    the step (the token and the position live on the device, the argmax feeds
+    both forward). The step is one launch (fleet_decode_step); the same 32 tokens are also timed with
     one launch per stage (embed, per layer attention and FFN, lm_head,
     argmax) for comparison."""
     from fleet_moe import layout as lay_mod, ops, synth_gpu

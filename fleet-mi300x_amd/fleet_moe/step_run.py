@@ -2,8 +2,9 @@
 
 The full-decode leg of bench.py prefills its KV cache with a 1,024-token
 prompt and compares with separate launches (thousands of dispatches); this
-run fills the cache rows 0..1023 with seeded bf16 values instead and launches the step eagerly a few times from position 1024, so a
-rocprofv3 counter pass sees a handful of step dispatches:
+run fills the cache rows 0..1023 with seeded bf16 values instead and launches
+the step eagerly a few times from position 1024, so a rocprofv3 counter pass
+sees a handful of step dispatches:
 
   cd fleet-mi300x_amd
   rocprofv3 --pmc FETCH_SIZE --kernel-include-regex 'step_kernel|stream_read|FillFunctor' \\
