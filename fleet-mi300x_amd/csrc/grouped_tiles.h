@@ -11,7 +11,8 @@
 // slices' sums added in fp32 (error against 64 bits 2.0e-4 at 256 tokens, 2.2e-4
 // in the other plan, which chains 32).
 //
-// R = 2, NT = 4 (128 KB of weights in flight per CU): 256 tokens in 285 us; with
+// R = 2, NT = 4 (128 KB of weights in flight per CU): 256 tokens in 285 us (the
+// routed workgroups first, as in all figures of this paragraph); with
 // R = 1 and NT = 3: 335; NT = 2, R = 2: 292, but 332 against 272 under Zipf
 // routing, whose popular experts fill blocks of 64. Persistent workgroups that
 // carry the stream across tiles: 358. The plan for fewer tokens: 468. With one K

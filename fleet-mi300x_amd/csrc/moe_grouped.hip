@@ -31,7 +31,7 @@
 //   (epoch << 32 | payload, device-scope stores and loads; no grid barrier).
 // T > 8: two launches on the stream, G, then D + C; h crosses the kernel
 //   boundary as plain bf16.
-// T >= kTileTokens (84): grouped_tiles.h.
+// T >= kTileTokens (65): grouped_tiles.h.
 // Partials bf16(w * bf16(d)) (shared: bf16(d), or with two launches the two
 // fp32 K-half sums) are published per (token, slot) as tagged words; phase C
 // sums them in slot order: out[t] = bf16(bf16(sum_k part[t][k]) + shared[t]).
@@ -101,11 +101,10 @@ struct Layout {
 // From this many tokens on, the step runs as tiles (grouped_tiles.h). Above 64
 // tokens the shared expert takes a second pass of the MFMA items here, each
 // reading its weights anew, and every 32-row item of an expert with few tokens
-// leaves waves idle (uniform / Zipf(1.1) routing, us): 80 tokens 294 / 179 here,
-// 241 / 179 as tiles; 96: 330 / 209 and 234 / 188; 128: 421 / 266 and 243 / 211;
-// 256: 468 / 390 and 285 / 272. At 72 tokens the Zipf step is still faster here
-// (168 and 177).
-constexpr int kTileTokens = 84;
+// leaves waves idle (routing and experts, uniform / experts alone, Zipf(1.1), us):
+// 65 tokens 246 / 152 here, 208 / 150 as tiles; 72: 276 / 166 and 209 / 151; 83:
+// 308 / 185 and 210 / 155. At 64 tokens it is 206 / 117 here and 203 / 143 as tiles.
+constexpr int kTileTokens = 65;
 
 __host__ __device__ constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 

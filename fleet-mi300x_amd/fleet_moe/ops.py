@@ -502,8 +502,8 @@ class Decoder:
         self.reset(0)
         done = 0
         n = min(tokens.numel(), self.max_pos)
-        # from 4 tokens on: 3 take 4.7 ms together and 3.9 as steps, 4 take 5.0
-        # and 5.2, 8 take 6.0 and 10.4, 384 take 23 and 514 (few tokens select
+        # from 4 tokens on: 3 take 4.7 ms together and 3.9 as steps, 4 take 4.6
+        # and 5.2, 8 take 5.4 and 10.4, 384 take 23 and 514 (few tokens select
         # nearly as many experts' weights, and leave most of a 16-token tile empty)
         if self.fused and tokens.dim() == 1 and n >= 4:
             t = tokens[:n].to(device=self.blob.device, dtype=torch.int32).contiguous()

@@ -197,11 +197,12 @@ def test_grouped_call_count_wrap_restarts_a_clean_workspace(dev):
     assert runner.status() == 0
 
 
-@pytest.mark.parametrize("T, routing", [(83, "uniform"), (84, "uniform"), (84, "zipf"),
+@pytest.mark.parametrize("T, routing", [(64, "zipf"), (65, "uniform"), (65, "hot"),
+                                        (83, "uniform"), (84, "uniform"), (84, "zipf"),
                                         (97, "hot"), (129, "zipf"), (193, "uniform"),
                                         (255, "hot"), (256, "zipf"), (256, "one")])
 def test_grouped_tiles(dev, T, routing):
-    """The tiled plan from its first token count (84) to the largest, at block
+    """The tiled plan from its first token count (65) to the largest, at block
     edges (m = 1 mod 16, 64 + 1, 256): uniform and Zipf routing, the same six
     experts for all (blocks of 64 of one expert), and one expert six times
     per token (24 blocks). bf16 tolerance, as for the other plans. (The oracle
