@@ -1,22 +1,29 @@
 // The grouped step's kernels for many tokens (launch_grouped draws the line):
 // every unit -- the shared expert, each selected expert -- is cut into
-// workgroups of 16 R W weight rows x up to 16 NT tokens, bf16 MFMA 16x16x32.
+// workgroups of 16 R W weight rows x up to 16 NT tokens, bf16 MFMA 16x16x32;
+// experts with at most 8 tokens run the other plan's VALU items.
 //
 // HBM bound: 17.3 MB per selected expert and 34.6 MB for the shared one, at 31
 // FLOP per byte and 256 tokens. A wave's weights go from HBM into registers (16
 // R rows x 256 K, refilled for the next slice as they are used), so every weight
 // byte is written to and read from LDS once, by its own wave, whatever the number
 // of tokens; the token rows pass through LDS, two slices in turn, each read by
-// the workgroup's four waves. Sums: 8 MFMAs in a chain per 256-K slice, the
-// slices' sums added in fp32 (error against 64 bits 2.0e-4 at 256 tokens, 2.2e-4
-// in the other plan, which chains 32).
+// the workgroup's four waves.
 //
-// R = 2, NT = 4 (128 KB of weights in flight per CU): 256 tokens in 285 us (the
-// routed workgroups first, as in all figures of this paragraph); with
-// R = 1 and NT = 3: 335; NT = 2, R = 2: 292, but 332 against 272 under Zipf
-// routing, whose popular experts fill blocks of 64. Persistent workgroups that
-// carry the stream across tiles: 358. The plan for fewer tokens: 468. With one K
-// step ahead (R = 1) in the down launch alone: 300.
+// Every sum is the other plan's, bit for bit (gemm): a token's result is the same
+// in any block, at any place in the batch and from call to call. Walking K from
+// eight different slices, which changes the sums with the workgroup, took
+// 258 us where this takes 269 (256 tokens with the router; 128: 216 / 231; 65:
+// 208 / 221). The other plan takes 474, 417 and 246.
+//
+// R = 2, NT = 4 holds 128 KB of weights in flight per CU. Other shapes, with K
+// walked from any slice and the routed workgroups first (256 tokens 285 us): R =
+// 1 and NT = 3: 335; NT = 2, R = 2: 292, but 332 against 272 under Zipf routing,
+// whose popular experts fill blocks of 64. Persistent workgroups that carry the
+// stream across tiles: 358. With one K step ahead (R = 1) in the down launch
+// alone: 300. As it is now: chains taken slice by slice in turn 263 for 264 us; a
+// VALU item's rows loaded during the one before 227 for 231 at 128 tokens and no
+// gain at 256: not worth their lines.
 //
 // Launches: the tables (one workgroup), gate / up + SwiGLU, down + routing weight,
 // combine; data crosses them as plain memory.
@@ -54,7 +61,8 @@ struct Params {
 };
 
 // One workgroup; ids outside [0, 64) are clamped and reported, as in the other
-// plan. The order of an expert's entries does not reach any result.
+// plan. The entries of an expert come in no fixed order, which reaches no result:
+// an entry's sums do not depend on its block or its place there.
 __global__ __launch_bounds__(1024) void table_kernel(const int32_t* ids, int n, int tok, Header* hdr,
                                                      Table* tab) {
     __shared__ int cnt[kRouted], at[kRouted];
@@ -102,49 +110,70 @@ struct Lds {
     alignas(16) uint8_t turn[W][16 * kTurnPitch];
 };
 
-// y[n][v] = row 4 q + v of the wave's 16 rows (from `w`) x token 16 n + l % 16;
-// xrow(i): the bf16 row of the workgroup's i-th token.
+// y[r][n][v] = row 16 r + 4 q + v of the wave's rows (from `w`) x token 16 n + l %
+// 16; xrow(i): the row of `x` (bf16 [][K]) of the workgroup's i-th token.
 // A weight load takes eight rows' 128-byte lines, eight lanes to a line. (In the
 // MFMA's own layout, lane l = row l % 16, the four lanes of a row are 16 apart:
 // every 16 lanes touch 16 lines, 64 bytes of each per load, and the stream stops
 // at 4.9 TB/s.) Two such loads, 16 rows x two steps, change to the MFMA's layout
 // through LDS.
+// The sums are those of the other plan's MFMA items, bit for bit and whatever the
+// block, the batch or the workgroup: one chain over the even slices, one over the
+// odd, added; 2816 values as two halves of 1408, added. Which chain and which half
+// come first is free (an addition's operands may change places), so workgroups
+// start at different ones: rows are 4 KB (2816 B) apart, and all waves walking
+// them from the left would meet in the same memory channels.
 template <int K, int NT, int R, int W, class XRow>
-__device__ __forceinline__ void gemm(const uint16_t* w, XRow&& xrow, Lds<NT, W>& L,
-                                     f32x4 (&y)[R][NT]) {
+__device__ __forceinline__ void gemm(const uint16_t* w, const uint16_t* x, XRow&& xrow,
+                                     Lds<NT, W>& L, f32x4 (&y)[R][NT]) {
     constexpr int kChunks = K / kChunk;                  // 16-byte chunks per row
     constexpr int kTokChunks = kSliceK / kChunk;         // 32 per slice
     constexpr int P = 16 * NT * kTokChunks / (64 * W);
-    static_assert(16 * NT * kTokChunks % (64 * W) == 0 && K % 64 == 0, "whole chunks, whole lines");
+    constexpr int kHalves = K == kSharedInter ? 2 : 1, kHalfChunks = kChunks / kHalves;
+    constexpr int kPer = (kHalfChunks / kTokChunks + 1) / 2;     // slices per chain
+    constexpr int kChains = 2 * kHalves;
+    static_assert(16 * NT * kTokChunks % (64 * W) == 0 && K % (64 * kHalves) == 0 &&
+                      (2 * kPer - 1) * kTokChunks < kHalfChunks && kHalfChunks <= 2 * kPer * kTokChunks,
+                  "whole chunks, whole lines, every slice holds some");
     const int tid = threadIdx.x, lane = tid & (kLanes - 1), j = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const u32x4* wp = reinterpret_cast<const u32x4*>(w) + (lane >> 3) * kChunks + (lane & 7);
     uint8_t* const turn = L.turn[wave];
     uint8_t* const tw = turn + (lane >> 3) * kTurnPitch + 16 * (lane & 7);
     const uint8_t* const tr = turn + j * kTurnPitch + 16 * q;
-    const u32x4* src[P];
+    uint32_t src[P];                                     // byte offsets from x: < 8 MB
     const int c = tid % kTokChunks;                      // 64 W is a multiple of 32
 #pragma unroll
     for (int i = 0; i < P; ++i)
-        src[i] = reinterpret_cast<const u32x4*>(xrow((tid + 64 * W * i) / kTokChunks)) + c;
+        src[i] = (uint32_t)(xrow((tid + 64 * W * i) / kTokChunks) * (2 * K) + 16 * c);
     const int dst = (tid / kTokChunks) * kPitch + 16 * c;
     constexpr int kDst = 64 * W / kTokChunks * kPitch;
     u32x4 raw[R][kSteps / 2][2], xs[P];
-    auto load_w = [&](int p, int c0) {                   // steps 2 p, 2 p + 1 of the slice at c0
-        if (c0 + 8 * p < kChunks)                        // uniform
+    // slice `i` of the chain taken ch-th: its first chunk and its chunks
+    const int start = (int)(blockIdx.x / kXcds % kChains);
+    struct Slice {
+        int c0, n;
+    };
+    auto slice = [&](int ch, int i) {
+        const int chain = ch ^ start, s = (2 * i + (chain & 1)) * kTokChunks;
+        return Slice{(chain >> 1) * kHalfChunks + s, min(kTokChunks, kHalfChunks - s)};
+    };
+    auto load_w = [&](int p, Slice z) {                  // steps 2 p, 2 p + 1
+        if (8 * p < z.n)                                 // uniform
 #pragma unroll
             for (int r = 0; r < R; ++r)
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
-                    raw[r][p][h] = ld_stream(wp + (16 * r + 8 * h) * kChunks + c0 + 8 * p);
+                    raw[r][p][h] = ld_stream(wp + (16 * r + 8 * h) * kChunks + z.c0 + 8 * p);
     };
-    auto load_x = [&](int c0) {
-        if (c0 + c < kChunks)
+    auto load_x = [&](Slice z) {
+        if (c < z.n)
 #pragma unroll
-            for (int i = 0; i < P; ++i) xs[i] = ld_global(src[i] + c0);
+            for (int i = 0; i < P; ++i) xs[i] = ld_global(reinterpret_cast<const u32x4*>(
+                    reinterpret_cast<const uint8_t*>(x) + 16 * z.c0 + src[i]));
     };
-    auto put = [&](int buf, int c0) {
-        if (c0 + c < kChunks)
+    auto put = [&](int buf, Slice z) {
+        if (c < z.n)
 #pragma unroll
             for (int i = 0; i < P; ++i)
                 *reinterpret_cast<u32x4*>(L.x[buf] + dst + i * kDst) = xs[i];
@@ -154,73 +183,87 @@ __device__ __forceinline__ void gemm(const uint16_t* w, XRow&& xrow, Lds<NT, W>&
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
-    // Workgroups start at different slices: rows are 4 KB (2816 B) apart, and all
-    // waves walking them from the left would meet in the same memory channels.
-    constexpr int kSlices = (kChunks + kTokChunks - 1) / kTokChunks;
-    int c0 = (int)(blockIdx.x / kXcds % kSlices) * kTokChunks;
-    load_x(c0);
+    Slice z = slice(0, 0);
+    load_x(z);
 #pragma unroll
-    for (int p = 0; p < kSteps / 2; ++p) load_w(p, c0);
-    put(0, c0);
+    for (int p = 0; p < kSteps / 2; ++p) load_w(p, z);
+    put(0, z);
     barrier();
+    f32x4 lo[kHalves == 2 ? R : 1][kHalves == 2 ? NT : 1];      // the first half's sums
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int n = 0; n < NT; ++n) y[r][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int buf = 0;
 #pragma unroll 1
-    for (int it = 0; it < kSlices; ++it) {
-        const bool more = it + 1 < kSlices;
-        const int buf = it & 1, nx = c0 + kTokChunks < kChunks ? c0 + kTokChunks : 0;
-        if (more) load_x(nx);                            // uniform but for the tail's chunks
-        const uint8_t* xp = L.x[buf] + j * kPitch + 16 * q;
+    for (int ch = 0; ch < kChains; ++ch) {
         f32x4 t[R][NT];
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
             for (int n = 0; n < NT; ++n) t[r][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int i = 0; i < kPer; ++i, buf ^= 1) {
+            const bool more = i + 1 < kPer || ch + 1 < kChains;
+            const Slice nx = i + 1 < kPer ? slice(ch, i + 1) : slice(ch + 1, 0);
+            if (more) load_x(nx);                        // uniform but for the tail's chunks
+            const uint8_t* xp = L.x[buf] + j * kPitch + 16 * q;
 #pragma unroll
-        for (int p = 0; p < kSteps / 2; ++p) {
-            if (c0 + 8 * p < kChunks) {                  // uniform
-                u32x4 a[R][2];
+            for (int p = 0; p < kSteps / 2; ++p) {
+                if (8 * p < z.n) {                       // uniform
+                    u32x4 a[R][2];
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
+                    for (int r = 0; r < R; ++r) {
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        *reinterpret_cast<u32x4*>(tw + 8 * h * kTurnPitch) = raw[r][p][h];
-                    lds_wave_sync();
+                        for (int h = 0; h < 2; ++h)
+                            *reinterpret_cast<u32x4*>(tw + 8 * h * kTurnPitch) = raw[r][p][h];
+                        lds_wave_sync();
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        a[r][h] = *reinterpret_cast<const u32x4*>(tr + 64 * h);
-                    lds_wave_sync();
-                }
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int n = 0; n < NT; ++n) {
-                        const u32x4 b = *reinterpret_cast<const u32x4*>(xp + 16 * n * kPitch +
-                                                                       64 * (2 * p + h));
-#pragma unroll
-                        for (int r = 0; r < R; ++r) t[r][n] = mfma16(a[r][h], b, t[r][n]);
+                        for (int h = 0; h < 2; ++h)
+                            a[r][h] = *reinterpret_cast<const u32x4*>(tr + 64 * h);
+                        lds_wave_sync();
                     }
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int n = 0; n < NT; ++n) {
+                            const u32x4 b = *reinterpret_cast<const u32x4*>(xp + 16 * n * kPitch +
+                                                                           64 * (2 * p + h));
+#pragma unroll
+                            for (int r = 0; r < R; ++r) t[r][n] = mfma16(a[r][h], b, t[r][n]);
+                        }
+                }
+                if (p == kSteps / 4 && more) put(buf ^ 1, nx);
+                if (more) load_w(p, nx);
             }
-            if (p == kSteps / 4 && more) put(buf ^ 1, nx);
-            if (more) load_w(p, nx);
+            z = nx;
+            barrier();
         }
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
-            for (int n = 0; n < NT; ++n) y[r][n] += t[r][n];
-        c0 = nx;
-        barrier();
+            for (int n = 0; n < NT; ++n) {
+                if (ch % 2 == 0) {
+                    if constexpr (kHalves == 2) lo[r][n] = y[r][n];
+                    y[r][n] = t[r][n];
+                } else {
+                    y[r][n] += t[r][n];
+                }
+            }
     }
+    if constexpr (kHalves == 2)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) y[r][n] += lo[r][n];
 }
 
 // This workgroup's token block of a routed expert (row tile `tile` of `tiles`,
 // entries [first, first + m)): the workgroups of one XCD (wg % 8) take a
-// block's row tiles in turn, so its token rows are fetched into one L2. False
-// past the last block.
+// block's row tiles in turn, so its token rows are fetched into one L2. few: the
+// expert is a VALU unit. False past the last block.
 __device__ __forceinline__ bool routed_block(const Table* tab, int wg, int tok, int tiles, int& e,
-                                             int& tile, int& first, int& m) {
+                                             int& tile, int& first, int& m, bool& few) {
     const int lane = threadIdx.x & (kLanes - 1);
     const int local = wg / kXcds, b = wg % kXcds + kXcds * (local / tiles);
     tile = local % tiles;
@@ -231,6 +274,7 @@ __device__ __forceinline__ bool routed_block(const Table* tab, int wg, int tok, 
     const int j0 = tok * (b - tab->blk[e]);
     first = tab->off[e] + j0;
     m = min(tok, tab->off[e + 1] - first);
+    few = is_v(tab->off[e + 1] - tab->off[e]);
     return true;
 }
 
@@ -241,9 +285,9 @@ __device__ __forceinline__ void g_tile(const Params& P, const uint16_t* wt, int 
     const int lane = threadIdx.x & (kLanes - 1), i = lane & 15, q = lane >> 4;
     const int row0 = 16 * R * (W * tile + wave);
     f32x4 y[R][NT];
-    gemm<kHidden, NT, R, W>(wt + (int64_t)row0 * kHidden, [&](int k) {
+    gemm<kHidden, NT, R, W>(wt + (int64_t)row0 * kHidden, P.x, [&](int k) {
         const int j = first + min(k, m - 1);
-        return P.x + (int64_t)(shared ? j : P.tab->ent[j] / kTopK) * kHidden;
+        return shared ? j : P.tab->ent[j] / kTopK;
     }, *static_cast<Lds<NT, W>*>(lds), y);
     uint16_t* out = shared ? P.h + (int64_t)P.T * kTopK * kInter : P.h;
     const int pitch = shared ? kSharedInter : kInter;
@@ -260,6 +304,55 @@ __device__ __forceinline__ void g_tile(const Params& P, const uint16_t* wt, int 
             }
 }
 
+// Experts with at most 8 tokens: the other plan's VALU items (a wave each, one
+// after the other), whose sums are another tree than the matrix cores'. Their
+// tokens' rows sit in LDS, in front of the waves' reduction words.
+constexpr int kFewRed = kVMax * kHidden * 2;
+static_assert(kFewRed + 4 * kLanes * 4 <= (int)sizeof(Lds<4, 4>) && kInter <= kHidden, "rows fit");
+
+template <int M, int ROWS, int W>
+__device__ __forceinline__ void g_few(const Params& P, const uint16_t* wt, int tile, int first, int m,
+                                      uint8_t* lds) {
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int k = tid; k < m * kRowChunks; k += 64 * W) {
+        const int j = k / kRowChunks, c = k - j * kRowChunks;
+        reinterpret_cast<u32x4*>(lds)[k] = ld_global(
+            reinterpret_cast<const u32x4*>(P.x + (int64_t)(P.tab->ent[first + j] / kTopK) * kHidden) +
+            c);
+    }
+    __syncthreads();
+    float* const red = reinterpret_cast<float*>(lds + kFewRed) + kLanes * wave;
+    const u32x4* rows = reinterpret_cast<const u32x4*>(wt) + (int64_t)ROWS * tile * kRowChunks;
+    uint32_t* h = reinterpret_cast<uint32_t*>(P.h) + (int64_t)first * (kInter / 2) + ROWS / 4 * tile;
+#pragma unroll 1
+    for (int i = wave; i < ROWS / 4; i += W)
+        g_pairs_v<M>(rows + 4 * i * kRowChunks, lds, m, red,
+                     [&](int j, uint32_t word) { h[j * (kInter / 2) + i] = word; });
+}
+
+template <int M, int ROWS, int W>
+__device__ __forceinline__ void d_few(const Params& P, const uint16_t* wt, int tile, int first, int m,
+                                      uint8_t* lds) {
+    constexpr int R = M <= 4 ? 8 : 4;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const u32x4* h = reinterpret_cast<const u32x4*>(P.h + (int64_t)first * kInter);
+    for (int k = tid; k < m * kInterChunks; k += 64 * W)
+        reinterpret_cast<u32x4*>(lds)[k] = ld_global(h + k);
+    __syncthreads();
+    float* const red = reinterpret_cast<float*>(lds + kFewRed) + kLanes * wave;
+    const u32x4* rows = reinterpret_cast<const u32x4*>(wt) + (int64_t)ROWS * tile * kInterChunks;
+#pragma unroll 1
+    for (int i = wave; i < ROWS / R; i += W)
+        d_rows_v<M, kInter, R>(rows + R * i * kInterChunks, lds, m, red,
+                               [&](int j, int wp, float a, float b) {
+            const int en = P.tab->ent[first + j], t = en / kTopK;
+            const int64_t slot = (int64_t)t * kSlots + (en - t * kTopK);
+            const float w = P.weights[en];
+            *reinterpret_cast<uint32_t*>(P.part + slot * kHidden + ROWS * tile + R * i + 2 * wp) =
+                pack_bf16(w * bf16r(a), w * bf16r(b));
+        });
+}
+
 template <int NTM, int R, int W>
 __global__ __launch_bounds__(64 * W, 2) void g_kernel(Params P) {
     __shared__ Lds<NTM, W> S;
@@ -268,8 +361,18 @@ __global__ __launch_bounds__(64 * W, 2) void g_kernel(Params P) {
     const uint16_t* wt;
     const bool shared = (int)blockIdx.x < P.shared_wgs;
     if (!shared) {
-        if (!routed_block(P.tab, (int)blockIdx.x - P.shared_wgs, 16 * NTM, 2 * kInter / (16 * R * W), e, tile, first, m)) return;
+        bool few = false;
+        if (!routed_block(P.tab, (int)blockIdx.x - P.shared_wgs, 16 * NTM,
+                          2 * kInter / (16 * R * W), e, tile, first, m, few))
+            return;
         wt = P.experts + (int64_t)e * P.stride;
+        if (few) {
+            uint8_t* const b = static_cast<uint8_t*>(lds);
+            if (m == 1) return g_few<1, 16 * R * W, W>(P, wt, tile, first, m, b);
+            if (m == 2) return g_few<2, 16 * R * W, W>(P, wt, tile, first, m, b);
+            if (m <= 4) return g_few<4, 16 * R * W, W>(P, wt, tile, first, m, b);
+            return g_few<8, 16 * R * W, W>(P, wt, tile, first, m, b);
+        }
     } else {
         constexpr int kTiles = 2 * kSharedInter / (16 * R * W);
         const int b = blockIdx.x;
@@ -296,9 +399,8 @@ __device__ __forceinline__ void d_tile(const Params& P, const uint16_t* wt, int 
     const int row0 = 16 * R * (W * tile + wave);
     const uint16_t* h = shared ? P.h + (int64_t)P.T * kTopK * kInter : P.h;
     f32x4 y[R][NT];
-    gemm<K, NT, R, W>(wt + (int64_t)row0 * K,
-                   [&](int k) { return h + (int64_t)(first + min(k, m - 1)) * K; },
-                   *static_cast<Lds<NT, W>*>(lds), y);
+    gemm<K, NT, R, W>(wt + (int64_t)row0 * K, h, [&](int k) { return first + min(k, m - 1); },
+                      *static_cast<Lds<NT, W>*>(lds), y);
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         if (16 * n + i >= m) continue;
@@ -341,9 +443,19 @@ __global__ __launch_bounds__(64 * W, 2) void d_kernel(Params P) {
     constexpr int kTiles = kHidden / (16 * R * W);
     int e = 0, tile = 0, first = 0, m = 0;
     if ((int)blockIdx.x >= P.shared_wgs) {
-        if (!routed_block(P.tab, (int)blockIdx.x - P.shared_wgs, 16 * NTM, kTiles, e, tile, first, m)) return;
-        d_block<kInter, NTM, R, W>(P, P.experts + (int64_t)e * P.stride + (int64_t)2 * kInter * kHidden,
-                                tile, first, m, lds);
+        bool few = false;
+        if (!routed_block(P.tab, (int)blockIdx.x - P.shared_wgs, 16 * NTM, kTiles, e, tile, first, m,
+                          few))
+            return;
+        const uint16_t* wt = P.experts + (int64_t)e * P.stride + (int64_t)2 * kInter * kHidden;
+        if (few) {
+            uint8_t* const b = static_cast<uint8_t*>(lds);
+            if (m == 1) return d_few<1, 16 * R * W, W>(P, wt, tile, first, m, b);
+            if (m == 2) return d_few<2, 16 * R * W, W>(P, wt, tile, first, m, b);
+            if (m <= 4) return d_few<4, 16 * R * W, W>(P, wt, tile, first, m, b);
+            return d_few<8, 16 * R * W, W>(P, wt, tile, first, m, b);
+        }
+        d_block<kInter, NTM, R, W>(P, wt, tile, first, m, lds);
         return;
     }
     const int b = blockIdx.x;

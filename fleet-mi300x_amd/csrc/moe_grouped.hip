@@ -102,8 +102,9 @@ struct Layout {
 // tokens the shared expert takes a second pass of the MFMA items here, each
 // reading its weights anew, and every 32-row item of an expert with few tokens
 // leaves waves idle (routing and experts, uniform / experts alone, Zipf(1.1), us):
-// 65 tokens 246 / 152 here, 208 / 150 as tiles; 72: 276 / 166 and 209 / 151; 83:
-// 308 / 185 and 210 / 155. At 64 tokens it is 206 / 117 here and 203 / 143 as tiles.
+// 65 tokens 246 / 151 here, 221 / 159 as tiles; 72: 275 / 165 and 221 / 159; 128:
+// 417 / 264 and 231 / 186; 256: 474 / 383 and 269 / 250. At 64 tokens it is 205 / 117
+// here. Both plans give the same bits, so the line changes no result.
 constexpr int kTileTokens = 65;
 
 __host__ __device__ constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -489,16 +490,15 @@ __device__ __forceinline__ int token_of(const Lds& L, const Unit& u, int j) {
 
 // ---------------------------------------------------------------- phase G
 
-// VALU item: row pairs 2i, 2i+1 of a unit with m <= 8 tokens whose x rows sit
-// in LDS at `xs`. Writes h word i of every token (plain with two launches,
-// tagged with one).
-template <int M>
-__device__ __forceinline__ void g_item_v(const Params& P, Lds& L, const Unit& u, int i,
-                                         const uint8_t* xs, uint32_t epoch) {
+// VALU item: two gate/up row pairs (rows g0, u0, g1, u1 at `base`) against m <= M
+// tokens whose x rows sit in LDS at `xs`; `red`: 64 floats of the wave's own.
+// put(j, word): token j's two h values. A value's bits depend on its rows and its
+// token alone: 16 dot2 in a chain per lane, then wave_msum's tree.
+template <int M, class Put>
+__device__ __forceinline__ void g_pairs_v(const u32x4* base, const uint8_t* xs, int m, float* red,
+                                          Put&& put) {
     const int lane = threadIdx.x & (kLanes - 1);
-    const uint16_t* blk = u.expert < 0 ? P.shared : P.experts + (int64_t)u.expert * P.expert_stride;
-    const u32x4* base = reinterpret_cast<const u32x4*>(blk) + (int64_t)(2 * i) * 2 * kRowChunks;
-    u32x4 W[16];   // rows g(2i), u(2i), g(2i+1), u(2i+1): 4 chunks each
+    u32x4 W[16];   // 4 chunks of each row
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -510,7 +510,7 @@ __device__ __forceinline__ void g_item_v(const Params& P, Lds& L, const Unit& u,
     const u32x4* xr = reinterpret_cast<const u32x4*>(xs);
 #pragma unroll
     for (int j = 0; j < M; ++j) {
-        if (j < u.m) {
+        if (j < m) {
             u32x4 xq[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) xq[c] = xr[j * kRowChunks + lane + kLanes * c];
@@ -521,21 +521,31 @@ __device__ __forceinline__ void g_item_v(const Params& P, Lds& L, const Unit& u,
         }
     }
     const float tot = wave_msum<NV>(acc);
-    const int wave = threadIdx.x >> 6;
-    float* red = L.red[wave];
     red[msum_index<NV>(lane)] = tot;
     lds_wave_sync();
-    if (lane < u.m) {
+    if (lane < m) {
         const int j = lane;
         const float g0 = red[0 * M + j], u0 = red[1 * M + j];
         const float g1 = red[2 * M + j], u1 = red[3 * M + j];
         const float h0 = bf16r(bf16r(silu_rn(bf16r(g0))) * bf16r(u0));
         const float h1 = bf16r(bf16r(silu_rn(bf16r(g1))) * bf16r(u1));
-        const int64_t w = u.h_off + (int64_t)j * (gpairs_of(u) / 2) + i;
-        if (P.hp) P.hp[w] = pack_bf16(h0, h1);
-        else st_word(P.h + w, epoch, pack_bf16(h0, h1));
+        put(j, pack_bf16(h0, h1));
     }
     lds_wave_sync();
+}
+
+// Item i of a unit with m <= 8 tokens: row pairs 2i, 2i+1; h word i of every
+// token (plain with two launches, tagged with one).
+template <int M>
+__device__ __forceinline__ void g_item_v(const Params& P, Lds& L, const Unit& u, int i,
+                                         const uint8_t* xs, uint32_t epoch) {
+    const uint16_t* blk = u.expert < 0 ? P.shared : P.experts + (int64_t)u.expert * P.expert_stride;
+    const u32x4* base = reinterpret_cast<const u32x4*>(blk) + (int64_t)(2 * i) * 2 * kRowChunks;
+    g_pairs_v<M>(base, xs, u.m, L.red[threadIdx.x >> 6], [&](int j, uint32_t word) {
+        const int64_t w = u.h_off + (int64_t)j * (gpairs_of(u) / 2) + i;
+        if (P.hp) P.hp[w] = word;
+        else st_word(P.h + w, epoch, word);
+    });
 }
 
 // ---------------------------------------------------------------- phase D
@@ -562,21 +572,16 @@ __device__ __forceinline__ void put_part(const Params& P, const Lds& L, const Un
     st_word(P.part + ((int64_t)t * kSlots + slot) * kPartWords + word, epoch, pack_bf16(a, b));
 }
 
-// VALU item: R rows of the unit's down matrix (R x M <= 32), m <= M tokens
-// whose h rows sit in LDS at `hs` (bf16 [m][I]).
-template <int M, bool SH, int R>
-__device__ __forceinline__ void d_item_v(const Params& P, Lds& L, const Unit& u, int i,
-                                         const uint8_t* hs, uint32_t epoch) {
-    constexpr int K = SH ? kSharedInter : kInter;
+// VALU item: R rows of K values at `base` (R x M <= 32) against m <= M tokens
+// whose h rows sit in LDS at `hs` (bf16 [m][K]); `red` as above. put(j, wp, a, b):
+// token j's fp32 sums of rows 2 wp, 2 wp + 1.
+template <int M, int K, int R, class Put>
+__device__ __forceinline__ void d_rows_v(const u32x4* base, const uint8_t* hs, int m, float* red,
+                                         Put&& put) {
     constexpr int C = K / kChunk;          // 16-byte chunks per row: 176 / 352
     constexpr int G = (C + kLanes - 1) / kLanes;   // 3 / 6
     static_assert(R * M <= 32 && R % 2 == 0, "item shape");
     const int lane = threadIdx.x & (kLanes - 1);
-    const int row0 = R * i;
-    const uint16_t* dn = SH ? P.shared + (int64_t)2 * kSharedInter * kHidden
-                            : P.experts + (int64_t)u.expert * P.expert_stride +
-                                  (int64_t)2 * kInter * kHidden;
-    const u32x4* base = reinterpret_cast<const u32x4*>(dn) + (int64_t)row0 * C;
     u32x4 W[R * G];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -592,7 +597,7 @@ __device__ __forceinline__ void d_item_v(const Params& P, Lds& L, const Unit& u,
     const u32x4* hr = reinterpret_cast<const u32x4*>(hs);
 #pragma unroll
     for (int j = 0; j < M; ++j) {
-        if (j < u.m) {
+        if (j < m) {
             u32x4 H[G];
 #pragma unroll
             for (int g = 0; g < G; ++g) {
@@ -606,16 +611,28 @@ __device__ __forceinline__ void d_item_v(const Params& P, Lds& L, const Unit& u,
         }
     }
     const float tot = wave_msum<NV>(acc);
-    const int wave = threadIdx.x >> 6;
-    float* red = L.red[wave];
     red[msum_index<NV>(lane)] = tot;
     lds_wave_sync();
-    if (lane < u.m * (R / 2)) {
+    if (lane < m * (R / 2)) {
         const int j = lane / (R / 2), wp = lane - j * (R / 2);
-        put_part(P, L, u, j, row0 / 2 + wp, red[(2 * wp) * M + j], red[(2 * wp + 1) * M + j],
-                 epoch);
+        put(j, wp, red[(2 * wp) * M + j], red[(2 * wp + 1) * M + j]);
     }
     lds_wave_sync();
+}
+
+// Item i of a unit: down rows R i .. R i + R - 1.
+template <int M, bool SH, int R>
+__device__ __forceinline__ void d_item_v(const Params& P, Lds& L, const Unit& u, int i,
+                                         const uint8_t* hs, uint32_t epoch) {
+    constexpr int K = SH ? kSharedInter : kInter;
+    const int row0 = R * i;
+    const uint16_t* dn = SH ? P.shared + (int64_t)2 * kSharedInter * kHidden
+                            : P.experts + (int64_t)u.expert * P.expert_stride +
+                                  (int64_t)2 * kInter * kHidden;
+    d_rows_v<M, K, R>(reinterpret_cast<const u32x4*>(dn) + (int64_t)row0 * (K / kChunk), hs, u.m,
+                      L.red[threadIdx.x >> 6], [&](int j, int wp, float a, float b) {
+                          put_part(P, L, u, j, row0 / 2 + wp, a, b, epoch);
+                      });
 }
 
 // ---------------------------------------------------------------- MFMA stream

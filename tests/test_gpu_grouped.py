@@ -232,6 +232,72 @@ def test_grouped_tiles(dev, T, routing):
     assert runner.status() == 0
 
 
+def routing_of(T: int, kind: str) -> np.ndarray:
+    """ids [T][6]: "windows": every expert's tokens lie in one window of 64, from
+    one token to the whole window per expert; "hot": six experts for all; "one":
+    one expert, six times; "skewed": experts of 1 to T tokens anywhere."""
+    g = np.random.default_rng(T)
+    if kind == "hot":
+        return np.tile(np.array([5, 17, 3, 63, 0, 41], np.int32), (T, 1))
+    if kind == "one":
+        return np.full((T, 6), 9, np.int32)
+    if kind == "skewed":
+        p = np.arange(1, 65) ** -1.5
+        return np.stack([g.choice(64, 6, replace=False, p=p / p.sum()) for _ in range(T)]
+                        ).astype(np.int32)
+    ids = np.empty((T, 6), np.int32)
+    for n, w in enumerate(range(0, T, 64)):
+        p = np.arange(1, 17) ** -1.5
+        for t in range(w, min(w + 64, T)):
+            ids[t] = 4 * g.choice(16, 6, replace=False, p=p / p.sum()) + n
+    return ids
+
+
+def device_step(T: int, ids: np.ndarray):
+    x = torch.from_numpy(orc.bf16_bits(orc.rms_norm(synth.hidden_inputs(400 + T, T))).view(np.int16))
+    ws = torch.rand((T, 6), generator=torch.Generator().manual_seed(T))
+    return x.cuda(), torch.from_numpy(ids).cuda(), ws.cuda()
+
+
+@pytest.mark.parametrize("T, kind", [(73, "windows"), (128, "windows"), (201, "windows"),
+                                     (256, "windows"), (137, "hot"), (256, "hot"), (256, "one")])
+def test_grouped_tiles_are_the_other_plans_bits(dev, T, kind):
+    """Where every unit holds at most 8 tokens in steps of 64 exactly when it does
+    in the whole step, the tiles give the bits of those steps (the other plan):
+    the same sums in the same order, in units of 1 to 256 tokens."""
+    layer, pl = dev
+    runner = ops.GroupedRunner(T, DSV2_LITE)
+    ids = routing_of(T, kind)
+    counts = np.bincount(ids.ravel(), minlength=64)
+    say(f"tiles against steps T={T} {kind} counts {sorted(set(counts.tolist()))}")
+    a = device_step(T, ids)
+    got = runner.run(layer, *a)
+    parts = [runner.run(layer, *(v[k: k + 64].contiguous() for v in a)) for k in range(0, T, 64)]
+    torch.cuda.synchronize()
+    assert torch.equal(got, torch.cat(parts))
+    assert runner.status() == 0
+
+
+@pytest.mark.parametrize("T, kind", [(66, "skewed"), (97, "hot"), (150, "hot"), (192, "skewed"),
+                                     (200, "hot"), (256, "skewed"), (256, "one")])
+def test_grouped_tiles_do_not_depend_on_the_order(dev, T, kind):
+    """The same call gives the same bits every time, and a token's result does not
+    depend on its place in the batch: experts that fill several token blocks,
+    whose tokens fall into them in no fixed order."""
+    layer, pl = dev
+    runner = ops.GroupedRunner(T, DSV2_LITE)
+    x, ids, ws = device_step(T, routing_of(T, kind))
+    want = runner.run(layer, x, ids, ws)
+    g = torch.Generator().manual_seed(T)
+    for n in range(4):
+        say(f"order T={T} {kind} {n}")
+        assert torch.equal(runner.run(layer, x, ids, ws), want), n
+        p = torch.randperm(T, generator=g).cuda()
+        got = runner.run(layer, x[p].contiguous(), ids[p].contiguous(), ws[p].contiguous())
+        assert torch.equal(got, want[p]), n
+    assert runner.status() == 0
+
+
 def test_grouped_plans_share_a_workspace(dev):
     """Tiled and tagged-word steps in turn on one workspace, a tile step with
     ids out of range, and both under graph capture: every result equals that
