@@ -31,7 +31,7 @@
 //   (epoch << 32 | payload, device-scope stores and loads; no grid barrier).
 // T > 8: two launches on the stream, G, then D + C; h crosses the kernel
 //   boundary as plain bf16.
-// T >= kTileTokens (65): grouped_tiles.h.
+// T > kTagTokens (64): grouped_tiles.h.
 // Partials bf16(w * bf16(d)) (shared: bf16(d), or with two launches the two
 // fp32 K-half sums) are published per (token, slot) as tagged words; phase C
 // sums them in slot order: out[t] = bf16(bf16(sum_k part[t][k]) + shared[t]).
@@ -49,12 +49,23 @@ namespace grouped {
 
 constexpr int kMaxTokens = 256;
 constexpr int kMaxEntries = kMaxTokens * kTopK;     // 1536
-constexpr int kMaxChunks = kMaxEntries / kLanes;    // 24 chunks of 64 entries
+// Up to this many tokens the step runs as described above (tagged words), from 65
+// on as tiles (grouped_tiles.h). Above 64 tokens the shared expert would take a
+// second pass of the MFMA items here, each reading its weights anew, and every
+// 32-row item of an expert with few tokens leaves waves idle (routing and experts,
+// uniform / experts alone, Zipf(1.1), us): 65 tokens 246 / 151 here, 221 / 159 as
+// tiles; 72: 275 / 165 and 221 / 159; 128: 417 / 264 and 231 / 186; 256: 474 / 383
+// and 269 / 250. At 64 tokens it is 205 / 117 here. Both plans give the same bits,
+// so the line changes no result.
+constexpr int kTagTokens = 64;
+constexpr int kTagEntries = kTagTokens * kTopK;     // 384
+constexpr int kTagChunks = kTagEntries / kLanes;    // 6 chunks of 64 entries
 constexpr int kWG = 256;
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * kLanes;
 constexpr int kVMax = 8;                // VALU path for units of at most 8 tokens
-constexpr int kMGroup = 64;             // tokens per MFMA pass (4 tiles of 16)
+constexpr int kMGroup = 64;             // tokens per MFMA pass (4 tiles of 16); a unit has more
+                                        // where a token names one expert several times
 constexpr int kUnitsMax = 1 + kRouted;
 constexpr int kSegMax = 4;
 constexpr int kSlots = kTopK + 1;       // partial slots per token: 6 routed + shared
@@ -95,17 +106,8 @@ static_assert(offsetof(Header, abort) == 8, "status word offset");
 constexpr int kTabBytes = 16 + kUnitsMax * 6 * 4 + kMaxEntries * 2;
 
 struct Layout {
-    size_t tab, h, hp, part, sp, pp, pe, total;
+    size_t tab, h, hp, part, sp, pp, total;
 };
-
-// From this many tokens on, the step runs as tiles (grouped_tiles.h). Above 64
-// tokens the shared expert takes a second pass of the MFMA items here, each
-// reading its weights anew, and every 32-row item of an expert with few tokens
-// leaves waves idle (routing and experts, uniform / experts alone, Zipf(1.1), us):
-// 65 tokens 246 / 151 here, 221 / 159 as tiles; 72: 275 / 165 and 221 / 159; 128:
-// 417 / 264 and 231 / 186; 256: 474 / 383 and 269 / 250. At 64 tokens it is 205 / 117
-// here. Both plans give the same bits, so the line changes no result.
-constexpr int kTileTokens = 65;
 
 __host__ __device__ constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
@@ -114,14 +116,13 @@ __host__ __device__ constexpr Layout layout(int max_tokens) {
     L.tab = align256(sizeof(Header));
     L.h = L.tab + align256(kTabBytes);
     L.hp = L.h + align256((size_t)(max_tokens < kVMax ? max_tokens : kVMax) * kHWordsPerToken * 8);
+    const size_t tagged = max_tokens < kTagTokens ? max_tokens : kTagTokens;
     L.part = L.hp + align256((size_t)max_tokens * kHWordsPerToken * 4);
-    L.sp = L.part + align256((size_t)max_tokens * kSlots * kPartWords * 8);
-    L.pp = L.sp + align256((size_t)max_tokens * 2 * kHidden * 8);
+    L.sp = L.part + align256(tagged * kSlots * kPartWords * 8);
+    L.pp = L.sp + align256(tagged * 2 * kHidden * 8);
     // plain partials of the tiles: a place of their own, as the tagged words
     // must never hold anything but tagged words
-    const size_t tiled = max_tokens < kTileTokens ? 0 : (size_t)max_tokens;
-    L.pe = L.pp + tiled * kSlots * kHidden * 2;
-    L.total = L.pe + align256(tiled * kTopK * 8);
+    L.total = L.pp + (max_tokens > kTagTokens ? (size_t)max_tokens * kSlots * kHidden * 2 : 0);
     return L;
 }
 
@@ -139,7 +140,7 @@ struct Params {
     uint64_t* part;            // tagged partial words [T][7][1024]
     uint64_t* sp;              // tagged fp32 shared down sums [T][2 K halves][2048] (two launches)
     struct Tab* tab;           // dispatch tables handed from launch 1 to launch 2
-    size_t ws_tail16;          // 16-byte words of the workspace after the header
+    size_t ws_tail16;          // 16-byte words from the header to the last tagged one
     int T;
 };
 
@@ -155,7 +156,7 @@ struct Unit {
 struct Tab {
     int n_units, g_total, d_total, pad;
     Unit unit[kUnitsMax];
-    int16_t ent[kMaxEntries];
+    int16_t ent[kTagEntries];
 };
 static_assert(sizeof(Tab) <= kTabBytes && sizeof(Unit) == 6 * 4, "table blob");
 
@@ -165,7 +166,7 @@ struct Seg {
 };
 
 struct Lds {
-    int16_t ent[kMaxEntries];          // sorted position -> flat entry (t * 6 + k)
+    int16_t ent[kTagEntries];          // sorted position -> flat entry (t * 6 + k)
     int cnt[kRouted];
     int off[kRouted];
     Unit unit[kUnitsMax];
@@ -180,9 +181,9 @@ struct Lds {
         alignas(16) uint8_t stage[kStageBytes];          // VALU units: x or h rows
         alignas(16) uint8_t ring[kRing * kSliceA + kXchBytes];   // MFMA items
         struct {                                         // prologue only
-            int8_t id[kMaxEntries];      // ids, clamped to [0, 64)
-            int16_t rank[kMaxEntries];   // rank of an entry among equal ids of its chunk
-            int ccnt[kMaxChunks][kRouted];   // per-chunk counts, then per-chunk offsets
+            int8_t id[kTagEntries];      // ids, clamped to [0, 64)
+            int16_t rank[kTagEntries];   // rank of an entry among equal ids of its chunk
+            int ccnt[kTagChunks][kRouted];   // per-chunk counts, then per-chunk offsets
         } pro;
     };
 };
@@ -1223,7 +1224,7 @@ static int launch_grouped(const fleet_moe_layer* layer, int32_t n_tokens, const 
                           const float* weights, const uint16_t* x_norm, uint16_t* out,
                           char* ws, int max_tokens, hipStream_t stream) {
     const grouped::Layout L = grouped::layout(max_tokens);
-    if (n_tokens >= grouped::kTileTokens && max_tokens >= grouped::kTileTokens) {
+    if (n_tokens > grouped::kTagTokens) {       // max_tokens >= n_tokens: laid out
         grouped::tiles::Params Q{};
         Q.experts = layer->experts;
         Q.shared = layer->shared;
@@ -1253,7 +1254,7 @@ static int launch_grouped(const fleet_moe_layer* layer, int32_t n_tokens, const 
     P.part = reinterpret_cast<uint64_t*>(ws + L.part);
     P.sp = reinterpret_cast<uint64_t*>(ws + L.sp);
     P.tab = reinterpret_cast<grouped::Tab*>(ws + L.tab);
-    P.ws_tail16 = (L.total - sizeof(grouped::Header)) / 16;
+    P.ws_tail16 = (L.pp - sizeof(grouped::Header)) / 16;
     P.T = n_tokens;
     if (n_tokens <= grouped::kVMax) {
         P.hp = nullptr;

@@ -57,6 +57,10 @@ def test_workspace_sizes(lib):
     g64 = lib.fleet_moe_grouped_workspace_bytes(ctypes.byref(d), 64)
     g16 = lib.fleet_moe_grouped_workspace_bytes(ctypes.byref(d), 16)
     assert g64 > g16 > 0
+    # from 65 tokens on a token adds its h rows and its seven plain partials, no more
+    g128 = lib.fleet_moe_grouped_workspace_bytes(ctypes.byref(d), 128)
+    g256 = lib.fleet_moe_grouped_workspace_bytes(ctypes.byref(d), 256)
+    assert g256 - g128 == 128 * (2 * (6 * 1408 + 2816) + 7 * 2048 * 2)
     assert lib.fleet_moe_grouped_workspace_bytes(ctypes.byref(d), 0) == 0
     assert lib.fleet_moe_grouped_workspace_bytes(ctypes.byref(d), 100_000) == 0
 

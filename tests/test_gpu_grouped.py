@@ -197,6 +197,26 @@ def test_grouped_call_count_wrap_restarts_a_clean_workspace(dev):
     assert runner.status() == 0
 
 
+def test_grouped_call_count_wrap_beside_tiles(dev):
+    """The same on a workspace for 256 tokens, tile steps (which take no number)
+    between the calls: the tagged words alone are cleared, and all of them."""
+    layer, pl = dev
+    runner = ops.GroupedRunner(256, DSV2_LITE)
+    start = 0xFFFFFFFD
+    head0 = np.array([start, (start * 256) & 0xFFFFFFFF], np.uint32)
+    runner.workspace[:8].copy_(torch.from_numpy(head0.view(np.uint8)).cuda())
+    for n, T in enumerate((64, 256, 64, 8, 65, 64)):
+        xn = orc.rms_norm(synth.hidden_inputs(130 + n, T))
+        _, ids, ws = orc.route(pl.router_f32(), xn)
+        a = (torch.from_numpy(orc.bf16_bits(xn).view(np.int16)).cuda(),
+             torch.from_numpy(ids).cuda(), torch.from_numpy(ws).cuda())
+        say(f"grouped wrap beside tiles, call {n} T={T}")
+        got = runner.run(layer, *a)
+        assert torch.equal(got, ops.GroupedRunner(T, DSV2_LITE).run(layer, *a)), f"call {n} T={T}"
+    assert runner.workspace[:8].cpu().numpy().view(np.uint32).tolist() == [2, 512]
+    assert runner.status() == 0
+
+
 @pytest.mark.parametrize("T, routing", [(64, "zipf"), (65, "uniform"), (65, "hot"),
                                         (83, "uniform"), (84, "uniform"), (84, "zipf"),
                                         (97, "hot"), (129, "zipf"), (193, "uniform"),
