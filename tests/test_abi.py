@@ -159,6 +159,55 @@ def test_attention_entry_points_reject_bad_arguments_without_device(lib):
                                     ctypes.byref(d), None) == _lib.ERR_ARG
 
 
+def test_prompt_entry_points_reject_bad_arguments_without_device(lib):
+    d = c_dims(DSV2_LITE)
+    n = lib.fleet_prefill_workspace_bytes(ctypes.byref(d))
+    assert n % 256 == 0 and (100 << 20) < n < (160 << 20)
+    assert lib.fleet_prefill_workspace_bytes(ctypes.byref(c_dims(MoeDims(hidden=4096)))) == 0
+    assert lib.fleet_prefill_workspace_bytes(None) == 0
+    model = dict(layers=None, n_layers=2, max_pos=128, embed=256, final_norm=None, lm_head=None,
+                 rope_cos=256, rope_sin=256)
+    attn = _lib.FleetAttnLayer(256, 256, 256, 256, 256)
+    dense = dict(attn=attn, moe=_lib.FleetMoeLayer(256, None, None, 0, None), dense=256, cache=256)
+    moe = dict(attn=attn, dense=None, cache=256,
+               moe=_lib.FleetMoeLayer(256, 256, 256, DSV2_LITE.expert_stride, 256))
+
+    def call(m=None, rows=(dense, moe), dims=d, **kw):
+        a = {**dict(tokens=256, n=4, pos0=0, x=256, status=256, ws=256, bytes=n), **kw}
+        fm = _lib.FleetStepModel(**{**model, **(m or {})})
+        table = (_lib.FleetStepLayer * len(rows))(*(_lib.FleetStepLayer(**r) for r in rows))
+        return lib.fleet_prefill(ctypes.byref(fm), table, a["tokens"], a["n"], a["pos0"], a["x"],
+                                 a["status"], a["ws"], a["bytes"], ctypes.byref(dims), None)
+
+    arg = [dict(tokens=None), dict(tokens=258), dict(n=0), dict(n=129), dict(n=-1), dict(pos0=-1),
+           dict(pos0=125), dict(pos0=2**31 - 1), dict(x=None), dict(x=258), dict(status=None),
+           dict(status=257), dict(ws=None), dict(ws=384 + 16), dict(m=dict(n_layers=0)),
+           dict(m=dict(n_layers=65)), dict(m=dict(max_pos=0)), dict(m=dict(max_pos=4097)),
+           dict(m=dict(embed=None)), dict(m=dict(embed=264)), dict(m=dict(rope_cos=None)),
+           dict(m=dict(rope_sin=258))]
+    for at in range(5):                      # norm_in and kv_a_norm may be null, not misaligned
+        ptrs = [256] * 5
+        ptrs[at] = 257 if at in (0, 2) else None
+        arg.append(dict(rows=(dense, {**moe, "attn": _lib.FleetAttnLayer(*ptrs)})))
+    for k in ("router", "experts", "shared"):
+        row = {**moe, "moe": _lib.FleetMoeLayer(256, 256, 256, DSV2_LITE.expert_stride, 256)}
+        setattr(row["moe"], k, None)
+        arg.append(dict(rows=(dense, row)))
+    arg += [dict(rows=({**dense, "cache": None}, moe)), dict(rows=({**dense, "dense": 264}, moe)),
+            dict(rows=(dense, {**moe, "cache": 264}))]
+    for kw in arg:
+        assert call(**kw) == _lib.ERR_ARG, kw
+    for stride in (DSV2_LITE.expert_stride - 8, DSV2_LITE.expert_stride + 4):
+        row = {**moe, "moe": _lib.FleetMoeLayer(256, 256, 256, stride, 256)}
+        assert call(rows=(dense, row)) == _lib.ERR_DIMS
+    assert call(dims=c_dims(MoeDims(moe_inter=1024))) == _lib.ERR_DIMS
+    assert call(bytes=n - 256) == _lib.ERR_WORKSPACE
+    assert lib.fleet_moe_router_topk_bf16(256, 256, 1, None, None, 256, 256, None,
+                                          ctypes.byref(d), None) == _lib.ERR_ARG
+    assert lib.fleet_moe_router_topk_bf16(256, 256, 1, None, None, 256, 256, 264,
+                                          ctypes.byref(d), None) == _lib.ERR_ARG
+
+
 def test_trace_build_exports_the_library_and_its_trace_hooks():
     """The stage-trace build (a diagnostic variant of the same sources) binds
     like the library and adds only its three trace hooks; the library itself

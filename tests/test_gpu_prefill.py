@@ -1,8 +1,10 @@
 """GPU: a prompt taken through the layers together (fleet_prefill) leaves what
-teacher-forced decode steps leave, bit for bit: every cache row, the last
-token's residual, the pick and the position. The steps themselves are checked
-against the oracle in test_gpu_decode_model.py and test_gpu_step.py, so no
-tolerance is needed. Lengths around the 16-token tiles, the
+teacher-forced decode steps leave: every cache row, the last token's residual,
+the pick and the position, compared bit for bit. The steps themselves are
+checked against the oracle in test_gpu_decode_model.py and test_gpu_step.py. (The
+attention's fp64 sums alone are taken in another order than the steps', a
+difference of some 1e-8 of the fp32 unit they are rounded to; with the fixed
+tokens and weights here it reaches no bit.) Lengths around the 16-token tiles, the
 changes of shape (65, 177, 257, 401) and the 528-token chunk."""
 from __future__ import annotations
 
@@ -68,6 +70,47 @@ def test_prefill_equals_steps(pair, n):
     tokens = torch.randint(0, lay_mod.VOCAB, (n,), generator=g, device="cuda", dtype=torch.int32)
     check(pair, tokens)
     assert pair[0].status() == 0 and pair[1].status() == 0
+
+
+def test_long_prompt(pair):
+    """Three chunks, and attention over more than a thousand cache rows."""
+    got, want = (ops.Decoder(d.blob, d.layout, DSV2_LITE, max_pos=1120, fused=d.fused) for d in pair)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    tokens = torch.randint(0, lay_mod.VOCAB, (1100,), generator=g, device="cuda", dtype=torch.int32)
+    check((got, want), tokens)
+    assert got.status() == 0 and want.status() == 0
+
+
+@pytest.mark.parametrize("parts", [(37, 60), (1, 2, 130), (530, 5, 40)])
+def test_prompt_in_parts(pair, parts):
+    """fleet_prefill from a position other than 0 continues the rows that are
+    there: a prompt given in parts leaves what it leaves in one piece."""
+    import ctypes
+
+    from fleet_moe import _lib
+    got, want = pair
+    g = torch.Generator(device="cuda").manual_seed(sum(parts))
+    tokens = torch.randint(0, lay_mod.VOCAB, (sum(parts),), generator=g, device="cuda",
+                           dtype=torch.int32)
+    for d in pair:
+        d.cache.zero_()
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    lib, at = _lib.load(), 0
+    for n in parts:
+        say(f"part {n} at {at}")
+        rc = lib.fleet_prefill(ctypes.byref(got.step_model), got.step_rows,
+                               tokens[at:].data_ptr(), n, at, got.x.data_ptr(), status.data_ptr(),
+                               got.prefill_ws.data_ptr(), got.prefill_ws.numel(),
+                               ctypes.byref(got.attn._dims),
+                               torch.cuda.current_stream().cuda_stream)
+        _lib.check(rc, "fleet_prefill")
+        at += n
+    torch.cuda.synchronize()
+    say("steps")
+    want.prefill(tokens)
+    torch.cuda.synchronize()
+    assert torch.equal(got.cache, want.cache) and torch.equal(got.x, want.x)
+    assert int(status.item()) == 0
 
 
 def test_wide_exponents_and_zero_rows(pair):
