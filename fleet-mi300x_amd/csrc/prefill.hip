@@ -918,11 +918,12 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
         const int T = n_tokens - c0 < chunk ? n_tokens - c0 : chunk;
         const int p0 = pos0 + c0;
         // Tokens per block of an expert. Narrow blocks take few registers and
-        // little LDS, so three (16) or two (32) workgroups of four waves share a
-        // CU; wide ones split a weight once for more tokens. Blocks of 16 / 32 /
-        // 48, ms: 128 tokens 13.9 / 14.8 / 15.4, 192: 17.5 / 17.3, 256: 21.4 / 20.3 /
-        // 21.0, 384: 27.9 / 25.7 / 25.7, 528: 37.7 / 33.4 / 32.5
-        const int block = T <= 176 ? 16 : T <= 400 ? 32 : 48;
+        // little LDS, so three workgroups of four waves share a CU; wide ones split
+        // a weight once for more tokens. Blocks of 16 / 48, ms: 96 tokens 10.7 /
+        // 11.4, 129: 12.9 / 13.2, 136: 13.3 / 13.3, 144: 13.7 / 13.5, 176: 14.9 / 14.5,
+        // 256: 18.8 / 17.0, 384: 25.8 / 21.8, 528: 34.7 / 28.6. (Blocks of 32, two workgroups a
+        // CU: 14.0 against 14.1 at 160 and nowhere better by more; 384: 22.6.)
+        const int block = T <= 136 ? 16 : 48;
         hipLaunchKernelGGL(embed_norm_kernel, dim3(T), dim3(kThreads), 0, stream, model->embed,
                            tokens + c0, layers[0].attn.norm_in, eps, x, norm_out, status);
         for (int i = 0; i < model->n_layers; ++i) {
@@ -977,7 +978,6 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
                 launch(P, T * kTopK, bytes(L.hd), metas(L.hm), bytes(L.hsd), metas(L.hsm), stream);
             };
             if (block == 16) experts(launch_experts<1, 1, 1, 4>);
-            else if (block == 32) experts(launch_experts<2, 1, 1, 4>);
             else experts(launch_experts<3, 1, 1, 8>);
             hipLaunchKernelGGL(combine_norm_kernel, dim3(T), dim3(kThreads), 0, stream, part, x,
                                next, eps, last ? no_out : norm_out);
