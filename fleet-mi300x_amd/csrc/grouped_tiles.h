@@ -36,12 +36,10 @@ namespace tiles {
 constexpr int kSteps = 8;                     // MFMA steps (32 K) per slice
 constexpr int kSliceK = 32 * kSteps;          // 256
 constexpr int kPitch = kSliceK * 2 + 16;      // LDS bytes per token: 16 tokens' chunks hit 64 banks
-constexpr int kXcds = 8;
+using blocks::kXcds;
 
-// Entries sorted by expert, and the first entry and token block of each.
 struct Table {
-    int32_t off[kRouted + 1];
-    int32_t blk[kRouted + 1];
+    blocks::Table b;
     int16_t ent[kMaxEntries];
 };
 static_assert(sizeof(Table) <= kTabBytes, "shares the place of the other plan's tables");
@@ -65,41 +63,10 @@ struct Params {
 // an entry's sums do not depend on its block or its place there.
 __global__ __launch_bounds__(1024) void table_kernel(const int32_t* ids, int n, int tok, Header* hdr,
                                                      Table* tab) {
-    __shared__ int cnt[kRouted], at[kRouted];
-    const int tid = threadIdx.x;
-    if (tid < kRouted) cnt[tid] = 0;
-    __syncthreads();
-    int id[2];
-    bool bad = false;
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const int k = tid + 1024 * r;
-        const int raw = k < n ? ids[k] : 0;
-        id[r] = min(max(raw, 0), kRouted - 1);
-        bad |= raw != id[r];
-        if (k < n) atomicAdd(&cnt[id[r]], 1);
-    }
-    if (__ballot(bad) && (tid & (kLanes - 1)) == 0) flag_abort(hdr, FLEET_MOE_ABORT_BAD_ID);
-    __syncthreads();
-    if (tid < kLanes) {
-        const int c = cnt[tid], b = (c + tok - 1) / tok;
-        const int oi = wave_incl_scan(c), bi = wave_incl_scan(b);
-        at[tid] = oi - c;
-        tab->off[tid] = oi - c;
-        tab->blk[tid] = bi - b;
-        if (tid == kRouted - 1) {
-            tab->off[kRouted] = oi;
-            tab->blk[kRouted] = bi;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const int k = tid + 1024 * r;
-        if (k < n) tab->ent[atomicAdd(&at[id[r]], 1)] = (int16_t)k;
-    }
+    const bool bad = blocks::build<2>(ids, n, tok, &tab->b, tab->ent);
+    if (__ballot(bad) && (threadIdx.x & (kLanes - 1)) == 0) flag_abort(hdr, FLEET_MOE_ABORT_BAD_ID);
 }
-static_assert(kMaxEntries <= 2048, "two entries per thread");
+static_assert(kMaxEntries <= 2 * 1024, "two entries per thread");
 
 // LDS of a workgroup: two slices of its tokens' rows, and per wave the turn buffer
 // (two steps of 16 rows).
@@ -258,23 +225,13 @@ __device__ __forceinline__ void gemm(const uint16_t* w, const uint16_t* x, XRow&
             for (int n = 0; n < NT; ++n) y[r][n] += lo[r][n];
 }
 
-// This workgroup's token block of a routed expert (row tile `tile` of `tiles`,
-// entries [first, first + m)): the workgroups of one XCD (wg % 8) take a
-// block's row tiles in turn, so its token rows are fetched into one L2. few: the
-// expert is a VALU unit. False past the last block.
-__device__ __forceinline__ bool routed_block(const Table* tab, int wg, int tok, int tiles, int& e,
-                                             int& tile, int& first, int& m, bool& few) {
-    const int lane = threadIdx.x & (kLanes - 1);
-    const int local = wg / kXcds, b = wg % kXcds + kXcds * (local / tiles);
-    tile = local % tiles;
-    if (b >= tab->blk[kRouted]) return false;
-    // the last expert that starts at or before b (one without tokens starts
-    // where the next does)
-    e = __builtin_popcountll(__ballot(tab->blk[lane] <= b)) - 1;
-    const int j0 = tok * (b - tab->blk[e]);
-    first = tab->off[e] + j0;
-    m = min(tok, tab->off[e + 1] - first);
-    few = is_v(tab->off[e + 1] - tab->off[e]);
+// This workgroup's token block of a routed expert. few: the expert is a VALU unit.
+// False past the last block.
+__device__ __forceinline__ bool routed_block(const Params& P, int tok, int tiles, int& e, int& tile,
+                                             int& first, int& m, bool& few) {
+    if (!blocks::of(&P.tab->b, (int)blockIdx.x - P.shared_wgs, tok, tiles, e, tile, first, m))
+        return false;
+    few = is_v(P.tab->b.off[e + 1] - P.tab->b.off[e]);
     return true;
 }
 
@@ -362,9 +319,7 @@ __global__ __launch_bounds__(64 * W, 2) void g_kernel(Params P) {
     const bool shared = (int)blockIdx.x < P.shared_wgs;
     if (!shared) {
         bool few = false;
-        if (!routed_block(P.tab, (int)blockIdx.x - P.shared_wgs, 16 * NTM,
-                          2 * kInter / (16 * R * W), e, tile, first, m, few))
-            return;
+        if (!routed_block(P, 16 * NTM, 2 * kInter / (16 * R * W), e, tile, first, m, few)) return;
         wt = P.experts + (int64_t)e * P.stride;
         if (few) {
             uint8_t* const b = static_cast<uint8_t*>(lds);
@@ -444,9 +399,7 @@ __global__ __launch_bounds__(64 * W, 2) void d_kernel(Params P) {
     int e = 0, tile = 0, first = 0, m = 0;
     if ((int)blockIdx.x >= P.shared_wgs) {
         bool few = false;
-        if (!routed_block(P.tab, (int)blockIdx.x - P.shared_wgs, 16 * NTM, kTiles, e, tile, first, m,
-                          few))
-            return;
+        if (!routed_block(P, 16 * NTM, kTiles, e, tile, first, m, few)) return;
         const uint16_t* wt = P.experts + (int64_t)e * P.stride + (int64_t)2 * kInter * kHidden;
         if (few) {
             uint8_t* const b = static_cast<uint8_t*>(lds);
@@ -499,9 +452,7 @@ static void launch(Params P, const int32_t* ids, Header* hdr, Table* tab, hipStr
     // rows twice as long, and started last they ran alone at the end of a launch
     // (routing and experts of 84 / 128 / 256 tokens 240 / 244 / 286 us with the
     // routed ones first, now 217 / 216 / 258).
-    // At most one partly filled block per selected expert.
-    const int blocks = (n < kRouted ? n : kRouted) + n / kTok;
-    const int bx = (blocks + kXcds - 1) / kXcds * kXcds, sb = (P.T + kTok - 1) / kTok;
+    const int bx = blocks::most(n, kTok), sb = (P.T + kTok - 1) / kTok;
     P.shared_wgs = sb * (2 * kSharedInter / (16 * R * W));
     hipLaunchKernelGGL((g_kernel<NTM, R, W>), dim3(P.shared_wgs + bx * (2 * kInter / (16 * R * W))),
                        dim3(64 * W), 0, s, P);

@@ -283,6 +283,19 @@ __device__ __forceinline__ double wave_sum64(double v) {
     return (readlane64(v, 0) + readlane64(v, 16)) + (readlane64(v, 32) + readlane64(v, 48));
 }
 
+// Inclusive prefix sum over the 64 lanes (all lanes active), DPP only:
+// row_shr 1, 2, 4, 8 within each row of 16 (lanes without a source add 0),
+// then row_bcast 15 into rows 1 and 3 and row_bcast 31 into rows 2 and 3.
+__device__ __forceinline__ int wave_incl_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
 // Value of lane 0 in every lane (all lanes must be active).
 __device__ __forceinline__ int wave_bcast(int v) { return __builtin_amdgcn_readfirstlane(v); }
 

@@ -42,7 +42,7 @@
 #include <mutex>
 #include <vector>
 
-#include "moe_common.h"
+#include "expert_blocks.h"
 
 namespace fleet_moe {
 namespace grouped {
@@ -253,19 +253,6 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 __device__ __forceinline__ f32x4 mfma16(const u32x4& a, const u32x4& b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-// Inclusive prefix sum over the 64 lanes (all lanes active), DPP only:
-// row_shr 1, 2, 4, 8 within each row of 16 (lanes without a source add 0),
-// then row_bcast 15 into rows 1 and 3 and row_bcast 31 into rows 2 and 3.
-__device__ __forceinline__ int wave_incl_scan(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
-    return v;
 }
 
 // Workgroup-local ticket, the same value in every lane.

@@ -24,6 +24,7 @@
 
 #include "attn_body.h"
 #include "digit_gemm.h"
+#include "expert_blocks.h"
 
 namespace fleet_moe {
 namespace pre {
@@ -42,7 +43,6 @@ constexpr int kWaves = kThreads / kLanes;
 constexpr int kChunkTokens = 528;       // tokens per chunk: h, partials and q of a chunk stay resident
 constexpr int kQDimC = kLora + kRope;   // 576: q_c and q_pe of a head
 constexpr int kSlots = kTopK + 1;
-constexpr int kXcds = 8;
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
@@ -60,11 +60,6 @@ __device__ __forceinline__ double widen(const u32x4& w, int e) {
 // four consecutive rows 4 q .. 4 q + 3 of D (register pair v: row 4 q + v).
 __device__ __forceinline__ int perm16(int i) { return 4 * (i & 3) + (i >> 2); }
 
-struct Tables {
-    int32_t off[kRouted + 1];     // first sorted entry of an expert
-    int32_t blk[kRouted + 1];     // first token block of an expert
-};
-
 struct Layout {
     size_t tab, ent, x, xn, xnf, qkv, q, oc, heads, ids, w, h, hs, part;
     size_t xd, headsd, hd, hsd;             // digit rows, 3 bytes a value
@@ -79,7 +74,7 @@ __host__ constexpr Layout layout(int dense_inter) {
     const size_t hs = (size_t)(dense_inter > kSharedInter ? dense_inter : kSharedInter);
     Layout L{};
     L.tab = 0;
-    L.ent = up256(sizeof(Tables));
+    L.ent = up256(sizeof(blocks::Table));
     L.x = L.ent + up256(T * kTopK * 4);
     L.xn = L.x + T * kHidden * 4;
     L.xnf = L.xn + T * kHidden * 2;
@@ -601,41 +596,19 @@ __global__ __launch_bounds__(kThreads) void uv_kernel(const float* oc, const uin
 
 // ---------------------------------------------------------------- experts
 
-// Entries (token * 6 + slot) sorted by expert and each expert's blocks of `tok`
-// tokens, one workgroup. The order of an
-// expert's entries does not matter: each entry's results are its own.
+// The sorted entries and blocks of a chunk's tokens, one workgroup. (Ids are
+// clamped: logits that are not numbers can leave one outside the table. The order of
+// an expert's entries does not matter: each entry's results are its own.)
 __global__ __launch_bounds__(1024) void table_kernel(const int32_t* ids, int n, int tok,
-                                                     Tables* tab, int32_t* ent) {
-    __shared__ int cnt[kRouted], at[kRouted];
-    const int tid = threadIdx.x;
-    if (tid < kRouted) cnt[tid] = 0;
-    __syncthreads();
-    // (clamped: logits that are not numbers can leave an id outside the table)
-    for (int k = tid; k < n; k += 1024) atomicAdd(&cnt[min(max(ids[k], 0), kRouted - 1)], 1);
-    __syncthreads();
-    if (tid < kRouted) {
-        int off = 0, blk = 0;
-        for (int e = 0; e < tid; ++e) {
-            off += cnt[e];
-            blk += (cnt[e] + tok - 1) / tok;
-        }
-        at[tid] = off;
-        tab->off[tid] = off;
-        tab->blk[tid] = blk;
-        if (tid == kRouted - 1) {
-            tab->off[kRouted] = off + cnt[tid];
-            tab->blk[kRouted] = blk + (cnt[tid] + tok - 1) / tok;
-        }
-    }
-    __syncthreads();
-    for (int k = tid; k < n; k += 1024) ent[atomicAdd(&at[min(max(ids[k], 0), kRouted - 1)], 1)] = k;
+                                                     blocks::Table* tab, int32_t* ent) {
+    blocks::build<(kChunkTokens * kTopK + 1023) / 1024>(ids, n, tok, tab, ent);
 }
 
 struct ExpertParams {
     const uint16_t* experts;
     int64_t stride;
     const uint16_t* shared;
-    const Tables* tab;
+    const blocks::Table* tab;
     const int32_t* ent;
     const float* weights;
     Rows xn;                // [T][H]
@@ -647,24 +620,6 @@ struct ExpertParams {
     int T;
     int shared_wgs;         // workgroups of the shared expert's tiles, then those of routed ones
 };
-
-// This workgroup's token block of a routed expert: workgroups of one XCD
-// (wg % 8) take all row tiles of a block in turn, so a block's token
-// rows are fetched into one L2. False past the last block.
-__device__ __forceinline__ bool routed_block(const Tables* tab, int wg, int tok, int tiles,
-                                             int& e, int& tile, int& j0, int& m, int& base) {
-    const int lane = threadIdx.x & (kLanes - 1);
-    const int xcd = wg % kXcds, local = wg / kXcds;
-    const int b = xcd + kXcds * (local / tiles);
-    tile = local % tiles;
-    if (b >= tab->blk[kRouted]) return false;
-    e = __builtin_popcountll(__ballot(tab->blk[lane] <= b)) - 1;   // the last expert starting at or
-    // before b (an expert without tokens starts where the next one does)
-    base = tab->off[e];
-    j0 = tok * (b - tab->blk[e]);
-    m = min(tok, tab->off[e + 1] - base - j0);
-    return true;
-}
 
 template <int NT, int KS, int NW>
 __device__ __forceinline__ void gate_up_tile(const ExpertParams& P, const uint16_t* W, int tile,
@@ -693,23 +648,22 @@ template <int NTM, int KS, int NW>
 __global__ __launch_bounds__(64 * NW, NTM == 1 ? 3 : 2) void gate_up_kernel(ExpertParams P) {
     using Sh = digit::Shape<NTM, KS, NW>;
     __shared__ typename Sh::Lds L;
-    int e = 0, tile = 0, j0 = 0, m = 0, base = 0;
+    int e = 0, tile = 0, first = 0, m = 0;
     const uint16_t* W;
     const bool shared = (int)blockIdx.x < P.shared_wgs;
     if (!shared) {
-        if (!routed_block(P.tab, (int)blockIdx.x - P.shared_wgs, Sh::kTok, 2 * kInter / Sh::kRows, e,
-                          tile, j0, m, base))
+        if (!blocks::of(P.tab, (int)blockIdx.x - P.shared_wgs, Sh::kTok, 2 * kInter / Sh::kRows, e,
+                        tile, first, m))
             return;
         W = P.experts + (int64_t)e * P.stride;
     } else {
         constexpr int kTiles = 2 * kSharedInter / Sh::kRows;
         const int b = blockIdx.x;
         tile = b % kTiles;
-        j0 = Sh::kTok * (b / kTiles);
-        m = min(Sh::kTok, P.T - j0);
+        first = Sh::kTok * (b / kTiles);
+        m = min(Sh::kTok, P.T - first);
         W = P.shared;
     }
-    const int first = base + j0;
     if constexpr (NTM > 1) {
         if (m <= 16) return gate_up_tile<1, KS, NW>(P, W, tile, shared, first, m, &L);
         if (m <= 32) return gate_up_tile<2, KS, NW>(P, W, tile, shared, first, m, &L);
@@ -762,35 +716,32 @@ __global__ __launch_bounds__(64 * NW, NTM == 1 ? 3 : 2) void down_kernel(ExpertP
     using Sh = digit::Shape<NTM, KS, NW>;
     __shared__ typename Sh::Lds L;
     constexpr int kTiles = kHidden / Sh::kRows;
-    int e = 0, tile = 0, j0 = 0, m = 0, base = 0;
+    int e = 0, tile = 0, first = 0, m = 0;
     if ((int)blockIdx.x >= P.shared_wgs) {
-        if (!routed_block(P.tab, (int)blockIdx.x - P.shared_wgs, Sh::kTok, kTiles, e, tile, j0, m,
-                          base))
+        if (!blocks::of(P.tab, (int)blockIdx.x - P.shared_wgs, Sh::kTok, kTiles, e, tile, first, m))
             return;
         down_block<kInter, NTM, KS, NW>(P, P.experts + (int64_t)e * P.stride +
                                            (int64_t)2 * kInter * kHidden,
-                                    tile, base + j0, m, &L);
+                                    tile, first, m, &L);
         return;
     }
     const int b = blockIdx.x;
     tile = b % kTiles;
-    j0 = Sh::kTok * (b / kTiles);
-    m = min(Sh::kTok, P.T - j0);
-    down_block<kSharedInter, NTM, KS, NW>(P, P.shared + (int64_t)2 * kSharedInter * kHidden, tile, j0,
-                                      m, &L);
+    first = Sh::kTok * (b / kTiles);
+    m = min(Sh::kTok, P.T - first);
+    down_block<kSharedInter, NTM, KS, NW>(P, P.shared + (int64_t)2 * kSharedInter * kHidden, tile,
+                                      first, m, &L);
 }
 
-// The two expert launches and the digits between them. `n` entries; at most one
-// partly filled block per selected expert. The shared expert's workgroups come
-// first: its blocks are full and its down rows twice as long, and started last
+// The two expert launches and the digits between them. `n` entries. The shared
+// expert's workgroups come first: its blocks are full and its down rows twice as long, and started last
 // they ran alone at the end of a launch (prompts of 4 / 8 / 64 / 384 tokens: 4.99 /
 // 5.88 / 9.45 / 22.8 ms with the routed ones first, now 4.64 / 5.39 / 8.95 / 22.5).
 template <int NTM, int KG, int KD, int NW>
 static void launch_experts(ExpertParams P, int n, uint8_t* hd, digit::Meta* hm, uint8_t* hsd,
                            digit::Meta* hsm, hipStream_t s) {
     constexpr int kTok = 16 * NTM;
-    const int blocks = (n < kRouted ? n : kRouted) + n / kTok;
-    const int bx = (blocks + kXcds - 1) / kXcds * kXcds, sb = (P.T + kTok - 1) / kTok;
+    const int bx = blocks::most(n, kTok), sb = (P.T + kTok - 1) / kTok;
     constexpr int kGRows = digit::Shape<NTM, KG, NW>::kRows;
     constexpr int kDRows = digit::Shape<NTM, KD, NW>::kRows;
     P.shared_wgs = sb * (2 * kSharedInter / kGRows);
@@ -890,7 +841,7 @@ extern "C" int fleet_prefill(const fleet_step_model* model, const fleet_step_lay
     if (workspace_bytes < L.total) return FLEET_MOE_ERR_WORKSPACE;
     if (int e = fleet_moe_check_device(1)) return e;
     char* ws = static_cast<char*>(workspace);
-    Tables* tab = reinterpret_cast<Tables*>(ws + L.tab);
+    blocks::Table* tab = reinterpret_cast<blocks::Table*>(ws + L.tab);
     int32_t* ent = reinterpret_cast<int32_t*>(ws + L.ent);
     float* x = reinterpret_cast<float*>(ws + L.x);
     uint16_t* xn = reinterpret_cast<uint16_t*>(ws + L.xn);
