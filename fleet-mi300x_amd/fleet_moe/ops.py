@@ -227,6 +227,8 @@ def moe(layer: DeviceLayer, x_norm: torch.Tensor, runner: GroupedRunner, stream=
     x_bits = torch.empty(x_norm.shape, dtype=torch.int16, device=x_norm.device)
     logits, ids, ws = _route(layer, x_norm, None, x_bits, stream)
     out = runner.run(layer, x_bits, ids, ws, stream)
+    if stream is not None:
+        x_bits.record_stream(stream)      # freed here, still read there
     return {"logits": logits, "ids": ids, "weights": ws, "out": out}
 
 

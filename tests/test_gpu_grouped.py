@@ -384,3 +384,22 @@ def test_moe_equals_its_parts(dev, T):
     ops._route(layer, odd, None, bits, None)
     torch.cuda.synchronize()
     assert torch.equal(bits, ops.f32_to_bf16_bits(odd))
+
+
+def test_moe_on_another_stream_keeps_its_rows(dev):
+    """ops.moe with a stream: the bf16 rows it makes are its own until that
+    stream has read them, whatever the current stream allocates meanwhile."""
+    layer, pl = dev
+    runner = ops.GroupedRunner(4, DSV2_LITE)
+    x = torch.from_numpy(orc.rms_norm(synth.hidden_inputs(330, 4))).cuda()
+    want = ops.moe(layer, x, runner)["out"].clone()
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(200_000_000)            # about 0.1 s
+    say("moe behind a sleeping stream")
+    r = ops.moe(layer, x, runner, stream=s)
+    mine = [torch.full((4, 2048), 77, dtype=torch.int16, device="cuda") for _ in range(8)]
+    torch.cuda.synchronize()
+    assert torch.equal(r["out"], want)
+    assert all(bool((m == 77).all()) for m in mine)
