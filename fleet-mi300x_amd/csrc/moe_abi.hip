@@ -94,10 +94,17 @@ namespace router {
 // the workgroup fills the CU: 16 waves, wave w rows 8 (w / 2) .. + 7, half w % 2
 // of K, every load issued before the first product, and one reduction of eight
 // sums per wave. (Four waves of 16 rows, a load and a reduction at a time: 9.2
-// us for one token.)
+// us for one token.) That workgroup is alone on its CU, also while one of its waves
+// takes the softmax and the six picks. From four tokens to a CU on, four waves take
+// a token instead and one token's picks run beside another's products (the whole
+// call with 16 / 4 waves, us: 512 tokens 13.4 / 15.3, 900: 20.8 / 21.2, 1024: 21.2 /
+// 21.3, 1536: 29.7 / 28.4, 8192: 144 / 122, 65,535: 1182 / 972).
 constexpr int kThreads = 1024;
 constexpr int kRowsPerWave = 8;
 constexpr int kHalf = kHidden / 2;
+constexpr int kManyThreads = 256;
+constexpr int kManyRowsPerWave = 16;
+constexpr int kManyTokens = 1024;
 
 struct Params {
     const u32x4* router;
@@ -110,6 +117,44 @@ struct Params {
     float scaling;
 };
 
+// Eight fp32 values of a row, and their bf16 bits.
+__device__ __forceinline__ void load_x8(const float* xt, int chunk, float (&v)[8]) {
+    const float4* p = reinterpret_cast<const float4*>(xt) + 2 * chunk;
+    const float4 a = p[0], b = p[1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ u32x4 bf16_x8(const float (&v)[8]) {
+    u32x4 o;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = bf16_bits(v[2 * q]) | (bf16_bits(v[2 * q + 1]) << 16);
+    return o;
+}
+
+__device__ __forceinline__ double dot8_xr(const u32x4& w, const float (&x)[8], double acc) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        acc += (double)(bf_lo(w[q]) * x[2 * q]);
+        acc += (double)(bf_hi(w[q]) * x[2 * q + 1]);
+    }
+    return acc;
+}
+
+// Softmax and picks of token t from one logit per lane, by one wave.
+__device__ __forceinline__ void pick(const Params& P, int t, float l, int* s_ids, float* s_w) {
+    const int lane = threadIdx.x & (kLanes - 1);
+    if (P.logits) P.logits[(int64_t)t * kRouted + lane] = l;
+    wave_softmax_topk(l, kRouted, kTopK, P.scaling, s_ids, s_w, P.bias);
+    // lanes < k read slots written by other lanes of this same wave
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    if (lane < kTopK) {
+        P.ids[(int64_t)t * kTopK + lane] = s_ids[lane];
+        P.weights[(int64_t)t * kTopK + lane] = s_w[lane];
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void router_topk_kernel(Params P) {
     __shared__ double s_part[2][kRouted];
     __shared__ int s_ids[8];
@@ -121,12 +166,7 @@ __global__ __launch_bounds__(kThreads) void router_topk_kernel(Params P) {
     const float* xt = P.x + (int64_t)t * kHidden + half * kHalf;
     float xr[2][8];
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const float4* p = reinterpret_cast<const float4*>(xt) + 2 * (lane + kLanes * m);
-        const float4 a = p[0], b = p[1];
-        xr[m][0] = a.x; xr[m][1] = a.y; xr[m][2] = a.z; xr[m][3] = a.w;
-        xr[m][4] = b.x; xr[m][5] = b.y; xr[m][6] = b.z; xr[m][7] = b.w;
-    }
+    for (int m = 0; m < 2; ++m) load_x8(xt, lane + kLanes * m, xr[m]);
     u32x4 w[kRowsPerWave][2];
 #pragma unroll
     for (int r = 0; r < kRowsPerWave; ++r)
@@ -137,42 +177,46 @@ __global__ __launch_bounds__(kThreads) void router_topk_kernel(Params P) {
     if (P.xb && row0 == 0) {
         u32x4* o = reinterpret_cast<u32x4*>(P.xb + (int64_t)t * kHidden + half * kHalf);
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            u32x4 v;
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                v[q] = bf16_bits(xr[m][2 * q]) | (bf16_bits(xr[m][2 * q + 1]) << 16);
-            o[lane + kLanes * m] = v;
-        }
+        for (int m = 0; m < 2; ++m) o[lane + kLanes * m] = bf16_x8(xr[m]);
     }
     double acc[kRowsPerWave];
 #pragma unroll
     for (int r = 0; r < kRowsPerWave; ++r) {
         acc[r] = 0.0;
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                acc[r] += (double)(bf_lo(w[r][m][q]) * xr[m][2 * q]);
-                acc[r] += (double)(bf_hi(w[r][m][q]) * xr[m][2 * q + 1]);
-            }
+        for (int m = 0; m < 2; ++m) acc[r] = dot8_xr(w[r][m], xr[m], acc[r]);
     }
     const double tot = attn::wave_msum64<kRowsPerWave>(acc);
     s_part[half][row0 + msum_index<kRowsPerWave>(lane)] = tot;   // lanes of an index agree
     __syncthreads();
-    if (wave == 0) {
-        const float l = (float)(s_part[0][lane] + s_part[1][lane]);
-        if (P.logits) P.logits[(int64_t)t * kRouted + lane] = l;
-        wave_softmax_topk(l, kRouted, kTopK, P.scaling, s_ids, s_w, P.bias);
-        // lanes < k read slots written by other lanes of this same wave
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-        if (lane < kTopK) {
-            P.ids[(int64_t)t * kTopK + lane] = s_ids[lane];
-            P.weights[(int64_t)t * kTopK + lane] = s_w[lane];
-        }
+    if (wave == 0) pick(P, t, (float)(s_part[0][lane] + s_part[1][lane]), s_ids, s_w);
+}
+
+__global__ __launch_bounds__(kManyThreads) void router_topk_many_kernel(Params P) {
+    __shared__ float s_logit[kRouted];
+    __shared__ int s_ids[8];
+    __shared__ float s_w[8];
+    const int t = blockIdx.x;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kLanes - 1);
+    float xr[4][8];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) load_x8(P.x + (int64_t)t * kHidden, lane + kLanes * m, xr[m]);
+    if (P.xb) {
+        u32x4* o = reinterpret_cast<u32x4*>(P.xb + (int64_t)t * kHidden) + lane;
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            if (m == wave) o[kLanes * m] = bf16_x8(xr[m]);
     }
+    for (int r = wave * kManyRowsPerWave; r < (wave + 1) * kManyRowsPerWave; ++r) {
+        const u32x4* row = P.router + (int64_t)r * kRowChunks;
+        double acc = 0.0;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc = dot8_xr(row[lane + kLanes * m], xr[m], acc);
+        acc = wave_sum64(acc);
+        if (lane == 0) s_logit[r] = (float)acc;
+    }
+    __syncthreads();
+    if (wave == 0) pick(P, t, s_logit[lane], s_ids, s_w);
 }
 
 }  // namespace router
@@ -251,8 +295,12 @@ static int launch_router(const uint16_t* w_router, const float* x_norm, int32_t 
     P.weights = weights;
     P.xb = x_bf16;
     P.scaling = dims->routed_scaling;
-    hipLaunchKernelGGL(router::router_topk_kernel, dim3(n_tokens), dim3(router::kThreads), 0,
-                       stream, P);
+    if (n_tokens < router::kManyTokens)
+        hipLaunchKernelGGL(router::router_topk_kernel, dim3(n_tokens), dim3(router::kThreads), 0,
+                           stream, P);
+    else
+        hipLaunchKernelGGL(router::router_topk_many_kernel, dim3(n_tokens),
+                           dim3(router::kManyThreads), 0, stream, P);
     return (int)hipGetLastError();
 }
 

@@ -386,6 +386,28 @@ def test_moe_equals_its_parts(dev, T):
     assert torch.equal(bits, ops.f32_to_bf16_bits(odd))
 
 
+@pytest.mark.parametrize("T", [1023, 1024, 2501])
+def test_route_of_many_tokens(dev, T):
+    """Both router kernels (four waves to a token from 1,024 tokens on) give the
+    same logits, picks, weights and bf16 rows, and the oracle's."""
+    layer, pl = dev
+    xn = orc.rms_norm(synth.hidden_inputs(500 + T, T))
+    x = torch.from_numpy(xn).cuda()
+    bias = torch.from_numpy(synth.zipf_logit_bias(5)).cuda()
+    bits = torch.empty((T, 2048), dtype=torch.int16, device="cuda")
+    say(f"route T={T}")
+    got = ops._route(layer, x, bias, bits, None)
+    parts = [ops.route(layer, x[k: k + 500].contiguous(), bias) for k in range(0, T, 500)]
+    torch.cuda.synchronize()
+    for a, b in zip(got, (torch.cat(v) for v in zip(*parts))):
+        assert torch.equal(a, b)
+    assert torch.equal(bits, ops.f32_to_bf16_bits(x))
+    logits, ids, ws = orc.route(pl.router_f32(), xn[-40:], logit_bias=synth.zipf_logit_bias(5))
+    assert np.array_equal(got[0][-40:].cpu().numpy(), logits)
+    assert np.array_equal(got[1][-40:].cpu().numpy(), ids)
+    assert np.array_equal(got[2][-40:].cpu().numpy(), ws)
+
+
 def test_moe_on_another_stream_keeps_its_rows(dev):
     """ops.moe with a stream: the bf16 rows it makes are its own until that
     stream has read them, whatever the current stream allocates meanwhile."""
