@@ -8,13 +8,17 @@
 // decode kernels do it, in fp64.
 //
 // Per 16 x 16 x 64 products the fp64 matrix cores take 1024 cycles and more
-// (v_mfma_f64_16x16x4); here the eight digit products that matter take 160, and
-// splitting 16 x 64 weights about 500 cycles of the vector ALU (v_perm_b32 and
-// v_cvt_i32_f32 issue every 6 to 8 cycles), whatever the number of tokens. A SIMD's
-// share of HBM delivers those weights in 770: up to 16 tokens per expert the
-// stream runs at 5 TB/s, beyond that the vector ALU and the matrix cores bound it.
-// The 27-layer prompt of 384 tokens went from 50.7 ms on the fp64 cores to 23.2,
-// 64 tokens from 24.0 to 9.5.
+// (v_mfma_f64_16x16x4); here the eight digit products that matter take 128, and
+// a step of 16 x 64 weights about 160 vector instructions, most of them the split
+// into digits, whatever the number of tokens: 640 issue cycles, against 770 in which a
+// SIMD's share of HBM delivers those weights.
+// Counters, experts' gate / up launch (share of the SIMDs' cycles): 8 tokens: vector
+// ALU 55 %, matrix cores 11 %, 4.3 TB/s, 1.75 waves per SIMD; 64: 72 / 14 %, 5.3 TB/s,
+// 2.3 waves; 384 (blocks of 48): 50 / 19 % (5 % at once), 3.5 TB/s, 1.55 waves, which
+// wait for memory or LDS 30 % of their time and to issue 29 %. The vector ALU comes
+// first, and no pipe is full: with two waves a SIMD they overlap by chance only.
+// The 27-layer prompt of 384 tokens went from 50.7 ms on the fp64 cores to 21.8,
+// 64 tokens from 24.0 to 9.0.
 //
 //   x (a token's row, K values): ix = round(x 2^sx), |ix| < 2^22, digits b2 b1
 //     b0 (ix = b2 2^16 + b1 2^8 + b0, |b2| <= 64, |b1|, |b0| <= 128), one

@@ -1,19 +1,22 @@
 // A prompt's tokens through the whole model, all tokens of a chunk at once.
 //
-// Semantics: fleet_prefill on tokens[0 .. n) at positions pos0 .. equals n
-// calls of fleet_decode_step without the lm_head (src/host/reference_decode.py:
-// 210-302 per token and layer), bit for bit: the cache rows it writes and the
-// last token's residual are what the steps leave. Every projection is the
-// exact dot product rounded once (to fp32, then bf16), scores, softmax and the
-// weighted sum of cache rows are fp64, o_c and q_c are rounded once to fp32,
-// as in the decode kernels.
+// Semantics: fleet_prefill on tokens[0 .. n) at positions pos0 .. does what n
+// calls of fleet_decode_step do without the lm_head (src/host/reference_decode.py:
+// 210-302 per token and layer): the cache rows it writes and the last token's
+// residual are what the steps leave. Norms, RoPE, routing and every projection are
+// the same numbers by construction (each dot product exact and rounded once, to fp32,
+// then bf16). Scores, softmax and the weighted sum of cache rows are fp64 as in the
+// steps, but summed in another order (rounds of 128 positions here, chunks and
+// batches there) before o_c is rounded to fp32. The two fp64 sums differ by some
+// 1e-8 of an fp32 unit, so an o_c may round the other way, by one fp32 unit, and a
+// head output whose bf16 rounding hangs on that unit would differ. No test has
+// shown one (up to 1,100 tokens, every bit compared); nothing excludes it.
 //
 // Stepping reads every weight once per token (1.36 ms a step, 515 ms for 384
-// tokens); here a weight is read once per chunk (384 tokens: 23.2 ms). The projections run as exact
-// integer products of digits (digit_gemm.h), which keeps up with HBM; the
+// tokens); here a weight is read once per chunk (384 tokens: 21.8 ms). The
+// projections run as exact integer products of digits (digit_gemm.h); the
 // attention's own products (q_c, scores, the weighted sum, W_UV), whose operands
-// are fp32 or fp64, run on the fp64 matrix cores (v_mfma_f64_16x16x4): their
-// products and sums are exact, or fp64 as in the decode kernels.
+// are fp32 or fp64, run on the fp64 matrix cores (v_mfma_f64_16x16x4).
 //
 // Operand layout of every fp64 MFMA below: lane l holds A[i = l % 16][k = l /
 // 16] and B[k = l / 16][j = l % 16], and D[4 v + l / 16][l % 16] in register
@@ -736,7 +739,7 @@ __global__ __launch_bounds__(64 * NW, NTM == 1 ? 3 : 2) void down_kernel(ExpertP
 // The two expert launches and the digits between them. `n` entries. The shared
 // expert's workgroups come first: its blocks are full and its down rows twice as long, and started last
 // they ran alone at the end of a launch (prompts of 4 / 8 / 64 / 384 tokens: 4.99 /
-// 5.88 / 9.45 / 22.8 ms with the routed ones first, now 4.64 / 5.39 / 8.95 / 22.5).
+// 5.88 / 9.45 / 22.8 ms with the routed ones first, 4.64 / 5.39 / 8.95 / 22.5 so).
 template <int NTM, int KG, int KD, int NW>
 static void launch_experts(ExpertParams P, int n, uint8_t* hd, digit::Meta* hm, uint8_t* hsd,
                            digit::Meta* hsm, hipStream_t s) {

@@ -500,12 +500,13 @@ class Decoder:
         cache rows 0..n-1; after it token_out holds the pick after the last
         prompt token and pos == n. With `fused`, all tokens go through each
         layer together (fleet_prefill), with the results of teacher-forced
-        steps bit for bit; otherwise they are teacher-forced steps."""
+        steps (equal in every bit in all tests; the attention's fp64 sums run
+        in another order); otherwise they are teacher-forced steps."""
         self.reset(0)
         done = 0
         n = min(tokens.numel(), self.max_pos)
-        # from 4 tokens on: 3 take 4.7 ms together and 3.9 as steps, 4 take 4.6
-        # and 5.2, 8 take 5.4 and 10.4, 384 take 23 and 514 (few tokens select
+        # from 4 tokens on: 3 take 4.3 ms together and 3.9 as steps, 4 take 4.6
+        # and 5.2, 8 take 5.3 and 10.4, 384 take 22 and 514 (few tokens select
         # nearly as many experts' weights, and leave most of a 16-token tile empty)
         if self.fused and tokens.dim() == 1 and n >= 4:
             t = tokens[:n].to(device=self.blob.device, dtype=torch.int32).contiguous()

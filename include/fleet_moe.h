@@ -300,11 +300,13 @@ size_t fleet_prefill_workspace_bytes(const fleet_moe_dims* dims);
 /* n_tokens prompt tokens (device int32) at positions pos0 .. through every
  * layer, all of a chunk's tokens at once: cache rows pos0 .. pos0 + n_tokens -
  * 1 of every layer and x_out (fp32[hidden], the last token's residual before
- * the final norm) are what n_tokens calls of fleet_decode_step leave, bit for
- * bit; no logits and no pick. layers: the HOST copy of model->layers (its
- * pointers are kernel arguments); model->lm_head and final_norm are not read.
- * Every projection is the exact dot product rounded once, as in the decode
- * kernels. status: a device uint32; a token outside the vocabulary sets
+ * the final norm) are what n_tokens calls of fleet_decode_step leave; no logits
+ * and no pick. layers: the HOST copy of model->layers (its pointers are kernel
+ * arguments); model->lm_head and final_norm are not read. Every projection is
+ * the exact dot product rounded once, as in the decode kernels; the attention's
+ * fp64 sums run in another order than theirs before they are rounded to fp32, so
+ * equality with the steps in every bit, which all tests show, is not guaranteed
+ * for a value on an fp32 rounding boundary. status: a device uint32; a token outside the vocabulary sets
  * FLEET_MOE_ABORT_TOKEN there and counts as a zero row (as in fleet_embed).
  * pos0 + n_tokens <= max_pos is checked here. No two workgroups wait for each
  * other; the workspace needs no clearing. */
