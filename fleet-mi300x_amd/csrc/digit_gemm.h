@@ -368,12 +368,13 @@ __device__ __forceinline__ void slice(u32x4 (&raw)[kSliceSteps][2], const uint8_
     }
 }
 
-// The whole workgroup: w is the first of its wave's 16 weight rows, xd(i) the digit row of the workgroup's i-th token (i < 16 NT). While a
-// round of KS slices is multiplied, the next one's weights (registers) and
-// digits (registers, then the other LDS buffer) are on their way: a wave's
-// loads complete in order, so digits loaded straight from memory would wait for
-// the weights issued before them. The KS waves of a row tile add their sums in
-// LDS; A is complete in those with wave % KS == 0.
+// The whole workgroup: w is the first of its wave's 16 weight rows, xd(i) the digit
+// row of the workgroup's i-th token (i < 16 NT). While a round of KS slices is
+// multiplied, the next one's weights (registers) and digits (registers, then the
+// other LDS buffer) are on their way: a wave's loads complete in order, so digits
+// loaded straight from memory would wait for the weights issued before them. The KS
+// waves of a row tile add their sums in LDS; A is complete in those with wave % KS
+// == 0.
 template <int K, int NT, int KS, int W, class XD>
 __device__ __forceinline__ void gemm(const uint16_t* w, XD&& xd,
                                      typename Shape<NT, KS, W>::Lds& L, Acc<NT>& A) {

@@ -736,10 +736,11 @@ __global__ __launch_bounds__(64 * NW, NTM == 1 ? 3 : 2) void down_kernel(ExpertP
                                       first, m, &L);
 }
 
-// The two expert launches and the digits between them. `n` entries. The shared
-// expert's workgroups come first: its blocks are full and its down rows twice as long, and started last
-// they ran alone at the end of a launch (prompts of 4 / 8 / 64 / 384 tokens: 4.99 /
-// 5.88 / 9.45 / 22.8 ms with the routed ones first, 4.64 / 5.39 / 8.95 / 22.5 so).
+// The two expert launches and the digits between them; `n` entries. The shared
+// expert's workgroups come first: its blocks are full and its down rows twice as
+// long, and started last they ran alone at the end of a launch (prompts of 4 / 8 /
+// 64 / 384 tokens: 4.99 / 5.88 / 9.45 / 22.8 ms with the routed ones first, 4.64 /
+// 5.39 / 8.95 / 22.5 so).
 template <int NTM, int KG, int KD, int NW>
 static void launch_experts(ExpertParams P, int n, uint8_t* hd, digit::Meta* hm, uint8_t* hsd,
                            digit::Meta* hsm, hipStream_t s) {
