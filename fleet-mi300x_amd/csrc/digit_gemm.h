@@ -13,7 +13,7 @@
 // into digits, whatever the number of tokens: 640 issue cycles, against 770 in which a
 // SIMD's share of HBM delivers those weights.
 // Counters, experts' gate / up launch (share of the SIMDs' cycles): 8 tokens: vector
-// ALU 55 %, matrix cores 11 %, 4.3 TB/s, 1.75 waves per SIMD; 64: 72 / 14 %, 5.3 TB/s,
+// ALU 55 %, matrix cores 11 %, 4.6 TB/s, 1.7 waves per SIMD; 64: 72 / 14 %, 5.1 TB/s,
 // 2.3 waves; 384 (blocks of 48): 50 / 19 % (5 % at once), 3.5 TB/s, 1.55 waves, which
 // wait for memory or LDS 30 % of their time and to issue 29 %. The vector ALU comes
 // first, and no pipe is full: with two waves a SIMD they overlap by chance only.

